@@ -3,8 +3,10 @@
 // Kernels and the C ABI declared in include/qd_attention.h:
 //
 //   decode_mfma_sk_kernel  the automatic path for 16-bit caches, head_dim
-//                          64/128/256, block_size a multiple of 16, group
-//                          size <= 16.  The (sequence, 16-token group)
+//                          64/96/128/256 and block_size a multiple of 16
+//                          (MfmaWave), or any other block_size and head_dim
+//                          a multiple of 8 (GenWave), and for large fp32
+//                          batches (MfmaWaveF32).  The (sequence, 16-token group)
 //                          space of the whole batch is cut into W equal
 //                          ranges, one per resident workgroup, so every
 //                          workgroup (and every XCD) streams the same number
@@ -87,6 +89,10 @@ struct DecodeParams {
   int kv_split;
   int kv_rows;
   int kv_g;
+  // Token -> page: t / P = umulhi(2t, page_mul) >> page_shift for 0 <= t < 2^31
+  // (page_divisor on the host).
+  uint32_t page_mul;
+  int page_shift;
 #ifdef QD_STAMPS
   uint64_t* stamps;  // diagnostic build: per-wave timestamps (stamp_wave)
 #endif
@@ -159,8 +165,11 @@ __device__ __forceinline__ int clamp_page(int32_t phys, int64_t num_blocks) {
   return phys;
 }
 
+// Page of token t >= 0 of a sequence.
+__device__ __forceinline__ int page_of(const DecodeParams& p, int t) {
+  return static_cast<int>(__umulhi(2u * static_cast<uint32_t>(t), p.page_mul) >> p.page_shift);
+}
 
-// Inclusive prefix sum over the 64 lanes.
 // ----------------------------------------------------------------------------
 // Portable VALU kernel
 // ----------------------------------------------------------------------------
@@ -1086,6 +1095,253 @@ struct MfmaWaveF32 : MfmaWave<D, QD_DTYPE_F32, PF, 1> {
   }
 };
 
+// One wave's decode state for one kv-head in the general layout: 16-bit
+// caches with any block_size and any head_dim Dm = p.D that is a multiple of
+// 8 up to 128 or of 16 up to 256 (VD = 64, 128 or 256 is the next V layout,
+// KC = 32-wide QK chunks covering Dm).  MfmaWave's lane layouts with two
+// changes:
+//   rows   a 16-token group may span pages, so lane r16 finds the pool row of
+//          token r16 (its page from a window of the table row in LDS, the
+//          division by block_size as a multiply) and the loads take their
+//          rows from those lanes (ds_bpermute): one LDS round trip per group
+//          whatever the block size, against a dependent table load per page.
+//   dims   pieces past a row's Dm elements re-read its last piece (no extra
+//          bytes from memory); K's pad columns are zero in the LDS tile and in
+//          the query, and V's pad columns reach only accumulators that are
+//          never stored.
+// The softmax weights enter the PV product as hi + lo for fp16 too (this
+// layout replaces the VALU kernel, which keeps them in fp32; the second half
+// of the 16x16x32 product costs nothing).
+//
+// Bound by HBM like MfmaWave.  Against the VALU kernel on the split layout
+// that served these shapes (us per call): fp16 head_dim 80, Hq32/Hkv32, P16,
+// B16, lengths U[256, 2048] (226 MB) 388.2 -> 57.0, 0.58 -> 4.0 TB/s; bf16
+// head_dim 128, Hq32/Hkv8, P8, B24, U[128, 3000] (135 MB) 109.0 -> 31.0.
+template <int VD, int KCG, int DT, int PF>
+struct GenWave : MfmaWave<VD, DT, PF, 1> {
+  using Base = MfmaWave<VD, DT, PF, 1>;
+  using Ops = MfmaOps<DT>;
+  using S = typename Elem<DT>::S;
+  static constexpr int EV = VD / 16;                // V elements per lane and row
+  static constexpr int kStride = 64 * KCG + 32;     // LDS bytes per K row
+  static constexpr int kTileBytes = 16 * kStride;
+  static constexpr int kWinPages = 512;             // table window (LDS)
+  struct Buf {
+    u32x4 k[KCG];
+    VRow<VD> v[4];
+    int tg;
+  };
+  u32x4 qg[KCG];
+  int dm;            // head_dim in memory
+  int krow[KCG];     // K load c of this lane: row of the group ...
+  int kcol[KCG];     // ... and byte offset in the row
+  int voff;          // byte offset of this lane's V piece
+  int32_t* win;      // this wave's table window
+
+  __device__ void init_lane_gen(const DecodeParams& p, char* ktile, int32_t* window) {
+    Base::init_lane();
+    dm = p.D;
+    win = window;
+    const int per_row = dm >> 3;  // 16-byte pieces of a K row
+#pragma unroll
+    for (int c = 0; c < KCG; ++c) {
+      const int piece = min(64 * c + this->lane, 16 * per_row - 1);
+      krow[c] = piece / per_row;
+      kcol[c] = 16 * (piece - krow[c] * per_row);
+    }
+    voff = 2 * min(EV * this->r16, dm - EV);
+    for (int o = 16 * this->lane; o < kTileBytes; o += 1024)
+      *reinterpret_cast<u32x4*>(ktile + o) = u32x4{0u, 0u, 0u, 0u};
+  }
+
+  // Table entries of pages [first, first + npages) into the window (at most
+  // kWinPages; entries past the table row stay 0, unused).
+  __device__ void load_window(const DecodeParams& p, int first, int npages) {
+    this->wbase = first;
+    const int n = min(min(npages, kWinPages), p.maxP - first);
+    for (int i = this->lane; i < n; i += 64) win[i] = this->trow[first + i];
+  }
+
+  __device__ int pages_to(const DecodeParams& p, int gb, int first) const {
+    const uint32_t last = min(16u * static_cast<uint32_t>(gb), static_cast<uint32_t>(this->len)) - 1u;
+    return page_of(p, static_cast<int>(last)) - first + 1;
+  }
+
+  __device__ void begin_item_gen(const DecodeParams& p, int b, int kvh, int valid_tokens, int ga, int gb) {
+    this->hcount = vhead_count(p, kvh);
+    const bool head_ok = this->r16 < this->hcount;
+    this->trow = p.table + static_cast<int64_t>(b) * p.maxP;
+    this->len = valid_tokens;
+    const int first = page_of(p, 16 * ga);
+    load_window(p, first, pages_to(p, gb, first));
+    const char* qp = static_cast<const char*>(p.q) +
+                     (static_cast<int64_t>(b) * p.Hq + vhead_base(p, kvh) + (head_ok ? this->r16 : 0)) * dm * 2;
+#pragma unroll
+    for (int c = 0; c < KCG; ++c) {
+      const int e = 32 * c + 8 * this->q4;
+      const u32x4 x = *reinterpret_cast<const u32x4*>(qp + 2 * min(e, dm - 8));
+      const u32x4 zero = {0u, 0u, 0u, 0u};
+      qg[c] = head_ok && e < dm ? x : zero;
+    }
+    this->m_run[0] = -INFINITY;
+    this->l_run[0] = 0.f;
+#pragma unroll
+    for (int d = 0; d < EV; ++d) this->acc[0][d] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const int64_t col = p.kv_split > 1 ? kvh / p.kv_split : kvh;
+    this->kbase = static_cast<const char*>(p.k) + col * dm * 2;
+    this->vbase = static_cast<const char*>(p.v) + col * dm * 2;
+  }
+
+  __device__ void issue(const DecodeParams& p, Buf& buf, int gi) {
+    const int tg = 16 * gi;
+    buf.tg = tg;
+    // Pool row of token r16 (tokens at or past the end re-read the last one);
+    // num_blocks * P < 2^31 (host check).
+    const int t = static_cast<int>(min(static_cast<uint32_t>(tg + this->r16), static_cast<uint32_t>(this->len - 1)));
+    const int page = page_of(p, t);
+    const int row = clamp_page(win[page - this->wbase], p.num_blocks) * p.P + (t - page * p.P);
+    const int64_t row_bytes = static_cast<int64_t>(p.kv_rows) * dm * 2;
+#pragma unroll
+    for (int c = 0; c < KCG; ++c) {
+      const int64_t r = __builtin_amdgcn_ds_bpermute(4 * krow[c], row);
+      buf.k[c] = stream_load16(this->kbase + r * row_bytes + kcol[c]);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int64_t r = __builtin_amdgcn_ds_bpermute(4 * (4 * this->q4 + i), row);
+      buf.v[i] = load_vrow<VD>(this->vbase + r * row_bytes + voff);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  }
+
+  __device__ void compute(const DecodeParams& p, const Buf& buf, char* ktile) {
+    const int last = this->len - 1 - buf.tg;
+#pragma unroll
+    for (int c = 0; c < KCG; ++c) *reinterpret_cast<u32x4*>(ktile + krow[c] * kStride + kcol[c]) = buf.k[c];
+    u32x4 ka[KCG];
+#pragma unroll
+    for (int c = 0; c < KCG; ++c)
+      ka[c] = *reinterpret_cast<const u32x4*>(ktile + this->r16 * kStride + 64 * c + 16 * this->q4);
+    f32x4 s = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int c = 0; c < KCG; ++c) s = Ops::qk(ka[c], qg[c], s);
+    float x[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) x[i] = (4 * this->q4 + i <= last) ? s[i] : -INFINITY;
+    float mx = fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3]));
+    mx = fmaxf(mx, __shfl_xor(mx, 16));
+    mx = fmaxf(mx, __shfl_xor(mx, 32));
+    const float mn = fmaxf(this->m_run[0], mx * p.sl2);
+    const float mref = mn == -INFINITY ? 0.f : mn;
+    const float alpha = fast_exp2(this->m_run[0] - mref);
+    float pr[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) pr[i] = fast_exp2(fmaf(x[i], p.sl2, -mref));
+    this->l_run[0] = fmaf(this->l_run[0], alpha, (pr[0] + pr[1]) + (pr[2] + pr[3]));
+    this->m_run[0] = mn;
+    if (__builtin_amdgcn_read_exec() & __ballot(alpha != 1.f)) {
+#pragma unroll
+      for (int d = 0; d < EV; ++d) this->acc[0][d] *= alpha;
+    }
+    const u32x2 hi = {Ops::pack2(pr[0], pr[1]), Ops::pack2(pr[2], pr[3])};
+    const u32x4 w = {hi[0], hi[1], Ops::rest2(pr[0], pr[1], hi[0]), Ops::rest2(pr[2], pr[3], hi[1])};
+#pragma unroll
+    for (int d = 0; d < EV; ++d) {
+      const uint32_t sel = (d & 1) ? 0x07060302u : 0x05040100u;
+      const uint32_t a0 = __builtin_amdgcn_perm(buf.v[1].w[d >> 1], buf.v[0].w[d >> 1], sel);
+      const uint32_t a1 = __builtin_amdgcn_perm(buf.v[3].w[d >> 1], buf.v[2].w[d >> 1], sel);
+      this->acc[0][d] = Ops::mma32(u32x4{a0, a1, a0, a1}, w, this->acc[0][d]);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  }
+
+  // MfmaWave::run over runs of groups whose tokens lie inside one window.
+  __device__ void run(const DecodeParams& p, int ga, int gb, char* ktile, bool lockstep = false) {
+    for (int g_lo = ga; g_lo < gb;) {
+      if (g_lo != ga) {  // the first window came with begin_item_gen
+        const int first = page_of(p, 16 * g_lo);
+        load_window(p, first, pages_to(p, gb, first));
+      }
+      const int64_t whole = static_cast<int64_t>(this->wbase + kWinPages) * p.P >> 4;  // groups inside the window
+      const int g_hi = whole < gb && page_of(p, this->len - 1) >= this->wbase + kWinPages ? static_cast<int>(whole) : gb;
+      const int n = g_hi - g_lo;
+      Buf buf[PF];
+      int i = 0;
+      if (n >= 2 * PF - 1) {
+#pragma unroll
+        for (int u = 0; u < PF - 1; ++u) issue(p, buf[u], g_lo + u);
+        for (; i + 2 * PF - 2 < n; i += PF) {
+          if (lockstep) __builtin_amdgcn_s_barrier();
+#pragma unroll
+          for (int u = 0; u < PF; ++u) {
+            issue(p, buf[(u + PF - 1) % PF], g_lo + i + u + PF - 1);
+            compute(p, buf[u], ktile);
+          }
+        }
+      } else {
+#pragma unroll
+        for (int u = 0; u < PF - 1; ++u)
+          if (u < n) issue(p, buf[u], g_lo + u);
+      }
+      for (; i < n; i += PF) {
+#pragma unroll
+        for (int u = 0; u < PF; ++u) {
+          if (i + u + PF - 1 < n) issue(p, buf[(u + PF - 1) % PF], g_lo + i + u + PF - 1);
+          if (i + u < n) compute(p, buf[u], ktile);
+        }
+      }
+      g_lo = g_hi;
+    }
+  }
+
+  // This lane's column block of the output row: columns EV*(4*q4+i) .. + EV-1
+  // for i = 0..3, whole blocks inside dm or past it.
+  __device__ bool block_ok(int i) const { return EV * (4 * this->q4 + i) < dm; }
+
+  __device__ void put_row(char* row, float l_tot) const {
+    const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      if (!block_ok(i)) continue;
+      uint32_t wv[EV / 2];
+#pragma unroll
+      for (int j = 0; j < EV; j += 2)
+        wv[j / 2] = Ops::pack2(l_tot > 0.f ? this->acc[0][j][i] * inv : 0.f,
+                               l_tot > 0.f ? this->acc[0][j + 1][i] * inv : 0.f);
+      store_words<EV / 2>(row + 2 * EV * (4 * this->q4 + i), wv);
+    }
+  }
+
+  // w: the lane's partial row {m (natural log), l, acc[dm]}, 8-byte aligned.
+  __device__ void put_partial(float* w, float l_tot) const {
+    if (this->q4 == 0) *reinterpret_cast<f32x2*>(w) = f32x2{this->m_run[0] * kLn2, l_tot};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      if (!block_ok(i)) continue;
+      float* dst = w + 2 + EV * (4 * this->q4 + i);
+#pragma unroll
+      for (int j = 0; j < EV; j += 2)
+        *reinterpret_cast<f32x2*>(dst + j) = f32x2{this->acc[0][j][i], this->acc[0][j + 1][i]};
+    }
+  }
+
+  __device__ void store_direct(const DecodeParams& p, int b, int kvh, int, float l_tot) {
+    if (this->r16 >= this->hcount) return;
+    put_row(reinterpret_cast<char*>(static_cast<S*>(p.out) +
+                                    (static_cast<int64_t>(b) * p.Hq + vhead_base(p, kvh) + this->r16) * dm),
+            l_tot);
+  }
+  __device__ void stage_direct(const DecodeParams&, char* area, int, float l_tot) {
+    if (this->r16 < this->hcount) put_row(area + this->r16 * dm * 2, l_tot);
+  }
+  __device__ void store_partial(const DecodeParams&, int, float* w, int64_t head_stride, float l_tot) {
+    if (this->r16 < this->hcount) put_partial(w + this->r16 * head_stride, l_tot);
+  }
+  __device__ void stage_partial(const DecodeParams&, char* area, int, float l_tot) {
+    if (this->r16 < this->hcount) put_partial(reinterpret_cast<float*>(area) + this->r16 * (dm + 2), l_tot);
+  }
+};
+
 // VALU compute of the same per-wave pipeline, for comparison with the MFMA
 // one (head_dim 128, one kv-head per wave, at most GV heads per group).
 // Same loads, table windows and partition as MfmaWave; only the math
@@ -1349,11 +1605,13 @@ __device__ __forceinline__ int seq_groups(const DecodeParams& p, int len_raw) {
 // (combine_groups).  Partials from an earlier kernel on the same stream are
 // read with plain loads; COH: sc1 loads, for partials that other workgroups
 // of the same launch wrote with sc1 stores.
-template <int D, int KB, bool COH = false>
+// GEN: rows of dm <= D elements (whole lane blocks inside dm or past it).
+template <int D, int KB, bool COH = false, bool GEN = false>
 struct MergeRows {
   static constexpr int EPL = D / 16;
   static constexpr int kBatch = KB;  // rows loaded per memory round trip
   int c16;
+  int dm = D;
   float M = -INFINITY, L = 0.f;
   float acc[EPL];
   float ms[kBatch], ls[kBatch], av[kBatch][EPL];
@@ -1375,9 +1633,10 @@ struct MergeRows {
       const f32x2 ml = COH ? coherent_load2(row) : *reinterpret_cast<const f32x2*>(row);
       ms[t] = ml[0];
       ls[t] = ml[1];
+      const int at = GEN ? min(c16 * EPL, dm - EPL) : c16 * EPL;
 #pragma unroll
       for (int e = 0; e < EPL; e += 2) {
-        const float* src = row + 2 + c16 * EPL + e;
+        const float* src = row + 2 + at + e;
         const f32x2 x = COH ? coherent_load2(src) : *reinterpret_cast<const f32x2*>(src);
         av[t][e] = x[0];
         av[t][e + 1] = x[1];
@@ -1436,7 +1695,7 @@ struct MergeRows {
   // 16-byte aligned (8-byte for 16-bit rows of D = 64).
   template <int DT>
   __device__ void store(bool active, typename Elem<DT>::S* out) const {
-    if (!active) return;
+    if (!active || (GEN && c16 * EPL >= dm)) return;
     const float inv = L > 0.f ? 1.f / L : 0.f;
     if constexpr (DT == QD_DTYPE_F32) {
       static_assert(EPL % 4 == 0, "fp32 rows: head_dim a multiple of 64");
@@ -1612,7 +1871,9 @@ __device__ __forceinline__ uint32_t arrive(const DecodeParams& p, int b, int kvh
 // that completes a counter (the nwg-th) merges that item's heads from all
 // nwg slots and resets the counter to zero.  No wave ever waits for
 // another, and the counters are left as they were found (zero).
-template <int D, int DT, int PF, int NKV, int GV = 0, bool FUSED = false, bool HOLD = false>
+//
+// KCG > 0: the general layout (GenWave), head_dim p.D in memory.
+template <int D, int DT, int PF, int NKV, int GV = 0, bool FUSED = false, bool HOLD = false, int KCG = 0>
 __global__ __launch_bounds__((64 * sk_max_waves<D, NKV, GV, PF, DT>())) void decode_mfma_sk_kernel(DecodeParams p) {
   static_assert(!(HOLD && (FUSED || GV > 0)), "results are held only by the MFMA kernel with the merge kernel");
   using S = typename Elem<DT>::S;
@@ -1623,7 +1884,11 @@ __global__ __launch_bounds__((64 * sk_max_waves<D, NKV, GV, PF, DT>())) void dec
   const int W = p.splits;
   const int B = p.B;
   static_assert(DT != QD_DTYPE_F32 || (NKV == 1 && GV == 0 && !FUSED), "fp32 caches: one kv-head per wave, merge kernel");
-  __shared__ __align__(16) char ktile[sk_max_waves<D, NKV, GV, PF, DT>()][KTile<D, DT == QD_DTYPE_F32 ? 4 : 2>::kBytes];
+  constexpr bool kGen = KCG > 0;
+  static_assert(!kGen || (NKV == 1 && GV == 0 && !FUSED && DT != QD_DTYPE_F32), "general layout: one kv-head per wave");
+  constexpr int kTileBytes = kGen ? 16 * (64 * KCG + 32) : KTile<D, DT == QD_DTYPE_F32 ? 4 : 2>::kBytes;
+  __shared__ __align__(16) char ktile[sk_max_waves<D, NKV, GV, PF, DT>()][kTileBytes];
+  const int dm = kGen ? p.D : D;  // head_dim in memory
   QD_STAMP(p, 0, stamp_now());
   QD_STAMP(p, 8, stamp_clock());
   QD_STAMP(p, 6, stamp_xcc());
@@ -1736,11 +2001,17 @@ __global__ __launch_bounds__((64 * sk_max_waves<D, NKV, GV, PF, DT>())) void dec
   // GV > 0: the VALU comparison variant (ValuWave, GV heads per group).
   using Wave = std::conditional_t<
       GV == 0,
-      std::conditional_t<DT == QD_DTYPE_F32, MfmaWaveF32<D, PF>, MfmaWave<D, DT, PF, NKV>>,
+      std::conditional_t<DT == QD_DTYPE_F32, MfmaWaveF32<D, PF>,
+                         std::conditional_t<kGen, GenWave<D, kGen ? KCG : 1, DT, PF>, MfmaWave<D, DT, PF, NKV>>>,
       ValuWave<D, DT, PF, (GV > 0 ? GV : 4)>>;
   Wave wv;
-  wv.init_lane();
-  const int64_t slot_floats = static_cast<int64_t>(p.Hq) * (D + 2);
+  if constexpr (kGen) {
+    __shared__ int32_t window[sk_max_waves<D, NKV, GV, PF, DT>()][Wave::kWinPages];
+    wv.init_lane_gen(p, ktile[wid], window[wid]);
+  } else {
+    wv.init_lane();
+  }
+  const int64_t slot_floats = static_cast<int64_t>(p.Hq) * (dm + 2);
   // FUSED: the split sequences of this range, {sequence, first workgroup,
   // workgroups}; the second is used when the range ends inside a sequence.
   int sp_b0 = -1, sp_f0 = 0, sp_n0 = 0, sp_b1 = -1, sp_f1 = 0, sp_n1 = 0;
@@ -1772,7 +2043,10 @@ __global__ __launch_bounds__((64 * sk_max_waves<D, NKV, GV, PF, DT>())) void dec
       if (FUSED && !whole && mid_range) sp_stashed = true;
       float* slot = p.ws + static_cast<int64_t>(w + b) * slot_floats;
       for (int kvh0 = wid * NKV; kvh0 < p.Hkv; kvh0 += nw * NKV) {
-        wv.begin_item(p, b, kvh0, len, i0);
+        if constexpr (kGen)
+          wv.begin_item_gen(p, b, kvh0, len, i0, i1);
+        else
+          wv.begin_item(p, b, kvh0, len, i0);
         // Every wave runs exactly one item here when the workgroup's waves
         // cover the kv-heads once, so all reach the same barriers.
         wv.run(p, i0, i1, ktile[wid], p.Hkv == nw * NKV);
@@ -1795,13 +2069,13 @@ __global__ __launch_bounds__((64 * sk_max_waves<D, NKV, GV, PF, DT>())) void dec
             if (whole)
               wv.store_direct(p, b, kvh0, j, l_tot);
             else
-              wv.store_partial(p, j, slot + static_cast<int64_t>(vhead_base(p, kvh0 + j)) * (D + 2), D + 2, l_tot);
+              wv.store_partial(p, j, slot + static_cast<int64_t>(vhead_base(p, kvh0 + j)) * (dm + 2), dm + 2, l_tot);
           }
         } else if constexpr (HOLD) {
           // The item's heads (fewer than NKV * g for a short last chunk of
           // a split kv-head): the flush writes exactly these rows.
           const int nheads = p.kv_split > 1 ? wv.hcount : NKV * p.g;
-          const int bytes = whole ? nheads * D * static_cast<int>(sizeof(S)) : nheads * (D + 2) * 4;
+          const int bytes = whole ? nheads * dm * static_cast<int>(sizeof(S)) : nheads * (dm + 2) * 4;
           char* area = wv.stage_slot(bytes);
 #pragma unroll
           for (int j = 0; j < NKV; ++j) {
@@ -1813,10 +2087,10 @@ __global__ __launch_bounds__((64 * sk_max_waves<D, NKV, GV, PF, DT>())) void dec
           }
           if (whole)
             wv.stage_commit(reinterpret_cast<char*>(static_cast<S*>(p.out) +
-                                                    (static_cast<int64_t>(b) * p.Hq + vhead_base(p, kvh0)) * D),
+                                                    (static_cast<int64_t>(b) * p.Hq + vhead_base(p, kvh0)) * dm),
                             bytes, 16);
           else
-            wv.stage_commit(reinterpret_cast<char*>(slot + static_cast<int64_t>(vhead_base(p, kvh0)) * (D + 2)),
+            wv.stage_commit(reinterpret_cast<char*>(slot + static_cast<int64_t>(vhead_base(p, kvh0)) * (dm + 2)),
                             bytes, 8);
         } else {
           wv.finish_item();
@@ -1911,7 +2185,8 @@ __global__ __launch_bounds__((64 * sk_max_waves<D, NKV, GV, PF, DT>())) void dec
 //           folds rows j4, j4+4, ... (4*KB rows per round trip), then the
 //           four group states are combined.  For sequences split over many
 //           workgroups.
-template <int D, int DT, int KB, int RG>
+// GEN: rows of p.D <= D elements (the general layout).
+template <int D, int DT, int KB, int RG, bool GEN = false>
 __global__ __launch_bounds__(64) void merge_sk_kernel(DecodeParams p) {
   using S = typename Elem<DT>::S;
   const int b = blockIdx.y;
@@ -1920,21 +2195,23 @@ __global__ __launch_bounds__(64) void merge_sk_kernel(DecodeParams p) {
   if (nwg <= 1) return;  // written directly, or an empty sequence (zero-filled)
   if (first < 0 || first + nwg > p.splits) return;  // spans are always inside [0, W)
   const int j4 = (threadIdx.x & 63) >> 4;
-  const int64_t slot_floats = static_cast<int64_t>(p.Hq) * (D + 2);
+  const int dm = GEN ? p.D : D;
+  const int64_t slot_floats = static_cast<int64_t>(p.Hq) * (dm + 2);
   const float* slots = p.ws + static_cast<int64_t>(first + b) * slot_floats;
-  MergeRows<D, KB> mr;
+  MergeRows<D, KB, false, GEN> mr;
+  mr.dm = dm;
   if constexpr (RG == 1) {
     const int hh = 4 * blockIdx.x + j4;
     const bool active = hh < p.Hq;
     const int64_t h = active ? hh : 0;
-    mr.fold_rows(slots + h * (D + 2), slot_floats, nwg);
-    mr.template store<DT>(active, static_cast<S*>(p.out) + (static_cast<int64_t>(b) * p.Hq + h) * D);
+    mr.fold_rows(slots + h * (dm + 2), slot_floats, nwg);
+    mr.template store<DT>(active, static_cast<S*>(p.out) + (static_cast<int64_t>(b) * p.Hq + h) * dm);
   } else {
     const int64_t h = blockIdx.x;
     const int nrows = nwg > j4 ? (nwg - j4 + RG - 1) / RG : 0;
-    mr.fold_rows(slots + (h + static_cast<int64_t>(j4) * p.Hq) * (D + 2), RG * slot_floats, nrows);
+    mr.fold_rows(slots + (h + static_cast<int64_t>(j4) * p.Hq) * (dm + 2), RG * slot_floats, nrows);
     mr.combine_groups();
-    mr.template store<DT>(j4 == 0, static_cast<S*>(p.out) + (static_cast<int64_t>(b) * p.Hq + h) * D);
+    mr.template store<DT>(j4 == 0, static_cast<S*>(p.out) + (static_cast<int64_t>(b) * p.Hq + h) * dm);
   }
 }
 
@@ -2173,6 +2450,58 @@ constexpr int64_t kSkWgBytes = int64_t{256} << 10;
 constexpr int kSkOversubscribe = QD_SK_OVERSUB;
 
 using KernelFn = void (*)(DecodeParams);
+
+// The general layout (GenWave): 16-bit caches whose block_size or head_dim
+// the kernels above do not take, head_dim a multiple of 8 up to 128 or of 16
+// up to 256, on the balanced path; odd multiples of 8 above 128 would end
+// inside a lane's V piece and stay on the VALU kernel.  Against the split
+// layout's VALU kernel (us per call, bf16/fp16): B64 Hq32/Hkv8 D72 P16 196.1 ->
+// 26.8, B16 D160 P32 327.3 -> 45.4, B16 D256 P8 136.0 -> 55.6, B16 D128 P1
+// U[1000, 6000] 89.7 -> 47.0, B64 Hq8/Hkv2 D32 28.9 -> 15.5, B1 Hq8/Hkv1 D16
+// 11.3 -> 9.4.  The one loss is a handful of groups that a workgroup's waves
+// cover in several passes of kv-heads, one after the other (B1/L128 Hkv32 D80
+// 18.5 -> 19.1, B1/L64 Hkv8 D256 16.8 -> 17.6): at most kGeneralFewGroups
+// groups in the largest batch then stay on the split layout.
+constexpr int64_t kGeneralFewGroups = 8;
+
+bool general_applies(int head_dim, int dtype) {
+  return (dtype == QD_DTYPE_F16 || dtype == QD_DTYPE_BF16) &&
+         (head_dim <= 128 ? head_dim % 8 == 0 : head_dim % 16 == 0 && head_dim <= 256);
+}
+
+// V layout (64, 128 or 256 columns) and 32-wide QK chunks of the general
+// kernel serving a head_dim.
+int general_vd(int head_dim) { return head_dim <= 64 ? 64 : head_dim <= 128 ? 128 : 256; }
+
+template <int DT, bool HOLD>
+KernelFn pick_general_sk(int head_dim) {
+  if (head_dim <= 64) return decode_mfma_sk_kernel<64, DT, 3, 1, 0, false, HOLD, 2>;
+  if (head_dim <= 96) return decode_mfma_sk_kernel<128, DT, 2, 1, 0, false, HOLD, 3>;
+  if (head_dim <= 128) return decode_mfma_sk_kernel<128, DT, 2, 1, 0, false, HOLD, 4>;
+  if (head_dim <= 192) return decode_mfma_sk_kernel<256, DT, 2, 1, 0, false, HOLD, 6>;
+  return decode_mfma_sk_kernel<256, DT, 2, 1, 0, false, HOLD, 8>;
+}
+
+KernelFn pick_general_sk_dt(int dtype, int head_dim, bool hold) {
+  if (dtype == QD_DTYPE_F16)
+    return hold ? pick_general_sk<QD_DTYPE_F16, true>(head_dim) : pick_general_sk<QD_DTYPE_F16, false>(head_dim);
+  return hold ? pick_general_sk<QD_DTYPE_BF16, true>(head_dim) : pick_general_sk<QD_DTYPE_BF16, false>(head_dim);
+}
+
+template <int DT, int KB, int RG>
+KernelFn pick_general_merge(int head_dim) {
+  switch (general_vd(head_dim)) {
+    case 64: return merge_sk_kernel<64, DT, KB, RG, true>;
+    case 128: return merge_sk_kernel<128, DT, KB, RG, true>;
+    default: return merge_sk_kernel<256, DT, KB, RG, true>;
+  }
+}
+
+KernelFn pick_general_merge_dt(int dtype, int head_dim, bool one_head) {
+  if (dtype == QD_DTYPE_F16)
+    return one_head ? pick_general_merge<QD_DTYPE_F16, 16, 4>(head_dim) : pick_general_merge<QD_DTYPE_F16, 8, 1>(head_dim);
+  return one_head ? pick_general_merge<QD_DTYPE_BF16, 16, 4>(head_dim) : pick_general_merge<QD_DTYPE_BF16, 8, 1>(head_dim);
+}
 
 template <int DT>
 KernelFn pick_mfma(int D) {
@@ -2490,6 +2819,7 @@ struct AutoPlan {
   size_t ws_bytes;  // scratch bytes (kCounterBytes of counters first)
   size_t meta_offset;  // stream-K: byte offset of the meta table in the scratch
   int kv_split;     // stream-K: virtual kv-heads per kv-head (DecodeParams::kv_split)
+  bool general;     // stream-K: the general layout (general_applies)
 };
 
 // Virtual kv-heads per kv-head for the stream-K path: 1 for groups of at
@@ -2539,19 +2869,25 @@ bool fused_applies(int batch, int q_heads, int kv_heads, int head_dim, int nkv, 
 // Chooses the automatic path from static shapes only.  `aligned` says
 // whether q/k/v/out are 16-byte aligned (the MFMA kernels' vector loads).
 int auto_plan(int batch, int q_heads, int kv_heads, int head_dim, int block_size, int max_pages,
-              int dtype, bool aligned, AutoPlan* ap, bool valu = false) {
-  *ap = AutoPlan{false, 0, 1, 1, false, false, 0, 0, 1, 0, kCounterBytes, 0, 1};
+              int dtype, bool aligned, AutoPlan* ap, bool valu = false, bool allow_general = true) {
+  *ap = AutoPlan{false, 0, 1, 1, false, false, 0, 0, 1, 0, kCounterBytes, 0, 1, false};
   if (batch <= 0) return QD_OK;
   const int split = kv_split_for(q_heads, kv_heads);
   const int vkv = kv_heads * (split > 0 ? split : 1);  // kv-heads as the stream-K kernel serves them
   const int gv = split > 0 ? kv_chunk_heads(q_heads, kv_heads, split) : 0;  // q-heads per one of them, at most
   const bool f32 = dtype == QD_DTYPE_F32;
-  if (aligned && split > 0 && (split == 1 || !valu) &&
-      (f32 ? !valu && f32_sk_applies(batch, q_heads, kv_heads, head_dim, block_size, max_pages, dtype)
-           : mfma_applies(vkv * gv, vkv, head_dim, block_size, dtype)) &&
-      batch <= kSkMaxBatch) {
+  const bool exact = f32 ? !valu && f32_sk_applies(batch, q_heads, kv_heads, head_dim, block_size, max_pages, dtype)
+                         : mfma_applies(vkv * gv, vkv, head_dim, block_size, dtype);
+  const int64_t gmax = static_cast<int64_t>(batch) * ((static_cast<int64_t>(max_pages) * block_size + 15) / 16);
+  const bool general = !exact && !valu && allow_general && general_applies(head_dim, dtype) &&
+                       (vkv == sk_wg_waves(vkv, 1, head_dim) || gmax > kGeneralFewGroups);
+  if (aligned && split > 0 && (split == 1 || !valu) && (exact || general) && batch <= kSkMaxBatch) {
     int nkv = 1;
-    const bool wide = !valu && !f32 && sk_wide_applies(vkv, head_dim);
+    const bool wide = !valu && !f32 && !general && sk_wide_applies(vkv, head_dim);
+    auto pick = [&](bool hold) {
+      return general ? pick_general_sk_dt(dtype, head_dim, hold)
+                     : pick_mfma_sk_dt(dtype, head_dim, nkv, wide && nkv == 1, false, hold);
+    };
     // fp32 at head_dim 128 holds 64 KB of K/V per group in flight: one wave
     // per SIMD (the 4-wave cap of the wide layout).
     int nw = sk_wg_waves(vkv, nkv, head_dim, valu, wide || (f32 && head_dim > 64));
@@ -2563,16 +2899,14 @@ int auto_plan(int batch, int q_heads, int kv_heads, int head_dim, int block_size
       }
     }
     const int g = gv;
-    KernelFn fn = valu ? pick_valu_sk_dt(dtype, g) : pick_mfma_sk_dt(dtype, head_dim, nkv, wide);
+    KernelFn fn = valu ? pick_valu_sk_dt(dtype, g) : pick(false);
     int resident = resident_blocks(fn, 64 * nw);
-    if (!valu && !f32 && split == 1 && sk_dual_applies(batch, kv_heads, head_dim, block_size, max_pages, resident)) {
+    if (!valu && !f32 && !general && split == 1 && sk_dual_applies(batch, kv_heads, head_dim, block_size, max_pages, resident)) {
       nkv = 2;
       nw = sk_wg_waves(kv_heads, nkv, head_dim);
       fn = pick_mfma_sk_dt(dtype, head_dim, nkv);
       resident = resident_blocks(fn, 64 * nw);
     }
-    const int64_t gmax = static_cast<int64_t>(batch) *
-                         ((static_cast<int64_t>(max_pages) * block_size + 15) / 16);
     const int64_t by_work = (gmax + kSkMinGroups - 1) / kSkMinGroups;
     const int64_t group_bytes = int64_t{16} * kv_heads * head_dim * 2 * (dtype == QD_DTYPE_F32 ? 4 : 2);
     const int64_t by_bytes = (gmax * group_bytes + kSkWgBytes - 1) / kSkWgBytes;
@@ -2593,7 +2927,7 @@ int auto_plan(int batch, int q_heads, int kv_heads, int head_dim, int block_size
     // while with two kv-heads per wave (Gemma-2-9B's shape) holding was level.
     const bool one_per_simd = nkv == 1 && (wide || head_dim > 128 || (f32 && head_dim > 64));
     if (!valu && !(one_per_simd && nw == vkv) && hold_results(batch, w)) {
-      const KernelFn hfn = pick_mfma_sk_dt(dtype, head_dim, nkv, wide && nkv == 1, false, true);
+      const KernelFn hfn = pick(true);
       ap->stage_bytes = stage_lds_bytes(g, head_dim, nkv, nw);
       if (!allow_dyn_lds(hfn)) return fail(QD_ERR_INVALID_VALUE, "dynamic LDS limit not raised");
       w = grid(resident_blocks(hfn, 64 * nw, ap->stage_bytes));
@@ -2606,6 +2940,7 @@ int auto_plan(int batch, int q_heads, int kv_heads, int head_dim, int block_size
       if (prod.stream_k && w > prod.wgs) w = prod.wgs;
     }
     ap->stream_k = true;
+    ap->general = general;
     ap->kv_split = split;
     ap->wgs = static_cast<int>(w);
     ap->wg_waves = nw;
@@ -2613,7 +2948,7 @@ int auto_plan(int batch, int q_heads, int kv_heads, int head_dim, int block_size
     ap->wide = wide && nkv == 1;
     ap->stash_bytes = fused_stash_bytes(vkv, head_dim, nkv, nw);  // used by the fused kernel only (split == 1)
     const KernelFn ffn = pick_mfma_sk_dt(dtype, head_dim, nkv, ap->wide, true);
-    if (kFusedByDefault && !valu && split == 1 && fused_applies(batch, q_heads, kv_heads, head_dim, nkv, w) &&
+    if (kFusedByDefault && !valu && !general && split == 1 && fused_applies(batch, q_heads, kv_heads, head_dim, nkv, w) &&
         ap->stash_bytes <= kFusedMaxStash && allow_dyn_lds(ffn)) {
       // The fused kernel's own occupancy (registers and the stash) bounds
       // the grid; without waits between workgroups a larger grid would
@@ -2665,6 +3000,17 @@ int check_launch_shapes(int batch, int q_heads, int kv_heads, int head_dim, int 
 uint64_t* g_stamps = nullptr;  // diagnostic build: qd_diag_set_stamps
 #endif
 
+// t / d = umulhi(2t, mul) >> shift for every 0 <= t < 2^31 (page_of): with
+// 2^(shift-1) < d <= 2^shift and mul = ceil(2^(31+shift) / d) <= 2^32 - 1, the
+// error mul*d - 2^(31+shift) is below d <= 2^shift, and t times it below
+// 2^(31+shift).
+void page_divisor(int d, uint32_t* mul, int* shift) {
+  int l = 0;
+  while ((int64_t{1} << l) < d) ++l;
+  *mul = static_cast<uint32_t>(((uint64_t{1} << (31 + l)) + d - 1) / d);
+  *shift = l;
+}
+
 DecodeParams make_params(const void* q, const void* k_cache, const void* v_cache,
                          const int32_t* block_table, const int32_t* context_lens, void* out,
                          void* workspace, int batch, int q_heads, int kv_heads, int head_dim,
@@ -2697,6 +3043,7 @@ DecodeParams make_params(const void* q, const void* k_cache, const void* v_cache
   prm.kv_split = 1;
   prm.kv_rows = kv_heads;
   prm.kv_g = prm.g;
+  page_divisor(block_size, &prm.page_mul, &prm.page_shift);
 #ifdef QD_STAMPS
   prm.stamps = g_stamps;
 #endif
@@ -2708,11 +3055,12 @@ DecodeParams make_params(const void* q, const void* k_cache, const void* v_cache
 // pointer alignment (QD_STAGE_VALU's plan runs on the same grid and fits).
 // 0 for invalid shapes.
 size_t auto_scratch_bytes(int batch, int q_heads, int kv_heads, int head_dim, int block_size, int max_pages,
-                          int dtype) {
+                          int dtype, bool allow_general = true) {
   if (check_launch_shapes(batch, q_heads, kv_heads, head_dim, block_size, max_pages, 1, dtype, 1.f) != QD_OK)
     return 0;
   AutoPlan a, b;
-  if (auto_plan(batch, q_heads, kv_heads, head_dim, block_size, max_pages, dtype, true, &a) != QD_OK ||
+  if (auto_plan(batch, q_heads, kv_heads, head_dim, block_size, max_pages, dtype, true, &a, false, allow_general) !=
+          QD_OK ||
       auto_plan(batch, q_heads, kv_heads, head_dim, block_size, max_pages, dtype, false, &b) != QD_OK)
     return 0;
   return a.ws_bytes > b.ws_bytes ? a.ws_bytes : b.ws_bytes;
@@ -2970,6 +3318,12 @@ int qd_gqa_decode_auto_stages(const void* q, const void* k_cache, const void* v_
   AutoPlan ap;
   st = auto_plan(batch, q_heads, kv_heads, head_dim, block_size, max_pages, dtype, aligned, &ap, valu);
   if (st != QD_OK) return st;
+  // The general layout takes whole calls, 32-bit pool rows, and a workspace
+  // of its plan's size; the split layout serves the rest.
+  if (ap.general && (stages != QD_STAGE_ALL || num_blocks * block_size > 2147483647LL || workspace_bytes < ap.ws_bytes)) {
+    st = auto_plan(batch, q_heads, kv_heads, head_dim, block_size, max_pages, dtype, aligned, &ap, valu, false);
+    if (st != QD_OK) return st;
+  }
   if (!workspace || workspace_bytes < ap.ws_bytes || !aligned16(workspace))
     return fail(QD_ERR_INVALID_VALUE, "workspace smaller than qd_gqa_decode_auto_workspace_bytes()");
   char* scratch = static_cast<char*>(workspace);
@@ -2983,7 +3337,7 @@ int qd_gqa_decode_auto_stages(const void* q, const void* k_cache, const void* v_
   }
   bool fused = ap.fused;
   if (unfused) fused = false;
-  if (force_fused) {
+  if (force_fused && !ap.general) {
     if (valu || dtype == QD_DTYPE_F32 || ap.kv_split > 1 || !fused_fits(batch, q_heads, kv_heads, head_dim, ap.wgs) ||
         ap.stash_bytes > kFusedMaxStash ||
         !allow_dyn_lds(pick_mfma_sk_dt(dtype, head_dim, ap.kv_per_wave, ap.wide, true)))
@@ -3007,6 +3361,14 @@ int qd_gqa_decode_auto_stages(const void* q, const void* k_cache, const void* v_
   }
   hipStream_t stm = static_cast<hipStream_t>(stream);
   (void)hipGetLastError();
+  if (ap.general) {
+    hipLaunchKernelGGL(pick_general_sk_dt(dtype, head_dim, ap.stage_bytes > 0), dim3(ap.wgs), dim3(64 * ap.wg_waves),
+                       ap.stage_bytes, stm, prm);
+    const bool one_head = merge_one_head_per_wave(batch, q_heads);
+    hipLaunchKernelGGL(pick_general_merge_dt(dtype, head_dim, one_head),
+                       dim3(one_head ? q_heads : (q_heads + 3) / 4, batch), dim3(64), 0, stm, prm);
+    return launch_error();
+  }
   if (fused) {
     // One kernel: decode and merge.  QD_STAGE_MERGE alone has nothing to do.
     if (stages & QD_STAGE_DECODE)
@@ -3046,7 +3408,9 @@ int qd_gqa_decode_auto_noalloc(const void* q, const void* k_cache, const void* v
                                scale);
   if (st != QD_OK) return st;
   if (batch == 0) return QD_OK;
-  const size_t need = auto_scratch_bytes(batch, q_heads, kv_heads, head_dim, block_size, max_pages, dtype);
+  size_t need = auto_scratch_bytes(batch, q_heads, kv_heads, head_dim, block_size, max_pages, dtype);
+  if (need > kNoAllocScratchBytes)  // what the split layout needs where the general one does not fit
+    need = auto_scratch_bytes(batch, q_heads, kv_heads, head_dim, block_size, max_pages, dtype, false);
   if (need > kNoAllocScratchBytes)
     return fail(QD_ERR_INVALID_VALUE, "shapes need " + std::to_string(need) +
                                           " bytes of scratch, more than the no-allocation scratch holds (" +
@@ -3065,6 +3429,9 @@ int qd_gqa_decode_auto_info(int batch, int q_heads, int kv_heads, int head_dim, 
     return -1;
   AutoPlan ap;
   if (auto_plan(batch, q_heads, kv_heads, head_dim, block_size, max_pages, dtype, true, &ap) != QD_OK)
+    return -1;
+  if (ap.general &&  // no stages there: reported as the split layout that serves what it does not take
+      auto_plan(batch, q_heads, kv_heads, head_dim, block_size, max_pages, dtype, true, &ap, false, false) != QD_OK)
     return -1;
   if (waves) *waves = ap.stream_k ? ap.wgs * ap.wg_waves : 0;
   if (splits) *splits = ap.splits;

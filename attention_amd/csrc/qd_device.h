@@ -197,8 +197,12 @@ struct MfmaOps<QD_DTYPE_F16> {
   }
   // fp16 keeps 11 significant bits: one rounding of the weights stays far
   // inside the 16-bit bar (measured 0.2 of it at worst), so no split.
+  // rest2 serves the kernels that split them all the same.
   static constexpr bool kSplitWeights = false;
-  __device__ static uint32_t rest2(float, float, uint32_t) { return 0u; }
+  __device__ static uint32_t rest2(float x, float y, uint32_t hi) {
+    const f32x2 v = __builtin_convertvector(__builtin_bit_cast(f16x2, hi), f32x2);
+    return pack2(x - v[0], y - v[1]);
+  }
 };
 
 // 8x8 transpose of 16-bit elements held in one lane: in[t] holds elements

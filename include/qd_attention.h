@@ -158,6 +158,12 @@ int qd_gqa_decode_kernel_kind(int q_heads, int kv_heads, int head_dim, int block
  *     workgroup to finish a piece of it (the fused merge, when the merge is
  *     short: see qd_gqa_decode_auto_info) or by a second kernel on the same
  *     stream;
+ *   - 16-bit caches with any other block_size, or a head_dim that is another
+ *     multiple of 8 up to 128 or of 16 up to 256 (same groups and batch,
+ *     num_blocks * block_size < 2^31): the same partition with the general
+ *     kernel, merged by a second kernel.  It serves whole calls only and is
+ *     reported as kind 0 by qd_gqa_decode_auto_info; with a workspace that
+ *     holds only the split layout's partials the split layout runs instead;
  *   - otherwise: the split layout of qd_gqa_decode_launch with the plan of
  *     qd_gqa_decode_plan.
  * The workspace is device memory, 16-byte aligned, of at least

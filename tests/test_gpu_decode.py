@@ -1078,3 +1078,71 @@ def test_generic_kernel_table_windows(gpu, shape):
         assert rc == 0, cabi.error_string(rc)
         torch.cuda.synchronize()
         assert_close(out, ref, DT_NAME[dtype], rows, f"splits={splits}")
+
+
+# (dtype, Hq, Hkv, D, P, lengths): the general layout of the balanced path, any
+# block_size and head_dims that are a multiple of 8 (of 16 above 128).
+GENERAL_SHAPES = [
+    (torch.float16, 32, 32, 80, 16, [1, 300, 2049, 0, 33]),                # head_dim 80, one q-head each
+    (torch.bfloat16, 32, 8, 80, 16, [17, 1000, 15, 16]),
+    (torch.bfloat16, 32, 8, 128, 8, [1, 7, 8, 9, 700, 3000]),              # groups over two pages
+    (torch.float16, 8, 2, 64, 1, [1, 16, 17, 511, 512, 513, 1700]),        # a page per token: several windows
+    (torch.bfloat16, 28, 4, 128, 3, [1537, 1536, 5, 4000]),                # windows ending inside a group
+    (torch.float16, 6, 3, 72, 12, [100, 1, 0, 999]),
+    (torch.bfloat16, 12, 12, 96, 24, [23, 24, 25, 1300]),                  # head_dim 96 on odd pages
+    (torch.float16, 5, 1, 8, 5, [3, 200]),                                 # the smallest head_dim
+    (torch.bfloat16, 16, 4, 40, 16, [300, 31]),
+    (torch.float16, 9, 3, 104, 16, [48, 777]),                             # a short last QK chunk
+    (torch.bfloat16, 8, 8, 112, 16, [1, 640, 1281]),
+    (torch.bfloat16, 16, 8, 160, 16, [65, 900, 2]),                        # the 256-column layout
+    (torch.float16, 8, 1, 192, 7, [6, 7, 8, 1500]),
+    (torch.bfloat16, 10, 2, 240, 32, [500, 33]),
+    (torch.float16, 16, 2, 256, 20, [19, 20, 21, 800]),
+    (torch.bfloat16, 40, 1, 80, 8, [129, 2500]),                           # 14 + 14 + 12 q-heads
+    (torch.float16, 32, 8, 80, 16, _fused_lengths(300, 1, 200, 141)),      # held result rows
+    (torch.bfloat16, 32, 1, 64, 1, _fused_lengths(300, 0, 120, 142)),
+    (torch.bfloat16, 8, 4, 192, 16, _fused_lengths(400, 1, 60, 143)),
+]
+
+
+@pytest.mark.parametrize("shape", GENERAL_SHAPES,
+                         ids=lambda s: f"{DT_NAME[s[0]]}-Hq{s[1]}-Hkv{s[2]}-D{s[3]}-P{s[4]}-B{len(s[5])}")
+def test_general_layout_matches_oracle(gpu, shape):
+    """Odd page sizes and head dims on the balanced path's general layout:
+    every row matches the oracle, with unused pages full of NaN/Inf and every
+    slot of the workspace NaN; the torch op gives the same bits.  A workspace
+    of the split layout's size runs the split layout instead, which matches
+    the oracle as well."""
+    dtype, hq, hkv, d, p, lengths = shape
+    say(f"general layout {DT_NAME[dtype]} Hq{hq} Hkv{hkv} D{d} P{p} B{len(lengths)}")
+    case = make_decode_case(lengths=lengths, q_heads=hq, kv_heads=hkv, head_dim=d, block_size=p, dtype=dtype, seed=144)
+    q, k, v, table, lens = to_dev(case, gpu)
+    ref, rows = oracle_rows((q, k, v, table, lens))
+    used = torch.zeros(k.shape[0], dtype=torch.bool)
+    for b, n in enumerate(lengths):
+        used[table[b, :-(-n // p)].long().cpu()] = True
+    k[~used.to(gpu)] = float("nan")
+    v[~used.to(gpu)] = float("inf")
+    for b, n in enumerate(lengths):
+        if n % p:  # unused slots of the last page
+            page = int(table[b, n // p])
+            k[page, n % p:] = float("inf")
+            v[page, n % p:] = float("nan")
+    maxp = table.shape[1]
+    ws = cabi.auto_workspace(len(lengths), hq, hkv, d, p, maxp, cabi.DTYPE[dtype], gpu, fill=0xFF)
+    out = torch.full_like(q, float("nan"))
+    rc = cabi.auto_launch(q, k, v, table, lens, out, scale=1 / math.sqrt(d), workspace=ws)
+    assert rc == 0, cabi.error_string(rc)
+    torch.cuda.synchronize()
+    assert_close(out, ref, DT_NAME[dtype], rows, "general layout")
+    assert torch.equal(out, attention_amd.gqa_decode(q, k, v, table, lens))
+    kind, waves, splits, _ = cabi.auto_info(len(lengths), hq, hkv, d, p, maxp, cabi.DTYPE[dtype])
+    assert (kind, waves) == (0, 0)
+    need = cabi.auto_counter_bytes() + cabi.lib().qd_gqa_decode_workspace_bytes(len(lengths), hq, d, splits)
+    if need >= ws.numel():
+        return  # the split layout's workspace holds the general plan's
+    split_out = torch.full_like(q, float("nan"))
+    rc = cabi.auto_launch(q, k, v, table, lens, split_out, scale=1 / math.sqrt(d), workspace=ws[:need])
+    assert rc == 0, cabi.error_string(rc)
+    torch.cuda.synchronize()
+    assert_close(split_out, ref, DT_NAME[dtype], rows, "split layout")
