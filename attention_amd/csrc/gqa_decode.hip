@@ -78,6 +78,7 @@ struct DecodeParams {
   float sl2;  // scale * log2(e)
   int* meta;      // stream-K path: per sequence {first workgroup, workgroups}
   int wg_waves;   // stream-K path: waves per workgroup
+  int kv_slices;  // stream-K path: workgroups (grid y) sharing a range's kv-heads
   uint32_t* ctr;  // fused stream-K path: arrival counter per (sequence, kv-head), zero between calls
   int stage_bytes;  // stream-K path: LDS bytes per wave for result rows held until the range ends
   // Stream-K path, groups of more than kMfmaHeads q-heads: each kv-head is
@@ -1844,7 +1845,9 @@ __device__ __forceinline__ uint32_t arrive(const DecodeParams& p, int b, int kvh
 // p.wg_waves waves; wave j of a workgroup serves kv-heads j*NKV .. j*NKV +
 // NKV-1, then the same plus wg_waves*NKV, ... so that a workgroup reads
 // whole cache rows (all kv-heads of a token) at once, which streams faster
-// from HBM than kv-head slices read at unrelated times.
+// from HBM than kv-head slices read at unrelated times.  A grid that leaves
+// CUs idle has p.kv_slices workgroups per range instead (grid y), which take
+// these passes in turn: slice y starts at pass y.
 //
 // Sequence b has n_b = ceil(len_b/16) groups and costs c_b = U*n_b + V
 // cost units (U = kSkGroupCost, V = kSkSeqCost; 0 when n_b = 0).  The
@@ -1883,6 +1886,7 @@ __global__ __launch_bounds__((64 * sk_max_waves<D, NKV, GV, PF, DT>())) void dec
   const int w = blockIdx.x;
   const int W = p.splits;
   const int B = p.B;
+  const int kv_slices = FUSED ? 1 : p.kv_slices;
   static_assert(DT != QD_DTYPE_F32 || (NKV == 1 && GV == 0 && !FUSED), "fp32 caches: one kv-head per wave, merge kernel");
   constexpr bool kGen = KCG > 0;
   static_assert(!kGen || (NKV == 1 && GV == 0 && !FUSED && DT != QD_DTYPE_F32), "general layout: one kv-head per wave");
@@ -1924,7 +1928,9 @@ __global__ __launch_bounds__((64 * sk_max_waves<D, NKV, GV, PF, DT>())) void dec
 
   // Empty sequences (no workgroup holds them): workgroup b % W writes their
   // zero rows (and, for merge_sk_kernel, a meta entry that says to skip them).
+  const int slice = FUSED ? 0 : static_cast<int>(blockIdx.y);
   auto zero_fill = [&](uint64_t mask, int c0) {
+    if (slice != 0) return;
     while (mask) {
       const int bb = c0 + __builtin_ctzll(mask);
       mask &= mask - 1;
@@ -2042,14 +2048,14 @@ __global__ __launch_bounds__((64 * sk_max_waves<D, NKV, GV, PF, DT>())) void dec
       const bool mid_range = cs + seq_cost(nb) < c1;
       if (FUSED && !whole && mid_range) sp_stashed = true;
       float* slot = p.ws + static_cast<int64_t>(w + b) * slot_floats;
-      for (int kvh0 = wid * NKV; kvh0 < p.Hkv; kvh0 += nw * NKV) {
+      for (int kvh0 = (slice * nw + wid) * NKV; kvh0 < p.Hkv; kvh0 += nw * NKV * kv_slices) {
         if constexpr (kGen)
           wv.begin_item_gen(p, b, kvh0, len, i0, i1);
         else
           wv.begin_item(p, b, kvh0, len, i0);
         // Every wave runs exactly one item here when the workgroup's waves
         // cover the kv-heads once, so all reach the same barriers.
-        wv.run(p, i0, i1, ktile[wid], p.Hkv == nw * NKV);
+        wv.run(p, i0, i1, ktile[wid], p.Hkv == nw * NKV * kv_slices);
         if constexpr (GV == 0 && FUSED) {
 #pragma unroll
           for (int j = 0; j < NKV; ++j) {
@@ -2119,7 +2125,7 @@ __global__ __launch_bounds__((64 * sk_max_waves<D, NKV, GV, PF, DT>())) void dec
         // workgroups span it, for merge_sk_kernel (also for a whole sequence,
         // so that nothing from an earlier call survives); wave 0 holds the
         // entry back with its result rows.
-        if (i0 == 0 && wid == 0) {
+        if (i0 == 0 && wid == 0 && slice == 0) {
           const int first = wg_of(x0);
           const int count = wg_of(x0 + kSkGroupCost * (nb - 1)) - first + 1;
           if constexpr (HOLD) {
@@ -2458,12 +2464,7 @@ using KernelFn = void (*)(DecodeParams);
 // layout's VALU kernel (us per call, bf16/fp16): B64 Hq32/Hkv8 D72 P16 196.1 ->
 // 26.8, B16 D160 P32 327.3 -> 45.4, B16 D256 P8 136.0 -> 55.6, B16 D128 P1
 // U[1000, 6000] 89.7 -> 47.0, B64 Hq8/Hkv2 D32 28.9 -> 15.5, B1 Hq8/Hkv1 D16
-// 11.3 -> 9.4.  The one loss is a handful of groups that a workgroup's waves
-// cover in several passes of kv-heads, one after the other (B1/L128 Hkv32 D80
-// 18.5 -> 19.1, B1/L64 Hkv8 D256 16.8 -> 17.6): at most kGeneralFewGroups
-// groups in the largest batch then stay on the split layout.
-constexpr int64_t kGeneralFewGroups = 8;
-
+// 11.3 -> 9.4.
 bool general_applies(int head_dim, int dtype) {
   return (dtype == QD_DTYPE_F16 || dtype == QD_DTYPE_BF16) &&
          (head_dim <= 128 ? head_dim % 8 == 0 : head_dim % 16 == 0 && head_dim <= 256);
@@ -2478,8 +2479,9 @@ KernelFn pick_general_sk(int head_dim) {
   if (head_dim <= 64) return decode_mfma_sk_kernel<64, DT, 3, 1, 0, false, HOLD, 2>;
   if (head_dim <= 96) return decode_mfma_sk_kernel<128, DT, 2, 1, 0, false, HOLD, 3>;
   if (head_dim <= 128) return decode_mfma_sk_kernel<128, DT, 2, 1, 0, false, HOLD, 4>;
-  if (head_dim <= 192) return decode_mfma_sk_kernel<256, DT, 2, 1, 0, false, HOLD, 6>;
-  return decode_mfma_sk_kernel<256, DT, 2, 1, 0, false, HOLD, 8>;
+  // One wave per SIMD: never held.
+  if (head_dim <= 192) return decode_mfma_sk_kernel<256, DT, 2, 1, 0, false, false, 6>;
+  return decode_mfma_sk_kernel<256, DT, 2, 1, 0, false, false, 8>;
 }
 
 KernelFn pick_general_sk_dt(int dtype, int head_dim, bool hold) {
@@ -2530,7 +2532,10 @@ constexpr int kSkWidePrefetch = 3;
 
 template <int DT, bool FUSED, bool HOLD>
 KernelFn pick_mfma_sk(int D, int nkv, bool wide) {
-  if (wide) return decode_mfma_sk_kernel<128, DT, kSkWidePrefetch, 1, 0, FUSED, HOLD>;
+  if constexpr (!HOLD) {  // one wave per SIMD: rows are stored after each item (auto_plan)
+    if (wide) return decode_mfma_sk_kernel<128, DT, kSkWidePrefetch, 1, 0, FUSED, HOLD>;
+    if (D == 256) return decode_mfma_sk_kernel<256, DT, 2, 1, 0, FUSED, HOLD>;
+  }
   if (nkv == 2) {
     switch (D) {
       case 64: return decode_mfma_sk_kernel<64, DT, kPrefetchDual, 2, 0, FUSED, HOLD>;
@@ -2540,8 +2545,7 @@ KernelFn pick_mfma_sk(int D, int nkv, bool wide) {
   switch (D) {
     case 64: return decode_mfma_sk_kernel<64, DT, kPrefetch64, 1, 0, FUSED, HOLD>;
     case 96: return decode_mfma_sk_kernel<96, DT, kPrefetch, 1, 0, FUSED, HOLD>;
-    case 128: return decode_mfma_sk_kernel<128, DT, kPrefetch, 1, 0, FUSED, HOLD>;
-    default: return decode_mfma_sk_kernel<256, DT, 2, 1, 0, FUSED, HOLD>;
+    default: return decode_mfma_sk_kernel<128, DT, kPrefetch, 1, 0, FUSED, HOLD>;
   }
 }
 
@@ -2553,8 +2557,7 @@ KernelFn pick_mfma_sk_dt(int dtype, int D, int nkv, bool wide = false, bool fuse
     if (D == 64)
       return hold ? decode_mfma_sk_kernel<64, QD_DTYPE_F32, kPrefetch, 1, 0, false, true>
                   : decode_mfma_sk_kernel<64, QD_DTYPE_F32, kPrefetch, 1, 0, false, false>;
-    return hold ? decode_mfma_sk_kernel<128, QD_DTYPE_F32, kPrefetch, 1, 0, false, true>
-                : decode_mfma_sk_kernel<128, QD_DTYPE_F32, kPrefetch, 1, 0, false, false>;
+    return decode_mfma_sk_kernel<128, QD_DTYPE_F32, kPrefetch, 1, 0, false, false>;
   }
   if (fused)
     return f16 ? pick_mfma_sk<QD_DTYPE_F16, true, false>(D, nkv, wide)
@@ -2781,6 +2784,23 @@ int sk_wg_waves(int kv_heads, int nkv, int head_dim, bool valu = false, bool wid
   return 1;
 }
 
+// Workgroups per range (DecodeParams::kv_slices) for waves that need `passes`
+// passes over the kv-heads: one per pass, on resident / passes ranges.  A
+// workgroup that walked the passes itself restarted its pipeline for each of
+// them on a range `passes` times shorter, and wrote (and merged) as many times
+// more partial rows; a pass over 4 or 8 kv-heads already reads 1 KB or more
+// of a token row at once.  Us per call, walking -> sliced: bf16 Hkv32 D128
+// B1/L100 18.4 -> 10.0, B1/L1000 24.7 -> 12.6, B16 U[100, 1000] 36.9 -> 31.2,
+// B32 U[500, 4096] (1.2 GB) 201.3 -> 190.9; Hkv16 D128 B16 U[1256, 4048] 77.9 ->
+// 62.4; Hkv32 D80 fp16 B16 U[256, 2048] 57.0 -> 49.7; Hkv8 D256 B8 U[1000,
+// 12000] 79.7 -> 71.4; fp32 Hkv8 D128 B16/L4096 112.9 -> 91.0; 24 virtual
+// kv-heads 69.3 -> 35.1.
+int kv_slices_for(int passes, int resident) {
+  for (int n = passes; n > 1; --n)
+    if (passes % n == 0 && n <= resident) return n;
+  return 1;
+}
+
 // Arrival counters of the fused stream-K path: one 32-bit word per
 // (sequence, kv-head), at the start of every automatic-path workspace.  The
 // place and size are fixed, so calls of any shape sharing a workspace never
@@ -2820,6 +2840,7 @@ struct AutoPlan {
   size_t meta_offset;  // stream-K: byte offset of the meta table in the scratch
   int kv_split;     // stream-K: virtual kv-heads per kv-head (DecodeParams::kv_split)
   bool general;     // stream-K: the general layout (general_applies)
+  int kv_slices;    // stream-K: workgroups per range (DecodeParams::kv_slices)
 };
 
 // Virtual kv-heads per kv-head for the stream-K path: 1 for groups of at
@@ -2870,7 +2891,7 @@ bool fused_applies(int batch, int q_heads, int kv_heads, int head_dim, int nkv, 
 // whether q/k/v/out are 16-byte aligned (the MFMA kernels' vector loads).
 int auto_plan(int batch, int q_heads, int kv_heads, int head_dim, int block_size, int max_pages,
               int dtype, bool aligned, AutoPlan* ap, bool valu = false, bool allow_general = true) {
-  *ap = AutoPlan{false, 0, 1, 1, false, false, 0, 0, 1, 0, kCounterBytes, 0, 1, false};
+  *ap = AutoPlan{false, 0, 1, 1, false, false, 0, 0, 1, 0, kCounterBytes, 0, 1, false, 1};
   if (batch <= 0) return QD_OK;
   const int split = kv_split_for(q_heads, kv_heads);
   const int vkv = kv_heads * (split > 0 ? split : 1);  // kv-heads as the stream-K kernel serves them
@@ -2879,8 +2900,7 @@ int auto_plan(int batch, int q_heads, int kv_heads, int head_dim, int block_size
   const bool exact = f32 ? !valu && f32_sk_applies(batch, q_heads, kv_heads, head_dim, block_size, max_pages, dtype)
                          : mfma_applies(vkv * gv, vkv, head_dim, block_size, dtype);
   const int64_t gmax = static_cast<int64_t>(batch) * ((static_cast<int64_t>(max_pages) * block_size + 15) / 16);
-  const bool general = !exact && !valu && allow_general && general_applies(head_dim, dtype) &&
-                       (vkv == sk_wg_waves(vkv, 1, head_dim) || gmax > kGeneralFewGroups);
+  const bool general = !exact && !valu && allow_general && general_applies(head_dim, dtype);
   if (aligned && split > 0 && (split == 1 || !valu) && (exact || general) && batch <= kSkMaxBatch) {
     int nkv = 1;
     const bool wide = !valu && !f32 && !general && sk_wide_applies(vkv, head_dim);
@@ -2918,19 +2938,28 @@ int auto_plan(int batch, int q_heads, int kv_heads, int head_dim, int block_size
       return w < 1 ? int64_t{1} : w;
     };
     int64_t w = grid(resident);
+    auto slice = [&] {
+      if (valu) return;
+      ap->kv_slices = kv_slices_for(vkv / (nkv * nw), resident);
+      w = std::min<int64_t>(w, resident / ap->kv_slices);
+    };
+    slice();
     // Result rows held in LDS until the range ends: the kernel's occupancy
     // with that LDS sets the grid.  Not where each wave runs alone on its
     // SIMD and serves a single kv-head per sequence (4 kv-heads at head_dim
-    // 128, head_dim 256 or fp32 head_dim 128 with at most 4 kv-heads): there
-    // the stores after each item measured faster (graph replays, B128/L1024:
-    // Qwen2.5-7B's shape 51.5 -> 47.2 us, Gemma-2-2B's 96.2 -> 87.4 us),
-    // while with two kv-heads per wave (Gemma-2-9B's shape) holding was level.
+    // 128, head_dim 256, fp32 head_dim 128: kv_slices_for gives every pass its
+    // workgroups): there the stores after each item measured faster (B128
+    // U[500, 1500] Hkv8 D256 179.4 held, 165.8 us stored; fp32 D128 199.7 and
+    // 171.6; Qwen2.5-7B's shape at B128/L1024 51.5 and 47.2), while with two
+    // kv-heads per wave (Gemma-2-9B's shape) holding was level.
     const bool one_per_simd = nkv == 1 && (wide || head_dim > 128 || (f32 && head_dim > 64));
-    if (!valu && !(one_per_simd && nw == vkv) && hold_results(batch, w)) {
+    if (!valu && !one_per_simd && hold_results(batch, w)) {
       const KernelFn hfn = pick(true);
       ap->stage_bytes = stage_lds_bytes(g, head_dim, nkv, nw);
       if (!allow_dyn_lds(hfn)) return fail(QD_ERR_INVALID_VALUE, "dynamic LDS limit not raised");
-      w = grid(resident_blocks(hfn, 64 * nw, ap->stage_bytes));
+      resident = resident_blocks(hfn, 64 * nw, ap->stage_bytes);
+      w = grid(resident);
+      slice();
     }
     if (valu) {
       // The comparison variant runs on the product plan's grid (and fits its
@@ -3038,6 +3067,7 @@ DecodeParams make_params(const void* q, const void* k_cache, const void* v_cache
   prm.sl2 = scale * kLog2e;
   prm.meta = nullptr;
   prm.wg_waves = 1;
+  prm.kv_slices = 1;
   prm.ctr = nullptr;
   prm.stage_bytes = 0;
   prm.kv_split = 1;
@@ -3351,6 +3381,7 @@ int qd_gqa_decode_auto_stages(const void* q, const void* k_cache, const void* v_
   prm.meta = reinterpret_cast<int*>(scratch + ap.meta_offset);
   prm.ctr = reinterpret_cast<uint32_t*>(scratch);
   prm.wg_waves = ap.wg_waves;
+  prm.kv_slices = fused ? 1 : ap.kv_slices;
   prm.stage_bytes = ap.stage_bytes ? static_cast<int>(ap.stage_bytes / ap.wg_waves) : 0;
   if (ap.kv_split > 1) {
     prm.Hkv = kv_heads * ap.kv_split;
@@ -3362,7 +3393,7 @@ int qd_gqa_decode_auto_stages(const void* q, const void* k_cache, const void* v_
   hipStream_t stm = static_cast<hipStream_t>(stream);
   (void)hipGetLastError();
   if (ap.general) {
-    hipLaunchKernelGGL(pick_general_sk_dt(dtype, head_dim, ap.stage_bytes > 0), dim3(ap.wgs), dim3(64 * ap.wg_waves),
+    hipLaunchKernelGGL(pick_general_sk_dt(dtype, head_dim, ap.stage_bytes > 0), dim3(ap.wgs, ap.kv_slices), dim3(64 * ap.wg_waves),
                        ap.stage_bytes, stm, prm);
     const bool one_head = merge_one_head_per_wave(batch, q_heads);
     hipLaunchKernelGGL(pick_general_merge_dt(dtype, head_dim, one_head),
@@ -3379,7 +3410,7 @@ int qd_gqa_decode_auto_stages(const void* q, const void* k_cache, const void* v_
   if (stages & QD_STAGE_DECODE)
     hipLaunchKernelGGL(valu ? pick_valu_sk_dt(dtype, q_heads / kv_heads)
                             : pick_mfma_sk_dt(dtype, head_dim, ap.kv_per_wave, ap.wide, false, ap.stage_bytes > 0),
-                       dim3(ap.wgs), dim3(64 * ap.wg_waves), ap.stage_bytes, stm, prm);
+                       dim3(ap.wgs, ap.kv_slices), dim3(64 * ap.wg_waves), ap.stage_bytes, stm, prm);
   if (stages & QD_STAGE_MERGE) {
     const bool one_head = merge_one_head_per_wave(batch, q_heads);
     hipLaunchKernelGGL(pick_merge_sk_dt(dtype, head_dim, one_head),
@@ -3433,7 +3464,7 @@ int qd_gqa_decode_auto_info(int batch, int q_heads, int kv_heads, int head_dim, 
   if (ap.general &&  // no stages there: reported as the split layout that serves what it does not take
       auto_plan(batch, q_heads, kv_heads, head_dim, block_size, max_pages, dtype, true, &ap, false, false) != QD_OK)
     return -1;
-  if (waves) *waves = ap.stream_k ? ap.wgs * ap.wg_waves : 0;
+  if (waves) *waves = ap.stream_k ? ap.wgs * ap.kv_slices * ap.wg_waves : 0;
   if (splits) *splits = ap.splits;
   if (chunk_pages) *chunk_pages = ap.chunk_pages;
   return ap.stream_k ? (ap.fused ? 2 : 1) : 0;
