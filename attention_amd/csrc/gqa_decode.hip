@@ -15,9 +15,11 @@
 //                          A sequence split across workgroups leaves
 //                          {m, l, acc} partials that merge_sk_kernel
 //                          combines.
-//   decode_mfma_kernel     the same per-wave pipeline over the reference's
-//                          explicit split layout: one wave per (sequence,
-//                          kv-head, split), partials [B,Hq,S,D+2].
+//   decode_wg_kernel       the same per-wave pipeline, one workgroup per
+//                          (sequence, kv-head, split), its waves' states
+//                          merged through LDS: short contexts as one launch,
+//                          and the reference's explicit split layout,
+//                          partials [B,Hq,S,D+2].
 //   decode_generic_kernel  every other shape/dtype the reference accepts
 //                          (fp32, any head_dim in [1,256], any block_size,
 //                          any group size) on the VALU: 16 lanes per token
@@ -1096,6 +1098,8 @@ struct MfmaWaveF32 : MfmaWave<D, QD_DTYPE_F32, PF, 1> {
   }
 };
 
+constexpr int kGenWinPages = 512;  // page-table window of the general layout (LDS, per wave)
+
 // One wave's decode state for one kv-head in the general layout: 16-bit
 // caches with any block_size and any head_dim Dm = p.D that is a multiple of
 // 8 up to 128 or of 16 up to 256 (VD = 64, 128 or 256 is the next V layout,
@@ -1126,7 +1130,7 @@ struct GenWave : MfmaWave<VD, DT, PF, 1> {
   static constexpr int EV = VD / 16;                // V elements per lane and row
   static constexpr int kStride = 64 * KCG + 32;     // LDS bytes per K row
   static constexpr int kTileBytes = 16 * kStride;
-  static constexpr int kWinPages = 512;             // table window (LDS)
+  static constexpr int kWinPages = kGenWinPages;
   struct Buf {
     u32x4 k[KCG];
     VRow<VD> v[4];
@@ -1563,33 +1567,6 @@ struct ValuWave : MfmaWave<D, DT, PF, 1> {
   }
 };
 
-// Explicit split layout.  grid: (splits, Hkv, B), block 64 (one wave per
-// (sequence, kv-head, split)).  Split z of a sequence covers whole pages
-// (chunk_info); a sequence with a single non-empty split is written
-// directly, otherwise every non-empty split writes its partial to
-// ws[b, h, z, :] for the split merge (combine_rows_kernel / combine_kernel).
-template <int D, int DT, int PF>
-__global__ __launch_bounds__(64) void decode_mfma_kernel(DecodeParams p) {
-  const int z = blockIdx.x;
-  const int kvh = blockIdx.y;
-  const int b = blockIdx.z;
-  const ChunkInfo ci = chunk_info(p, p.lens[b], z);
-  if (z >= (ci.nch > 1 ? ci.nch : 1)) return;
-
-  __shared__ __align__(16) char ktile[KTile<D>::kBytes];
-  MfmaWave<D, DT, PF, 1> wv;
-  wv.init_lane();
-  wv.begin_item(p, b, kvh, ci.te, ci.tb >> 4);
-  wv.run(p, ci.tb >> 4, (ci.te + 15) >> 4, ktile);  // tb is page aligned
-  const float l_tot = wv.total_l(0);
-  if (ci.nch <= 1) {
-    wv.store_direct(p, b, kvh, 0, l_tot);
-  } else {
-    float* w = p.ws + ((static_cast<int64_t>(b) * p.Hq + kvh * p.g) * p.splits + z) * (D + 2);
-    wv.store_partial(p, 0, w, static_cast<int64_t>(p.splits) * (D + 2), l_tot);
-  }
-}
-
 // 16-token groups of a sequence with `len` valid tokens.
 __device__ __forceinline__ int seq_groups(const DecodeParams& p, int len_raw) {
   return (clamp_len(p, len_raw) + 15) >> 4;
@@ -1740,6 +1717,157 @@ constexpr int sk_max_waves() {
   if (GV > 0) return kValuMaxWaves;
   if (DT == QD_DTYPE_F32) return D <= 64 ? kMaxWgWaves : kMaxWgWaves / 2;  // fp32 head_dim 128: 512 registers
   return (NKV == 1 && D <= 128 && (PF <= 2 || D <= 64)) ? kMaxWgWaves : kMaxWgWaves / 2;
+}
+
+// LDS of decode_wg_kernel for nw waves: a K tile (and, in the general layout,
+// a table window) per wave, and in the same place, once every wave is done
+// with them, the waves' accumulators ([wave][i][4-column piece][lane], 16
+// bytes each) and {m, l}.
+template <int D, int DT, int KCG>
+constexpr int wg_wave_tile_bytes() {
+  if (KCG > 0) return 16 * (64 * KCG + 32) + 4 * kGenWinPages;
+  return KTile<D, DT == QD_DTYPE_F32 ? 4 : 2>::kBytes;
+}
+constexpr int wg_wave_merge_bytes(int vd) { return (vd / 16) * 1024 + 512; }
+
+// One workgroup per (sequence, kv-head, split): grid (splits, Hkv, B), block
+// 64 * p.wg_waves.  Split z of a sequence covers whole pages (chunk_info;
+// without splits, the sequence); its 16-token groups go to the waves in
+// contiguous runs, each wave streams its run (MfmaWave and its variants), and
+// the waves' softmax states are merged through LDS (SoftmaxState::merge,
+// online_softmax.cuh:17-24, over all waves at once): wave i merges and stores
+// column pieces i, i + waves, .. of 4.  A sequence with a single non-empty
+// split is written directly, otherwise every non-empty split writes its
+// partial to ws[b, h, z, :] for the split merge (combine_rows_kernel /
+// combine_kernel).
+//
+// Bound by latency: the chain of length, table, K/V and the waves' groups one
+// after the other (the figures stand at wg_single_applies and wg_waves_for).
+// A lane keeps its own head and columns through the merge, so the exchange is
+// lane-contiguous 16-byte LDS accesses without conflicts.
+template <int D, int DT, int PF, int KCG = 0>
+__global__ __launch_bounds__((64 * sk_max_waves<D, 1, 0, PF, DT>())) void decode_wg_kernel(DecodeParams p) {
+  using S = typename Elem<DT>::S;
+  constexpr bool kGen = KCG > 0;
+  constexpr int DV = D / 16;
+  constexpr int kW = DV % 4 == 0 ? 4 : 2;  // floats per piece (head_dim 96: 6 columns per lane)
+  using Piece = std::conditional_t<kW == 4, f32x4, f32x2>;
+  constexpr int kPieces = DV / kW;
+  constexpr int kTile = wg_wave_tile_bytes<D, DT, KCG>();
+  const int z = blockIdx.x;
+  const int kvh = blockIdx.y;
+  const int b = blockIdx.z;
+  const ChunkInfo ci = chunk_info(p, p.lens[b], z);
+  if (z >= (ci.nch > 1 ? ci.nch : 1)) return;
+
+  extern __shared__ __align__(16) char wg_lds[];
+  const int lane = threadIdx.x & 63;
+  const int wid = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
+  const int dm = kGen ? p.D : D;
+  using Wave = std::conditional_t<
+      DT == QD_DTYPE_F32, MfmaWaveF32<D, PF>,
+      std::conditional_t<kGen, GenWave<D, kGen ? KCG : 1, DT, PF>, MfmaWave<D, DT, PF, 1>>>;
+  Wave wv;
+  char* tile = wg_lds + wid * kTile;
+  if constexpr (kGen)
+    wv.init_lane_gen(p, tile, reinterpret_cast<int32_t*>(tile + Wave::kTileBytes));
+  else
+    wv.init_lane();
+
+  const int ga = ci.tb >> 4;  // tb is 0 or a multiple of a page of whole groups
+  const int n = ((ci.te + 15) >> 4) - ga;
+  const int per = (n + p.wg_waves - 1) / p.wg_waves;
+  const int act = per > 0 ? (n + per - 1) / per : 0;  // waves with groups: the first `act`
+  const int g0 = ga + wid * per;
+  const int g1 = min(g0 + per, ga + n);
+  float l_tot = 0.f;
+  if (wid < act) {
+    if constexpr (kGen)
+      wv.begin_item_gen(p, b, kvh, ci.te, g0, g1);
+    else
+      wv.begin_item(p, b, kvh, ci.te, g0);
+    wv.run(p, g0, g1, tile);
+    l_tot = wv.total_l(0);
+  } else {
+    wv.hcount = vhead_count(p, kvh);
+    wv.m_run[0] = -INFINITY;
+#pragma unroll
+    for (int d = 0; d < DV; ++d) wv.acc[0][d] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+  const int64_t row0 = static_cast<int64_t>(b) * p.Hq + vhead_base(p, kvh);
+  const int64_t head_stride = static_cast<int64_t>(p.splits) * (dm + 2);
+  float* part = p.ws + (row0 * p.splits + z) * (dm + 2);
+  if (act <= 1) {  // uniform
+    if (wid == 0) {
+      if (ci.nch <= 1)
+        wv.store_direct(p, b, kvh, 0, l_tot);
+      else
+        wv.store_partial(p, 0, part, head_stride, l_tot);
+    }
+    return;
+  }
+
+  __syncthreads();  // the tiles' place is free
+  Piece* accs = reinterpret_cast<Piece*>(wg_lds);
+  f32x2* mls = reinterpret_cast<f32x2*>(wg_lds + p.wg_waves * DV * 1024);
+  if (wid < act) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int c = 0; c < kPieces; ++c) {
+        Piece a;
+#pragma unroll
+        for (int t = 0; t < kW; ++t) a[t] = wv.acc[0][kW * c + t][i];
+        accs[((wid * 4 + i) * kPieces + c) * 64 + lane] = a;
+      }
+    mls[wid * 64 + lane] = f32x2{wv.m_run[0], l_tot};
+  }
+  __syncthreads();
+  float M = -INFINITY;
+  for (int u = 0; u < act; ++u) {
+    const f32x2 ml = mls[u * 64 + lane];
+    if (ml[1] != 0.f) M = fmaxf(M, ml[0]);
+  }
+  const bool head_ok = wv.r16 < wv.hcount;
+  for (int i = wid; i < 4; i += p.wg_waves) {
+    float L = 0.f;
+    float o[DV];
+#pragma unroll
+    for (int d = 0; d < DV; ++d) o[d] = 0.f;
+    for (int u = 0; u < act; ++u) {
+      const f32x2 ml = mls[u * 64 + lane];
+      const float w = ml[1] == 0.f ? 0.f : fast_exp2(ml[0] - M);
+      L = fmaf(w, ml[1], L);
+#pragma unroll
+      for (int c = 0; c < kPieces; ++c) {
+        const Piece a = accs[((u * 4 + i) * kPieces + c) * 64 + lane];
+#pragma unroll
+        for (int t = 0; t < kW; ++t) o[kW * c + t] = fmaf(w, a[t], o[kW * c + t]);
+      }
+    }
+    const int col = DV * (4 * wv.q4 + i);
+    if (!head_ok || (kGen && col >= dm)) continue;
+    if (ci.nch <= 1) {
+      const float inv = L > 0.f ? 1.f / L : 0.f;
+#pragma unroll
+      for (int d = 0; d < DV; ++d) o[d] = L > 0.f ? o[d] * inv : 0.f;
+      S* dst = static_cast<S*>(p.out) + (row0 + wv.r16) * dm + col;
+      if constexpr (DT == QD_DTYPE_F32) {
+#pragma unroll
+        for (int d = 0; d < DV; d += 4) *reinterpret_cast<f32x4*>(dst + d) = f32x4{o[d], o[d + 1], o[d + 2], o[d + 3]};
+      } else {
+        uint32_t wd[DV / 2];
+#pragma unroll
+        for (int d = 0; d < DV; d += 2) wd[d / 2] = MfmaOps<DT>::pack2(o[d], o[d + 1]);
+        store_words<DV / 2>(reinterpret_cast<char*>(dst), wd);
+      }
+    } else {
+      float* w = part + wv.r16 * head_stride;
+      if (i == 0 && wv.q4 == 0) *reinterpret_cast<f32x2*>(w) = f32x2{M * kLn2, L};
+#pragma unroll
+      for (int d = 0; d < DV; d += 2) *reinterpret_cast<f32x2*>(w + 2 + col + d) = f32x2{o[d], o[d + 1]};
+    }
+  }
 }
 
 #ifndef QD_SK_SEQ_COST
@@ -2396,10 +2524,28 @@ constexpr int kMfmaHeads = 16;
 // measured slower.
 constexpr int64_t kF32SkTokens = 65536;
 
+// fp32 shapes that MfmaWaveF32 serves.
+bool f32_mfma_applies(int q_heads, int kv_heads, int head_dim, int block_size, int dtype) {
+  return dtype == QD_DTYPE_F32 && (head_dim == 64 || head_dim == 128) && block_size % 16 == 0 && kv_heads > 0 &&
+         q_heads % kv_heads == 0 && q_heads / kv_heads <= kMfmaHeads;
+}
+
+// The same kernel below that capacity, as a whole call only (stages and
+// qd_gqa_decode_auto_info keep the split layout there): since its kv-head
+// passes have workgroups of their own it wins from kF32GeneralTokens of
+// capacity on (Hq32/Hkv8 D128, us per call, split layout -> balanced: B16
+// U[64, 1024] 24.5 -> 20.4, B16/L1024 33.8 -> 32.4, B4/L4096 33.9 -> 32.2, Hkv1
+// B40 U[300, 1000] 25.4 -> 16.8; B4/L1024 16.5 -> 16.4, B1/L1024 11.9 -> 14.1).
+constexpr int64_t kF32GeneralTokens = 16384;
+
+bool f32_general_applies(int batch, int q_heads, int kv_heads, int head_dim, int block_size, int max_pages, int dtype) {
+  return f32_mfma_applies(q_heads, kv_heads, head_dim, block_size, dtype) &&
+         static_cast<int64_t>(batch) * max_pages * block_size >= kF32GeneralTokens;
+}
+
 bool f32_sk_applies(int batch, int q_heads, int kv_heads, int head_dim, int block_size, int max_pages, int dtype) {
-  if (dtype != QD_DTYPE_F32 || (head_dim != 64 && head_dim != 128) || block_size % 16 != 0) return false;
-  if (static_cast<int64_t>(batch) * max_pages * block_size < kF32SkTokens) return false;
-  return kv_heads > 0 && q_heads % kv_heads == 0 && q_heads / kv_heads <= kMfmaHeads;
+  return f32_mfma_applies(q_heads, kv_heads, head_dim, block_size, dtype) &&
+         static_cast<int64_t>(batch) * max_pages * block_size >= kF32SkTokens;
 }
 
 bool mfma_applies(int q_heads, int kv_heads, int head_dim, int block_size, int dtype) {
@@ -2505,14 +2651,45 @@ KernelFn pick_general_merge_dt(int dtype, int head_dim, bool one_head) {
   return one_head ? pick_general_merge<QD_DTYPE_BF16, 16, 4>(head_dim) : pick_general_merge<QD_DTYPE_BF16, 8, 1>(head_dim);
 }
 
+// decode_wg_kernel for a head_dim: exact layout (fp32: 64 or 128) or general.
 template <int DT>
-KernelFn pick_mfma(int D) {
+KernelFn pick_wg(int D) {
   switch (D) {
-    case 64: return decode_mfma_kernel<64, DT, kPrefetch>;
-    case 96: return decode_mfma_kernel<96, DT, kPrefetch>;
-    case 128: return decode_mfma_kernel<128, DT, kPrefetch>;
-    default: return decode_mfma_kernel<256, DT, 2>;
+    case 64: return decode_wg_kernel<64, DT, kPrefetch64>;
+    case 96: return decode_wg_kernel<96, DT, kPrefetch>;
+    case 128: return decode_wg_kernel<128, DT, kPrefetch>;
+    default: return decode_wg_kernel<256, DT, 2>;
   }
+}
+
+template <int DT>
+KernelFn pick_wg_general(int D) {
+  if (D <= 64) return decode_wg_kernel<64, DT, 3, 2>;
+  if (D <= 96) return decode_wg_kernel<128, DT, 2, 3>;
+  if (D <= 128) return decode_wg_kernel<128, DT, 2, 4>;
+  if (D <= 192) return decode_wg_kernel<256, DT, 2, 6>;
+  return decode_wg_kernel<256, DT, 2, 8>;
+}
+
+KernelFn pick_wg_dt(int dtype, int D, bool general) {
+  if (dtype == QD_DTYPE_F32)
+    return D == 64 ? decode_wg_kernel<64, QD_DTYPE_F32, kPrefetch> : decode_wg_kernel<128, QD_DTYPE_F32, kPrefetch>;
+  if (dtype == QD_DTYPE_F16) return general ? pick_wg_general<QD_DTYPE_F16>(D) : pick_wg<QD_DTYPE_F16>(D);
+  return general ? pick_wg_general<QD_DTYPE_BF16>(D) : pick_wg<QD_DTYPE_BF16>(D);
+}
+
+// Dynamic LDS of a decode_wg_kernel workgroup of nw waves.
+size_t wg_lds_bytes(int dtype, int D, bool general, int nw) {
+  const int vd = general ? general_vd(D) : D;
+  const int es = dtype == QD_DTYPE_F32 ? 4 : 2;
+  const int kc = D <= 64 ? 2 : D <= 96 ? 3 : D <= 128 ? 4 : D <= 192 ? 6 : 8;
+  const int tile = general ? 16 * (64 * kc + 32) + 2048 : 16 * (es * D + 32);
+  return static_cast<size_t>(nw) * std::max(tile, wg_wave_merge_bytes(vd));
+}
+
+// Most waves of a decode_wg_kernel workgroup (its launch bounds).
+int wg_max_waves(int dtype, int D) {
+  return D > 128 || (dtype == QD_DTYPE_F32 && D > 64) ? kMaxWgWaves / 2 : kMaxWgWaves;
 }
 
 #ifndef QD_PREFETCH_DUAL
@@ -2670,7 +2847,7 @@ int resident_blocks(KernelFn fn, int threads, size_t dyn_lds = 0) {
     int blocks;
   };
   static std::mutex mu;
-  static Entry cache[64];
+  static Entry cache[256];
   static int used = 0;
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess) dev = 0;
@@ -2687,7 +2864,7 @@ int resident_blocks(KernelFn fn, int threads, size_t dyn_lds = 0) {
     per_cu = 1;
   (void)hipGetLastError();
   const int blocks = cus * per_cu;
-  if (used < 64) cache[used++] = Entry{dev, fn, threads, dyn_lds, blocks};
+  if (used < 256) cache[used++] = Entry{dev, fn, threads, dyn_lds, blocks};
   return blocks;
 }
 
@@ -2736,7 +2913,7 @@ bool allow_dyn_lds(KernelFn fn) {
     bool ok;
   };
   static std::mutex mu;
-  static Entry cache[64];
+  static Entry cache[256];
   static int used = 0;
   int dev = 0, count = 0;
   if (hipGetDeviceCount(&count) != hipSuccess || count <= 0) {
@@ -2750,7 +2927,7 @@ bool allow_dyn_lds(KernelFn fn) {
   const bool ok = hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize,
                                       static_cast<int>(kFusedMaxStash)) == hipSuccess;
   (void)hipGetLastError();
-  if (used < 64) cache[used++] = Entry{dev, fn, ok};
+  if (used < 256) cache[used++] = Entry{dev, fn, ok};
   return ok;
 }
 
@@ -2825,6 +3002,72 @@ constexpr bool kFusedByDefault = false;
 // beyond it merge_sk_kernel's one-head-per-wave layout finishes sooner.
 constexpr int64_t kFusedMaxTrips = 2;
 
+// Waves per decode_wg_kernel workgroup for `wgs` workgroups of at most
+// `groups` 16-token groups each: 4, one per SIMD (the waves of a SIMD share its
+// issue slots, and a CU its load path: 8 waves were level with 4 or slower
+// except on long runs of head_dim 64), no more than there are groups.  Many
+// workgroups of few groups run single waves (bf16 Hq32/Hkv8 D128 B256/L64 19.5
+// us against 22.2 with 4 waves), fp32 head_dim 128 ones two (B64/L512 48.9
+// against 53.2), and head_dim 256 splits stay single waves unless they are
+// too few for the CUs (B8, 8 splits: 42.4 against 45.6).  With caller-given
+// splits, us per call with 1 -> 4 waves (graph replays): B4 U[2048, 4096] 4
+// splits 43.0 -> 20.5, 16 splits 18.7 -> 18.2; B1/L16000 16 splits 44.5 -> 21.6;
+// B16 4 splits 48.1 -> 44.2; D64 B32 8 splits 44.2 -> 38.9.
+int wg_waves_for(int64_t wgs, int64_t groups, int dtype, int head_dim) {
+  if (wgs > 1024 && groups <= 8) return 1;
+  int cap = 4;
+  if (dtype == QD_DTYPE_F32) {
+    if (head_dim > 64 && wgs >= 512) cap = 2;
+  } else if (head_dim <= 64) {
+    if (groups >= 64) cap = 8;
+  } else if (head_dim > 128 && wgs >= 256) {
+    cap = 1;
+  }
+  int nw = 1;
+  while (2 * nw <= cap && 2 * nw <= groups) nw *= 2;
+  return nw;
+}
+
+// Whether a call of `wgs` (sequence, kv-head) pairs of at most `groups`
+// 16-token groups each runs as one launch of decode_wg_kernel, without
+// splits: the second launch and the exchange through memory of the
+// alternatives cost 4-5 us, the longest sequence on one workgroup about 0.15
+// us per group (4 waves).  Graph replays, us per call, balanced (fp32: split
+// layout) -> one launch:
+//   bf16 Hq32/Hkv8 D128  B1/L128 11.9 -> 7.5, B1/L512 12.9 -> 11.9, B16/L256 17.2 ->
+//                        11.2, B64/L512 33.8 -> 27.9, B64 U[1, 1024] 36.0 -> 35.0
+//   bf16 Hq8/Hkv2 D64    B4/L512 10.6 -> 9.9, B256/L1024 34.2 -> 27.6
+//   fp32 Hq32/Hkv8 D128  B1/L128 12.8 -> 9.6, B16/L256 19.3 -> 16.3, B64/L512 60.0 -> 48.9
+// and what lies past the limits: more than 32 groups on few workgroups
+// (B1/L1024 13.9 -> 17.8), more than 64 (B64 U[1, 2048] 51.5 -> 60.8), more than
+// 32768 groups in all (B128 U[1, 1024] 54.7 -> 58.7); head_dim 256 past 16
+// groups (B16 U[1, 512] 19.2 -> 21.3); the general layout past 32 groups or
+// 16384 in all (D80 B64 U[1, 1024] 30.4 -> 34.1); fp32 D128 past 8 groups on few
+// workgroups (B4/L256 14.0 -> 15.1).
+bool wg_single_applies(int64_t wgs, int64_t groups, int dtype, int head_dim, bool general) {
+  int64_t most = 32, work = 32768;
+  if (dtype == QD_DTYPE_F32) {
+    most = wgs >= 512 ? 64 : wgs >= 128 ? (head_dim <= 64 ? 64 : 16) : (head_dim <= 64 ? 16 : 8);
+  } else if (head_dim > 128) {
+    most = 16;
+  } else if (general) {
+    work = 16384;
+  } else if (wgs >= 64) {
+    most = 64;
+  }
+  return groups <= most && groups * wgs <= work;
+}
+
+// Enqueues decode_wg_kernel with prm.wg_waves waves per workgroup.
+int launch_wg(const DecodeParams& prm, int dtype, int head_dim, bool general, int splits, int kv_heads, int batch,
+              hipStream_t st) {
+  const KernelFn fn = pick_wg_dt(dtype, head_dim, general);
+  if (!allow_dyn_lds(fn)) return fail(QD_ERR_INVALID_VALUE, "dynamic LDS limit not raised");
+  hipLaunchKernelGGL(fn, dim3(splits, kv_heads, batch), dim3(64 * prm.wg_waves),
+                     wg_lds_bytes(dtype, head_dim, general, prm.wg_waves), st, prm);
+  return QD_OK;
+}
+
 struct AutoPlan {
   bool stream_k;
   int wgs;          // stream-K grid (workgroups)
@@ -2841,6 +3084,7 @@ struct AutoPlan {
   int kv_split;     // stream-K: virtual kv-heads per kv-head (DecodeParams::kv_split)
   bool general;     // stream-K: the general layout (general_applies)
   int kv_slices;    // stream-K: workgroups per range (DecodeParams::kv_slices)
+  int wg_single;    // whole call in one launch of decode_wg_kernel: waves per workgroup, else 0
 };
 
 // Virtual kv-heads per kv-head for the stream-K path: 1 for groups of at
@@ -2891,7 +3135,7 @@ bool fused_applies(int batch, int q_heads, int kv_heads, int head_dim, int nkv, 
 // whether q/k/v/out are 16-byte aligned (the MFMA kernels' vector loads).
 int auto_plan(int batch, int q_heads, int kv_heads, int head_dim, int block_size, int max_pages,
               int dtype, bool aligned, AutoPlan* ap, bool valu = false, bool allow_general = true) {
-  *ap = AutoPlan{false, 0, 1, 1, false, false, 0, 0, 1, 0, kCounterBytes, 0, 1, false, 1};
+  *ap = AutoPlan{false, 0, 1, 1, false, false, 0, 0, 1, 0, kCounterBytes, 0, 1, false, 1, 0};
   if (batch <= 0) return QD_OK;
   const int split = kv_split_for(q_heads, kv_heads);
   const int vkv = kv_heads * (split > 0 ? split : 1);  // kv-heads as the stream-K kernel serves them
@@ -2899,13 +3143,21 @@ int auto_plan(int batch, int q_heads, int kv_heads, int head_dim, int block_size
   const bool f32 = dtype == QD_DTYPE_F32;
   const bool exact = f32 ? !valu && f32_sk_applies(batch, q_heads, kv_heads, head_dim, block_size, max_pages, dtype)
                          : mfma_applies(vkv * gv, vkv, head_dim, block_size, dtype);
-  const int64_t gmax = static_cast<int64_t>(batch) * ((static_cast<int64_t>(max_pages) * block_size + 15) / 16);
-  const bool general = !exact && !valu && allow_general && general_applies(head_dim, dtype);
+  const int64_t groups = (static_cast<int64_t>(max_pages) * block_size + 15) / 16;  // of one sequence, at most
+  const int64_t gmax = static_cast<int64_t>(batch) * groups;
+  const bool general =
+      !exact && !valu && allow_general &&
+      (f32 ? f32_general_applies(batch, q_heads, kv_heads, head_dim, block_size, max_pages, dtype)
+           : general_applies(head_dim, dtype));
+  if (aligned && split > 0 && !valu && (exact || general || f32_mfma_applies(q_heads, kv_heads, head_dim, block_size, dtype)))
+    ap->wg_single = vkv <= 65535 && wg_single_applies(static_cast<int64_t>(batch) * vkv, groups, dtype, head_dim, general && !f32)
+                        ? wg_waves_for(static_cast<int64_t>(batch) * vkv, groups, dtype, head_dim)
+                        : 0;
   if (aligned && split > 0 && (split == 1 || !valu) && (exact || general) && batch <= kSkMaxBatch) {
     int nkv = 1;
     const bool wide = !valu && !f32 && !general && sk_wide_applies(vkv, head_dim);
     auto pick = [&](bool hold) {
-      return general ? pick_general_sk_dt(dtype, head_dim, hold)
+      return general && !f32 ? pick_general_sk_dt(dtype, head_dim, hold)
                      : pick_mfma_sk_dt(dtype, head_dim, nkv, wide && nkv == 1, false, hold);
     };
     // fp32 at head_dim 128 holds 64 KB of K/V per group in flight: one wave
@@ -3296,9 +3548,11 @@ int qd_gqa_decode_launch(const void* q, const void* k_cache, const void* v_cache
                         (splits <= 1 || (reinterpret_cast<uintptr_t>(workspace) & 7u) == 0);
   (void)hipGetLastError();  // start from a clean error state
   if (use_mfma) {
-    const KernelFn fn = dtype == QD_DTYPE_F16 ? pick_mfma<QD_DTYPE_F16>(head_dim)
-                                              : pick_mfma<QD_DTYPE_BF16>(head_dim);
-    hipLaunchKernelGGL(fn, dim3(splits, kv_heads, batch), dim3(64), 0, stm, prm);
+    const int cp = chunk_pages > 0 ? chunk_pages : (max_pages + splits - 1) / splits;
+    prm.wg_waves = wg_waves_for(static_cast<int64_t>(splits) * kv_heads * batch,
+                                (static_cast<int64_t>(cp) * block_size + 15) / 16, dtype, head_dim);
+    st = launch_wg(prm, dtype, head_dim, false, splits, kv_heads, batch, stm);
+    if (st != QD_OK) return st;
   } else {
     KernelFn fn;
     switch (dtype) {
@@ -3357,7 +3611,9 @@ int qd_gqa_decode_auto_stages(const void* q, const void* k_cache, const void* v_
   if (!workspace || workspace_bytes < ap.ws_bytes || !aligned16(workspace))
     return fail(QD_ERR_INVALID_VALUE, "workspace smaller than qd_gqa_decode_auto_workspace_bytes()");
   char* scratch = static_cast<char*>(workspace);
-  if (!ap.stream_k) {
+  // Short contexts in one launch, unless a stage flag asks for another body.
+  const bool single = ap.wg_single > 0 && !unfused && !force_fused;
+  if (!ap.stream_k && !(single && stages == QD_STAGE_ALL)) {
     if (stages != QD_STAGE_ALL)
       return fail(QD_ERR_INVALID_VALUE, "stages apply to the balanced MFMA path only");
     return qd_gqa_decode_launch(q, k_cache, v_cache, block_table, context_lens, out,
@@ -3392,7 +3648,17 @@ int qd_gqa_decode_auto_stages(const void* q, const void* k_cache, const void* v_
   }
   hipStream_t stm = static_cast<hipStream_t>(stream);
   (void)hipGetLastError();
-  if (ap.general) {
+  if (single) {
+    // One kernel: QD_STAGE_MERGE alone has nothing to do.
+    prm.wg_waves = ap.wg_single;
+    prm.splits = 1;
+    if (stages & QD_STAGE_DECODE) {
+      st = launch_wg(prm, dtype, head_dim, ap.general, 1, prm.Hkv, batch, stm);
+      if (st != QD_OK) return st;
+    }
+    return launch_error();
+  }
+  if (ap.general && dtype != QD_DTYPE_F32) {
     hipLaunchKernelGGL(pick_general_sk_dt(dtype, head_dim, ap.stage_bytes > 0), dim3(ap.wgs, ap.kv_slices), dim3(64 * ap.wg_waves),
                        ap.stage_bytes, stm, prm);
     const bool one_head = merge_one_head_per_wave(batch, q_heads);

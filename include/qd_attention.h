@@ -164,6 +164,11 @@ int qd_gqa_decode_kernel_kind(int q_heads, int kv_heads, int head_dim, int block
  *     kernel, merged by a second kernel.  It serves whole calls only and is
  *     reported as kind 0 by qd_gqa_decode_auto_info; with a workspace that
  *     holds only the split layout's partials the split layout runs instead;
+ *   - short contexts (wg_single_applies in gqa_decode.hip: by max_pages *
+ *     block_size and the number of sequences and kv-heads) in one launch with
+ *     one workgroup per (sequence, kv-head), no partials; QD_STAGE_DECODE is
+ *     then the whole call and QD_STAGE_MERGE alone does nothing, and the
+ *     QD_STAGE_UNFUSED / FUSED / VALU bodies stay selectable;
  *   - otherwise: the split layout of qd_gqa_decode_launch with the plan of
  *     qd_gqa_decode_plan.
  * The workspace is device memory, 16-byte aligned, of at least

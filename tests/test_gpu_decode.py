@@ -1146,3 +1146,62 @@ def test_general_layout_matches_oracle(gpu, shape):
     assert rc == 0, cabi.error_string(rc)
     torch.cuda.synchronize()
     assert_close(split_out, ref, DT_NAME[dtype], rows, "split layout")
+
+
+# (dtype, Hq, Hkv, D, P, lengths): short contexts, one launch with the groups of a
+# sequence dealt to the waves of a workgroup (1, 2, 4 or 8 of them).
+ONE_LAUNCH_SHAPES = [
+    (torch.bfloat16, 32, 8, 128, 16, [1, 15, 16, 17, 0, 64, 65, 300, 512]),   # idle waves, a short last run
+    (torch.float16, 40, 8, 128, 32, [32, 33, 1, 96]),
+    (torch.bfloat16, 8, 2, 64, 16, [17, 100, 255, 512]),
+    (torch.float16, 8, 2, 64, 64, _fused_lengths(40, 0, 1024, 151)),          # 8 waves
+    (torch.bfloat16, 32, 32, 96, 16, [1, 49, 500]),                           # 6 columns per lane
+    (torch.float16, 16, 8, 256, 16, [1, 17, 255]),
+    (torch.bfloat16, 48, 1, 128, 16, [5, 200, 0, 333]),                       # 3 x 16 q-heads
+    (torch.float16, 71, 1, 64, 16, [1, 130]),                                 # 4 x 15 + 11
+    (torch.bfloat16, 32, 8, 80, 16, [1, 33, 250]),                            # general layout
+    (torch.float16, 9, 3, 112, 7, [6, 7, 8, 120, 0]),
+    (torch.bfloat16, 8, 4, 192, 5, [4, 80, 33]),
+    (torch.bfloat16, 8, 2, 64, 1, [100, 3]),
+    (torch.float32, 32, 8, 128, 16, [1, 16, 17, 0, 128]),
+    (torch.float32, 16, 4, 64, 32, [1, 33, 200, 256]),
+    (torch.float32, 8, 8, 128, 16, _fused_lengths(70, 1, 512, 152)),          # 2 waves
+    (torch.bfloat16, 32, 8, 128, 16, _fused_lengths(300, 0, 64, 153)),        # single waves
+]
+
+
+@pytest.mark.parametrize("shape", ONE_LAUNCH_SHAPES,
+                         ids=lambda s: f"{DT_NAME[s[0]]}-Hq{s[1]}-Hkv{s[2]}-D{s[3]}-P{s[4]}-B{len(s[5])}")
+def test_one_launch_short_contexts(gpu, shape):
+    """Short contexts in one launch: every row matches the oracle on a
+    NaN-filled workspace that the call leaves as it is (no partials), and the
+    torch op gives the same bits.  Where stages apply, QD_STAGE_DECODE is the
+    whole call, QD_STAGE_MERGE alone does nothing, and QD_STAGE_UNFUSED runs
+    the balanced kernel and its merge, which match the oracle as well."""
+    dtype, hq, hkv, d, p, lengths = shape
+    B = len(lengths)
+    say(f"one launch {DT_NAME[dtype]} Hq{hq} Hkv{hkv} D{d} P{p} B{B}")
+    case = to_dev(make_decode_case(lengths=lengths, q_heads=hq, kv_heads=hkv, head_dim=d, block_size=p, dtype=dtype,
+                                   seed=154), gpu)
+    q, maxp = case[0], case[3].shape[1]
+    ref, rows = oracle_rows(case)
+    ws = cabi.auto_workspace(B, hq, hkv, d, p, maxp, cabi.DTYPE[dtype], gpu, fill=0xFF)
+    before = ws.clone()
+
+    def run(stages, out):
+        rc = cabi.auto_launch(*case, out, scale=1 / math.sqrt(d), workspace=ws, stages=stages)
+        assert rc == 0, cabi.error_string(rc)
+        torch.cuda.synchronize()
+        return out
+
+    out = run(cabi.QD_STAGE_ALL, torch.full_like(q, float("nan")))
+    assert torch.equal(ws, before), "the call wrote partials"
+    assert_close(out, ref, DT_NAME[dtype], rows, "one launch")
+    assert torch.equal(out, attention_amd.gqa_decode(*case))
+    if cabi.auto_info(B, hq, hkv, d, p, maxp, cabi.DTYPE[dtype])[0] != 1:
+        return
+    assert torch.equal(out, run(cabi.QD_STAGE_DECODE, torch.full_like(q, float("nan"))))
+    merged = run(cabi.QD_STAGE_MERGE, torch.full_like(q, 7.0))
+    assert torch.equal(merged, torch.full_like(q, 7.0))
+    out = run(cabi.QD_STAGE_ALL | cabi.QD_STAGE_UNFUSED, torch.full_like(q, float("nan")))
+    assert_close(out, ref, DT_NAME[dtype], rows, "balanced")
