@@ -386,6 +386,7 @@ struct MlaParams {
   int B, T, H, Dc, Dr, W, P, maxP;
   int nk;  // indices per row, -1 = all tokens (dense)
   int causal, splits;
+  int fold;         // shared-tile kernel, folded queries: queries per sequence (H = fold * heads), else 1
   int head_groups;  // MFMA kernel: head groups (workgroups per tile range)
   int kch;          // MFMA kernel: ceil(W / 32)
   int nht, ds;      // MFMA kernel: head tiles per workgroup, latent slices per head tile
@@ -1697,6 +1698,10 @@ __global__ __launch_bounds__(kAttendThreads) void mla_attend_wave_kernel(MlaPara
 
 constexpr int kShThreads = 256;                         // four waves, 16 heads each
 constexpr int kShTokens = 32;                           // tokens per tile
+// What a tile's rows are: 32 consecutive tokens of a page; any 32 rows
+// (listed tokens, or pages that are no multiple of 16); or consecutive tokens
+// for all queries of a sequence at once.
+constexpr int kShDense = 0, kShGather = 1, kShFold = 2;
 constexpr int kShBufs = 4;                              // LDS tile ring
 constexpr int kShRowBytes = 2 * 576;                    // cache row: 512 latent + 64 rope, 16-bit
 #ifndef QD_MLA_SHARED_ROW_PAD
@@ -1708,6 +1713,7 @@ constexpr int kShTileBytes = kShLatBytes + kShTokens * 128;  // + rope rows
 constexpr int kShRows = 1024;                           // query rows (prologue arrays in the ring)
 constexpr int kShListTiles = 512;                       // tiles of one workgroup's range
 constexpr int kShCtlPad = 8;                            // placeholder entries after the tile list
+constexpr int kShGatherTiles = 256;                     // tiles of a range of gathered rows (row list in LDS)
 constexpr int kShDma = 9;                               // DMA instructions per wave per tile
 constexpr int kShColBlocks = 512 / 16;                  // PV output blocks of 16 latent columns
 #ifndef QD_MLA_SHARED_PV_AHEAD
@@ -1725,12 +1731,17 @@ constexpr int kShRowCost = QD_MLA_SHARED_ROW_COST;
 #define QD_MLA_SHARED_QK_AHEAD 6
 #endif
 
-__host__ __device__ constexpr size_t mla_shared_lds_bytes() {
-  return static_cast<size_t>(kShBufs) * kShTileBytes    // tile ring (prologue arrays before the first tile)
-         + static_cast<size_t>(kShListTiles + kShCtlPad) * 16;  // tile list
+// LDS tile buffers: gathered rows give one up for the row list.
+__host__ __device__ constexpr int shared_bufs(int mode) { return mode == kShGather ? kShBufs - 1 : kShBufs; }
+__host__ __device__ constexpr int shared_list_tiles(int mode) { return mode == kShGather ? kShGatherTiles : kShListTiles; }
+
+__host__ __device__ constexpr size_t mla_shared_lds_bytes(int mode) {
+  return static_cast<size_t>(shared_bufs(mode)) * kShTileBytes  // tile ring (prologue arrays before the first tile)
+         + static_cast<size_t>(shared_list_tiles(mode) + kShCtlPad) * 16  // tile list
+         + (mode == kShGather ? static_cast<size_t>(kShGatherTiles + kShCtlPad) * kShTokens * 4 : 0);  // row list
 }
 
-static_assert(kShRows * (4 + 4 + 8) + kShListTiles * 16 <= kShBufs * kShTileBytes,
+static_assert(kShRows * (4 + 4 + 8) + kShListTiles * 16 <= (kShBufs - 1) * kShTileBytes,
               "shared-tile kernel prologue arrays exceed the tile ring");
 
 // Wait for all but the last kVm vector-memory operations of this wave (loads
@@ -1820,13 +1831,34 @@ __device__ __forceinline__ void lds_wait_tied(u32x2& a, u32x2& b) {
 // both (the stores would otherwise hold the tile waits behind them).
 // NT: nontemporal cache loads (one head group); with several head groups
 // the tiles stay in L2 for the other groups' workgroups on the XCD.
-template <int DT, bool NT>
+//
+// MODE kShGather: a tile is any 32 cache rows, the listed tokens of a query
+// (p.nk >= 0) or the tokens of pages that hold no whole 16-token groups.  The
+// prologue looks up every row of the range (index, page) and leaves its pool
+// row in LDS; a step reads its wave's 8 rows a tile ahead, one LDS read.  A
+// listed token that is not visible reads a visible row of its tile with
+// weight 0, a tile without any leaves the list.  The list takes one ring
+// buffer.
+// Partials stay in fp32, as in the staged kernel that served these rows.
+// us per call against that kernel (bf16): 128 heads, 2048 listed of U[4096,
+// 16384] tokens, B16 90.8 -> 51.7 (attention stage 72.7 -> 34); fp16 64 heads B64
+// 135.7 -> 64.4; page size 1, 128 heads, B8 70.1 -> 49.7.
+//
+// MODE kShFold: the p.fold queries of a sequence are one row of p.fold *
+// heads heads ([B, T, H, *] is that already), so the cache is read once for
+// all of them; each lane masks the tokens its query does not see.
+// us per call (latent write and decode) against the wave kernel: fp16 2 x 32
+// heads, B48, U[512, 4096] 76.5 -> 56.5.  A token that some queries of its
+// sequence see must hold finite values, as any visible token must (an Inf or
+// NaN there reaches all of them).
+template <int DT, bool NT, int MODE>
 __global__ __launch_bounds__(kShThreads) void mla_attend_shared_kernel(MlaParams p) {
   using E = Elem<DT>;
   using Ops = MfmaOps<DT>;
   using S = typename E::S;
   constexpr int kDc = 512;
   constexpr int kW = 576;
+  constexpr int kBufs = shared_bufs(MODE);
   extern __shared__ __align__(16) char smem[];
   const int tid = static_cast<int>(threadIdx.x);
   const int lane = tid & 63;
@@ -1843,7 +1875,8 @@ __global__ __launch_bounds__(kShThreads) void mla_attend_shared_kernel(MlaParams
   if (w >= p.wgs) return;  // whole workgroup: uniform
 
   char* ring = smem;
-  i32x4* ctl = reinterpret_cast<i32x4*>(smem + kShBufs * kShTileBytes);
+  i32x4* ctl = reinterpret_cast<i32x4*>(smem + kBufs * kShTileBytes);
+  [[maybe_unused]] uint32_t* prow = reinterpret_cast<uint32_t*>(ctl + shared_list_tiles(MODE) + kShCtlPad);  // pool rows
   // Prologue arrays, inside the ring.
   int* rt = reinterpret_cast<int*>(ring);                      // [rows] tiles
   int* re = rt + kShRows;                                      // [rows] visible end
@@ -1859,9 +1892,15 @@ __global__ __launch_bounds__(kShThreads) void mla_attend_shared_kernel(MlaParams
 
   // --- Prologue -----------------------------------------------------------
   for (int r = tid; r < rows; r += kShThreads) {
-    const int end = row_end(p, r / p.T, r);
+    int end = 0;
+    if constexpr (MODE == kShFold) {
+      for (int t = 0; t < p.fold; ++t) end = max(end, row_end(p, r, static_cast<int64_t>(r) * p.fold + t));
+    } else {
+      end = row_end(p, r / p.T, r);
+    }
     re[r] = end;
-    rt[r] = (end + kShTokens - 1) / kShTokens;
+    const int count = MODE == kShGather && p.nk >= 0 ? (end > 0 ? p.nk : 0) : end;
+    rt[r] = (count + kShTokens - 1) / kShTokens;
   }
   __syncthreads();
   auto row_cost = [&](int tiles) { return tiles > 0 ? tiles + kShRowCost : 0; };
@@ -1899,20 +1938,26 @@ __global__ __launch_bounds__(kShThreads) void mla_attend_shared_kernel(MlaParams
       tl[t] = i32x4{0, 0, 0, -1};
       continue;
     }
+    const int whole = (first >= g0 && incl[r] <= g1) ? 1 : 0;
+    if (tir == 0 && hg == 0) {
+      // This workgroup holds the row's first tile: record its span.
+      p.meta[2 * r] = w;
+      p.meta[2 * r + 1] = wg_of(incl[r] - 1) - w + 1;
+    }
+    if constexpr (MODE == kShGather) {  // the rows and their mask follow once the list is compact
+      tl[t] = i32x4{tir, 0, whole << 16, r};
+      continue;
+    }
     const int tok0 = kShTokens * tir;
     const int pg = tok0 / p.P;  // the tile lies in one page (P % 32 == 0)
     int32_t phys = p.table[static_cast<int64_t>(r / p.T) * p.maxP + pg];
     if (phys < 0) phys = 0;
     if (phys >= p.num_blocks) phys = static_cast<int32_t>(p.num_blocks - 1);
     const int64_t base = (static_cast<int64_t>(phys) * p.P + (tok0 - pg * p.P)) * kW;
-    const int whole = (first >= g0 && incl[r] <= g1) ? 1 : 0;
+    // kShFold keeps the tile's place in the row above bit 7 (host check).
+    const int nv = min(kShTokens, re[r] - tok0);
     tl[t] = i32x4{static_cast<int>(base & 0xFFFFFFFF), static_cast<int>(base >> 32),
-                  min(kShTokens, re[r] - tok0) | (whole << 16), r};
-    if (tir == 0 && hg == 0) {
-      // This workgroup holds the row's first tile: record its span.
-      p.meta[2 * r] = w;
-      p.meta[2 * r + 1] = wg_of(incl[r] - 1) - w + 1;
-    }
+                  MODE == kShFold ? nv | (whole << 6) | (tir << 7) : nv | (whole << 16), r};
   }
   // Rows with no tile: zeros from workgroup (row % wgs), meta {0, 0}.
   for (int r = w; r < rows; r += p.wgs) {
@@ -1946,7 +1991,70 @@ __global__ __launch_bounds__(kShThreads) void mla_attend_shared_kernel(MlaParams
     if (lane < kShCtlPad) ctl[count + lane] = i32x4{0, 0, 1, -1};
   }
   __syncthreads();
-  const int n = *nreal;
+  int n = *nreal;
+  if constexpr (MODE == kShGather) {
+    // Pool rows of every tile (32 lanes each) and its mask of visible rows;
+    // the placeholder tile n reads row 0.
+    for (int i0 = 64 * wv; i0 < 32 * (n + 1); i0 += kShThreads) {
+      const int t = (i0 + lane) >> 5, i = lane & 31;
+      const i32x4 e = ctl[t];
+      const int r = e[3];
+      int tok = -1;
+      if (t < n) {
+        const int at = kShTokens * e[0] + i;
+        tok = p.nk < 0 ? at : at < p.nk ? p.idx[static_cast<int64_t>(r) * p.nk + at] : -1;
+        if (tok >= re[r]) tok = -1;
+      }
+      uint32_t pr = 0;
+      if (tok >= 0) {
+        int32_t phys = p.table[static_cast<int64_t>(r / p.T) * p.maxP + tok / p.P];
+        if (phys < 0) phys = 0;
+        if (phys >= p.num_blocks) phys = static_cast<int32_t>(p.num_blocks - 1);
+        pr = static_cast<uint32_t>(phys) * p.P + tok % p.P;
+      }
+      const uint32_t mask = static_cast<uint32_t>(__ballot(tok >= 0) >> (lane & 32));
+      const uint32_t other = __shfl(pr, (lane & 32) + (mask ? __builtin_ctz(mask) : 0));
+      prow[32 * t + i] = tok >= 0 ? pr : other;
+      if (i == 0 && t < n) ctl[t][1] = static_cast<int>(mask);
+    }
+    __syncthreads();
+    // Tiles without a visible row leave the list (their rows may hold
+    // anything); a row segment of such tiles only gives zeros or an empty
+    // partial.  An entry's first word becomes its place in the row list.
+    if (wv == 0) {
+      int count = 0;
+      for (int base = 0; base < n; base += 64) {
+        const int t = base + lane;
+        i32x4 e = t < n ? ctl[t] : i32x4{0, 0, 0, -1};
+        bool empty = t < n && (t == 0 || ctl[t - 1][3] != e[3]);
+        for (int u = t; empty && u < n && ctl[u][3] == e[3]; ++u) empty = ctl[u][1] == 0;
+        uint64_t em = __ballot(empty);
+        const bool keep = e[1] != 0;
+        const uint64_t bal = __ballot(keep);
+        e[0] = t;
+        if (keep) ctl[count + __popcll(bal & ((uint64_t{1} << lane) - 1))] = e;
+        count += __popcll(bal);
+        for (; em; em &= em - 1) {
+          const int src = __builtin_ctzll(em);
+          const int64_t r = __builtin_amdgcn_readlane(e[3], src);
+          const bool whole = (__builtin_amdgcn_readlane(e[2], src) >> 16) != 0;
+          const int hh = h0 + lane;
+          if (hh >= p.H) continue;
+          if (whole) {
+            for (int c = 0; c < kDc / 8; ++c)
+              *reinterpret_cast<u32x4*>(static_cast<S*>(p.out) + (r * p.H + hh) * kDc + 8 * c) = u32x4{0u, 0u, 0u, 0u};
+          } else {
+            *reinterpret_cast<f32x2*>(p.part + ((w + r) * p.H + hh) * static_cast<int64_t>(kDc + 2)) =
+                f32x2{-INFINITY, 0.f};
+          }
+        }
+      }
+      if (lane == 0) *nreal = count;
+      if (lane < kShCtlPad) ctl[count + lane] = i32x4{n, -1, 0, -1};
+    }
+    __syncthreads();
+    n = *nreal;
+  }
   __syncthreads();  // every wave has read the count before the ring is written
   if (n == 0) return;  // whole workgroup: uniform
   QD_MLA_STAMP(0, st_entry);
@@ -1958,15 +2066,20 @@ __global__ __launch_bounds__(kShThreads) void mla_attend_shared_kernel(MlaParams
   // issues the same loads).
   // Instruction k < 8 loads latent row 8 wv + k, instruction 8 the rope
   // bytes of rows 8 wv .. 8 wv + 7.
-  auto dma_one = [&](int t, const i32x4 e, int k) {
-    char* slot = ring + (t % kShBufs) * kShTileBytes;
+  // (kShGather: o is lane 8 k's pool row of tile row 8 wv + k.)
+  auto dma_one = [&](int t, const i32x4 e, uint32_t o, int k) {
+    char* slot = ring + (t % kBufs) * kShTileBytes;
     const int64_t base = static_cast<int64_t>(static_cast<uint32_t>(e[0])) | (static_cast<int64_t>(e[1]) << 32);
-    const int nv = e[2] & 0xFFFF;
+    const int nv = e[2] & (MODE == kShFold ? 0x3F : 0xFFFF);
     const char* tb = cache + 2 * base;
     if (k < 8) {
       const int R = 8 * wv + k;
       const int Rc = R < nv ? R : nv - 1;
-      const char* src = tb + Rc * kShRowBytes + 16 * lane;
+      const char* src =
+          MODE == kShGather
+              ? cache + static_cast<int64_t>(static_cast<uint32_t>(__builtin_amdgcn_readlane(o, 8 * k))) * kShRowBytes +
+                    16 * lane
+              : tb + Rc * kShRowBytes + 16 * lane;
       __builtin_amdgcn_global_load_lds(reinterpret_cast<const void*>(src),
                                        (__attribute__((address_space(3))) void*)(slot + R * kShLatStride), 16, 0,
                                        NT ? 2 : 0);
@@ -1974,21 +2087,28 @@ __global__ __launch_bounds__(kShThreads) void mla_attend_shared_kernel(MlaParams
       const int R = 8 * wv + (lane >> 3);
       const int Rc = R < nv ? R : nv - 1;
       const int c = (lane & 7) ^ ((R >> 1) & 7);
-      const char* src = tb + Rc * kShRowBytes + 2 * kDc + 16 * c;
+      const char* src = (MODE == kShGather ? cache + static_cast<int64_t>(o) * kShRowBytes : tb + Rc * kShRowBytes) +
+                        2 * kDc + 16 * c;
       __builtin_amdgcn_global_load_lds(reinterpret_cast<const void*>(src),
                                        (__attribute__((address_space(3))) void*)(slot + kShLatBytes + wv * 1024), 16,
                                        0, NT ? 2 : 0);
     }
   };
-  auto dma = [&](int t, const i32x4 e) {
+  auto dma = [&](int t, const i32x4 e, uint32_t o) {
 #pragma unroll
-    for (int k = 0; k < kShDma; ++k) dma_one(t, e, k);
+    for (int k = 0; k < kShDma; ++k) dma_one(t, e, o, k);
   };
+  auto pool_row = [&](int place) { return MODE == kShGather ? prow[32 * place + 8 * wv + (lane >> 3)] : 0u; };
   // This lane's head's query, 18 chunks of 32 elements ([q | q_rope]).
   // Heads past H read head 0's query (never stored; no select on the loaded
   // values, which would wait for every load in flight).
   u32x4 qv[18];
+  [[maybe_unused]] int q_pos = 0, q_len = 0;  // kShFold: this lane's query position, its sequence's length
   auto load_q = [&](int r) {
+    if constexpr (MODE == kShFold) {
+      q_pos = p.pos[static_cast<int64_t>(r) * p.fold + (h < p.H ? h : 0) / (p.H / p.fold)];
+      q_len = p.lens[r];
+    }
     const int64_t hr = static_cast<int64_t>(r) * p.H + (h < p.H ? h : 0);
     const char* qrow = static_cast<const char*>(p.q) + hr * kDc * 2;
     const char* rrow = static_cast<const char*>(p.qr) + hr * (kW - kDc) * 2;
@@ -2011,33 +2131,41 @@ __global__ __launch_bounds__(kShThreads) void mla_attend_shared_kernel(MlaParams
   // no register load is pending when the loop starts (the compiler would
   // otherwise wait for every load in flight, the whole ring, in every step).
 #pragma unroll
-  for (int t = 0; t < kShBufs - 1; ++t) dma(t, ctl[t]);
+  for (int t = 0; t < kBufs - 1; ++t) dma(t, ctl[t], pool_row(ctl[t][0]));
   load_q(ctl[0][3]);
   // List entries are read one step ahead of their use (an LDS round trip
   // at the top of each step would sit on the critical path): e_cur = tile
-  // t, r_nxt = row of tile t + 1, e_dma = tile t + kShBufs - 1.
-  i32x4 e_cur = ctl[0], e_dma = ctl[kShBufs - 1];
+  // t, r_nxt = row of tile t + 1, e_dma = tile t + kBufs - 1.
+  i32x4 e_cur = ctl[0], e_dma = ctl[kBufs - 1];
+  // kShGather: that tile's pool rows, and the place of the next one's.
+  [[maybe_unused]] uint32_t o_dma = pool_row(ctl[kBufs - 1][0]);
+  [[maybe_unused]] int j_dma = ctl[kBufs][0];
   int r_nxt = ctl[1][3];
   wait_vm_all();
   QD_MLA_STAMP(2, __builtin_amdgcn_s_memrealtime());
   int row = -1;
   for (int t = 0; t < n; ++t) {
-    dma_ring_barrier<(kShBufs - 2) * kShDma>();  // tile t in LDS; tile t-1 done by every wave
-    const i32x4 ed = e_dma;                       // tile t + kShBufs - 1, into tile t-1's slot
+    dma_ring_barrier<(kBufs - 2) * kShDma>();  // tile t in LDS; tile t-1 done by every wave
+    [[maybe_unused]] const uint32_t od = o_dma;
+    const i32x4 ed = e_dma;                       // tile t + kBufs - 1, into tile t-1's slot
     const i32x4 e = e_cur;
     const int r1 = r_nxt;
     e_cur = ctl[t + 1];
     r_nxt = ctl[t + 2][3];
-    e_dma = ctl[t + kShBufs];
-    const int nv = e[2] & 0xFFFF;
-    const bool whole = (e[2] >> 16) != 0;
+    e_dma = ctl[t + kBufs];
+    if constexpr (MODE == kShGather) {
+      o_dma = pool_row(j_dma);
+      j_dma = ctl[t + kBufs + 1][0];
+    }
+    const int nv = e[2] & (MODE == kShFold ? 0x3F : 0xFFFF);
+    const bool whole = MODE == kShFold ? (e[2] & 0x40) != 0 : (e[2] >> 16) != 0;
     const int r = e[3];
     const bool last = r1 != r;
     if (r != row) {
       row = r;
       reset();
     }
-    const char* slot = ring + (t % kShBufs) * kShTileBytes;
+    const char* slot = ring + (t % kBufs) * kShTileBytes;
 
     // QK for both 16-row blocks together (two MFMAs per chunk, one per
     // block), operands read kAhead chunks ahead: one chunk's MFMAs take 32
@@ -2073,7 +2201,7 @@ __global__ __launch_bounds__(kShThreads) void mla_attend_shared_kernel(MlaParams
         // The next tile's DMA, one instruction per chunk: issued together
         // after the barrier, the four waves' loads queue on the CU's load
         // path for about as long as the QK products take.
-        if (c < kShDma) dma_one(t + kShBufs - 1, ed, c);
+        if (c < kShDma) dma_one(t + kBufs - 1, ed, od, c);
         __builtin_amdgcn_sched_barrier(0);
       }
     }
@@ -2100,6 +2228,18 @@ __global__ __launch_bounds__(kShThreads) void mla_attend_shared_kernel(MlaParams
 #pragma unroll
       for (int i = 0; i < 4; ++i) x[tb][i] = st[i] * p.sl2;
     }
+    if constexpr (MODE == kShFold) {
+      // Tokens this lane's query does not see (row_end, with the table's
+      // capacity in nv), in the tiles that hold any.
+      const int tok0 = kShTokens * (e[2] >> 7);
+      const int seen = min(p.causal && q_pos < q_len ? q_pos + 1 : q_len, tok0 + nv) - tok0;
+      if (__ballot(seen < kShTokens)) {
+#pragma unroll
+        for (int tb = 0; tb < 2; ++tb)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) x[tb][i] = 16 * tb + 4 * q4 + i < seen ? x[tb][i] : -INFINITY;
+      }
+    }
     float mx = fmaxf(fmaxf(fmaxf(x[0][0], x[0][1]), fmaxf(x[0][2], x[0][3])),
                      fmaxf(fmaxf(x[1][0], x[1][1]), fmaxf(x[1][2], x[1][3])));
     mx = max_over_lane_groups(mx);
@@ -2119,7 +2259,12 @@ __global__ __launch_bounds__(kShThreads) void mla_attend_shared_kernel(MlaParams
       float pr[4];
 #pragma unroll
       for (int i = 0; i < 4; ++i) pr[i] = fast_exp2(x[tb][i] - m_use);
-      if (nv < kShTokens) {  // uniform
+      if constexpr (MODE == kShGather) {
+        if (e[1] != -1) {  // uniform
+#pragma unroll
+          for (int i = 0; i < 4; ++i) pr[i] = (e[1] >> (16 * tb + 4 * q4 + i)) & 1 ? pr[i] : 0.f;
+        }
+      } else if (MODE == kShDense && nv < kShTokens) {  // uniform
 #pragma unroll
         for (int i = 0; i < 4; ++i) pr[i] = 16 * tb + 4 * q4 + i < nv ? pr[i] : 0.f;
       }
@@ -2177,6 +2322,15 @@ __global__ __launch_bounds__(kShThreads) void mla_attend_shared_kernel(MlaParams
           for (int cb = 0; cb < kShColBlocks; ++cb)
             *reinterpret_cast<u32x2*>(orow + 16 * cb + 4 * q4) =
                 u32x2{Ops::pack2(acc[cb][0] * inv, acc[cb][1] * inv), Ops::pack2(acc[cb][2] * inv, acc[cb][3] * inv)};
+        } else if constexpr (MODE == kShGather) {
+          float* pr = p.part + ((static_cast<int64_t>(w) + r) * p.H + h) * static_cast<int64_t>(kDc + 2);
+          if (q4 == 0) *reinterpret_cast<f32x2*>(pr) = f32x2{m_run == -INFINITY ? -INFINITY : m_run * kLn2, Lt};
+#pragma unroll
+          for (int cb = 0; cb < kShColBlocks; ++cb) {
+            float* dst = pr + 2 + 16 * cb + 4 * q4;
+            *reinterpret_cast<f32x2*>(dst) = f32x2{acc[cb][0], acc[cb][1]};
+            *reinterpret_cast<f32x2*>(dst + 2) = f32x2{acc[cb][2], acc[cb][3]};
+          }
         } else {
           // Half-precision partial (kHalfHeader): acc / s_k in fp16, s_k the
           // largest |acc| of the head's 128-column block k (the 4 lanes q4 of
@@ -2529,6 +2683,7 @@ struct AttendPlan {
   int splits;  // VALU kernel
   bool wave;   // MFMA path through mla_attend_wave_kernel
   bool shared;  // MFMA path through mla_attend_shared_kernel
+  int mode;     // its tiles (kShDense, kShGather, kShFold)
 };
 
 // Smallest instantiated DMA-chunk count covering ceil(W/64), 0 if none.
@@ -2537,6 +2692,35 @@ int cpt_for(int W) {
   for (int c : {2, 5, 9, 10})
     if (need <= c) return c;
   return 0;
+}
+
+constexpr int kNoGather = 1 << 30;  // internal plan flag
+
+// Whether the q_len queries of a sequence run as one row of q_len * heads
+// heads of the shared-tile kernel (dense rows): from 32 on, where its workgroup
+// of 64 is half full (the wave kernel reads every cache row once per query and
+// 16 heads).  us per call, wave kernel -> folded: 2 x 16 heads B48 U[512, 4096]
+// 60.5 -> 50.2, B128 U[512, 2000] 91.8 -> 67.4; 3 x 16 B48 81.0 -> 55.0; 2 x 20 B48
+// 72.3 -> 51.4; 4 x 8 B16 50.7 -> 45.4.
+bool shared_fold_applies(int q_len, int heads) { return q_len * heads >= 32; }
+
+// Ranges (workgroups per head group) for `rows` rows of at most `tiles` tiles:
+// the CUs, but per row at most per_row * sqrt(tiles).  A row split over x
+// ranges takes tiles / x steps and then a fold of x partials, 8 per memory
+// round trip, so the best x grows with the square root of the tiles; one row
+// on every CU folded 256 of them.  The factors were swept from 0.25 to 8 over
+// 1-128 rows of 64-30000 tokens (graph replays, us per mla_decode, all CUs ->
+// now; full batches keep all CUs):
+//   wave kernel, 16 heads     B1/L500 56.4 -> 26.1, B1/L4000 125 -> 31.0, B1/L30000 220 -> 58.5,
+//                             B4/L4000 80.0 -> 40.0, B16/L4000 46.6 -> 40.9
+//   shared-tile, 128 heads    B1/L4000 81.2 -> 35.3, B1/L30000 132 -> 70.9, B4/L16000 75.8 -> 67.5
+//   staged, 16 heads, K 2048  B1 128 -> 42, B4 66.7 -> 43.9
+constexpr double kShRangesPerRow = 1.1, kWaveRangesPerRow = 0.6, kStagedRangesPerRow = 2.0;
+
+int range_count(int64_t rows, int64_t tiles, int groups, double per_row) {
+  const double per = std::ceil(per_row * std::sqrt(static_cast<double>(std::max<int64_t>(tiles, 1))));
+  const int64_t cap = rows * static_cast<int64_t>(per);
+  return static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(device_cus() / groups, cap)));
 }
 
 AttendPlan plan_attend(const AttendShape& a, int forced, int flags) {
@@ -2563,7 +2747,10 @@ AttendPlan plan_attend(const AttendShape& a, int forced, int flags) {
   const int64_t rows = static_cast<int64_t>(a.B) * a.T;
   if (pl.mfma) {
     // One resident workgroup per CU (the LDS ring), shared by the head groups.
-    pl.wgs = forced > 0 ? forced : std::max(1, device_cus() / pl.head_groups);
+    const int64_t cap = static_cast<int64_t>(a.maxP) * a.P;
+    pl.wgs = forced > 0 ? forced
+                        : range_count(rows, ((a.nk >= 0 ? a.nk : cap) + kTileTokens - 1) / kTileTokens, pl.head_groups,
+                                      kStagedRangesPerRow);
     pl.splits = 1;
     // The wave-streamed kernel: dense rows, Dc 512 / Dr 64 (instantiated),
     // pages of whole 16-token tiles, rows and tiles per workgroup within its
@@ -2575,16 +2762,24 @@ AttendPlan plan_attend(const AttendShape& a, int forced, int flags) {
     // The shared-tile kernel: the same dense shapes with 64 heads or more
     // and pages of whole 32-token tiles, 64 heads per workgroup of four
     // waves, one workgroup per CU.
-    const size_t slds = mla_shared_lds_bytes();
     const bool dense512 = a.Dc == 512 && a.Dr == 64 && a.nk < 0 && a.P % kSubTokens == 0;
-    if ((flags & (QD_FLAG_MLA_STAGED | QD_FLAG_MLA_WAVE)) == 0 && dense512 && a.P % kShTokens == 0 && a.H >= 64 &&
-        rows <= kShRows && slds <= static_cast<size_t>(device_max_lds())) {
-      const int groups = (a.H + 63) / 64;
-      const int wgs = forced > 0 ? forced : std::max(1, device_cus() / groups);
-      const int64_t smax =
-          rows * ((static_cast<int64_t>(a.maxP) * a.P + kShTokens - 1) / kShTokens + kShRowCost);
-      if ((smax + wgs - 1) / wgs + 1 <= kShListTiles) {
+    const bool paged32 = dense512 && a.P % kShTokens == 0;
+    const int mode = paged32 && a.T > 1 && shared_fold_applies(a.T, a.H) && cap < (int64_t{1} << 29) ? kShFold
+                     : paged32                                                                      ? kShDense
+                                                                                                    : kShGather;
+    const bool gather = (flags & kNoGather) == 0 && a.Dc == 512 && a.Dr == 64 && (a.nk >= 0 || a.P % kSubTokens != 0);
+    const int64_t sh_rows = mode == kShFold ? a.B : rows;
+    const int sh_heads = mode == kShFold ? a.T * a.H : a.H;
+    const size_t slds = mla_shared_lds_bytes(mode);
+    if ((flags & (QD_FLAG_MLA_STAGED | QD_FLAG_MLA_WAVE)) == 0 && (paged32 || gather) &&
+        (mode == kShFold || a.H >= 64) && sh_rows <= kShRows && slds <= static_cast<size_t>(device_max_lds())) {
+      const int groups = (sh_heads + 63) / 64;
+      const int64_t row_tiles = ((a.nk >= 0 ? a.nk : cap) + kShTokens - 1) / kShTokens;
+      const int wgs = forced > 0 ? forced : range_count(sh_rows, row_tiles, groups, kShRangesPerRow);
+      const int64_t smax = sh_rows * (row_tiles + kShRowCost);
+      if ((smax + wgs - 1) / wgs + 1 <= shared_list_tiles(mode)) {
         pl.shared = true;
+        pl.mode = mode;
         pl.nht = 1;
         pl.head_groups = groups;
         pl.wgs = wgs;
@@ -2594,7 +2789,8 @@ AttendPlan plan_attend(const AttendShape& a, int forced, int flags) {
     if (!pl.shared && (flags & QD_FLAG_MLA_STAGED) == 0 && dense512 && rows <= kWaveRows &&
         wlds <= static_cast<size_t>(device_max_lds())) {
       const int groups = ht;
-      const int wgs = forced > 0 ? forced : std::max(1, device_cus() / groups);
+      const int wgs =
+          forced > 0 ? forced : range_count(rows, (cap + kSubTokens - 1) / kSubTokens, groups, kWaveRangesPerRow);
       if ((gmax + wgs - 1) / wgs + 1 <= kWaveListTiles) {
         pl.wave = true;
         pl.nht = 1;
@@ -2627,12 +2823,22 @@ size_t round_up256(size_t x) { return (x + 255) / 256 * 256; }
 // acc[Dc]} for the shared-tile kernel (16-byte accumulator stores).
 // Floats per partial row: the half-precision rows of the shared-tile and
 // wave kernels (kHalfPst), the staged kernel's {m, l} + Dc fp32.
-bool half_partials(const AttendPlan& pl) { return pl.shared || pl.wave; }
+bool half_partials(const AttendPlan& pl) { return (pl.shared && pl.mode != kShGather) || pl.wave; }
+// The call as its kernel sees it: folded queries are heads of one row.
+AttendShape kernel_shape(const AttendShape& a, const AttendPlan& pl) {
+  AttendShape k = a;
+  if (pl.mfma && pl.shared && pl.mode == kShFold) {
+    k.H = a.T * a.H;
+    k.T = 1;
+  }
+  return k;
+}
 int partial_stride(const AttendShape& a, const AttendPlan& pl) {
   return half_partials(pl) ? kHalfPst : a.Dc + 2;
 }
 
-size_t attend_partial_bytes(const AttendShape& a, const AttendPlan& pl) {
+size_t attend_partial_bytes(const AttendShape& call, const AttendPlan& pl) {
+  const AttendShape a = kernel_shape(call, pl);
   const int64_t rows = static_cast<int64_t>(a.B) * a.T;
   if (pl.mfma)
     return round_up256(static_cast<size_t>(pl.wgs + rows) * a.H * partial_stride(a, pl) * sizeof(float)) +
@@ -2669,18 +2875,25 @@ hipError_t launch_attend_wave(const MlaParams& prm, const AttendPlan& pl, int64_
   return hipSuccess;
 }
 
-template <int DT, bool NT>
-hipError_t launch_attend_shared(const MlaParams& prm, const AttendPlan& pl, int64_t grid, hipStream_t st) {
-  auto fn = mla_attend_shared_kernel<DT, NT>;
+template <int DT, bool NT, int MODE>
+hipError_t launch_attend_shared_mode(const MlaParams& prm, const AttendPlan& pl, int64_t grid, hipStream_t st) {
+  auto fn = mla_attend_shared_kernel<DT, NT, MODE>;
   static std::once_flag once;
   static hipError_t attr = hipSuccess;
   std::call_once(once, [&] {
     attr = hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize,
-                               static_cast<int>(mla_shared_lds_bytes()));
+                               static_cast<int>(mla_shared_lds_bytes(MODE)));
   });
   if (attr != hipSuccess) return attr;
   hipLaunchKernelGGL(fn, dim3(static_cast<unsigned>(grid)), dim3(kShThreads), pl.lds, st, prm);
   return hipSuccess;
+}
+
+template <int DT, bool NT>
+hipError_t launch_attend_shared(const MlaParams& prm, const AttendPlan& pl, int64_t grid, hipStream_t st) {
+  if (pl.mode == kShGather) return launch_attend_shared_mode<DT, NT, kShGather>(prm, pl, grid, st);
+  if (pl.mode == kShFold) return launch_attend_shared_mode<DT, NT, kShFold>(prm, pl, grid, st);
+  return launch_attend_shared_mode<DT, NT, kShDense>(prm, pl, grid, st);
 }
 
 template <int DT>
@@ -2706,7 +2919,8 @@ struct PartialRefs {
   int64_t* gtotal;
   int* meta;
 };
-PartialRefs partial_refs(const AttendShape& a, const AttendPlan& pl, void* part_ws) {
+PartialRefs partial_refs(const AttendShape& call, const AttendPlan& pl, void* part_ws) {
+  const AttendShape a = kernel_shape(call, pl);
   const int64_t rows = static_cast<int64_t>(a.B) * a.T;
   char* meta =
       static_cast<char*>(part_ws) + round_up256(static_cast<size_t>(pl.wgs + rows) * a.H * partial_stride(a, pl) * 4);
@@ -2719,10 +2933,11 @@ uint64_t* g_mla_stamps = nullptr;  // diagnostic build: qd_diag_set_mla_stamps
 
 // skip_merge: the caller merges the split rows itself (mla_decode's value
 // projection, MFMA kernels with half-precision partials only).
-int run_attend(const AttendShape& a, const void* q, const void* qr, const void* cache, const int32_t* table,
+int run_attend(const AttendShape& call, const void* q, const void* qr, const void* cache, const int32_t* table,
                const int32_t* lens, const int32_t* pos, const int32_t* idx, int causal, int64_t num_blocks,
                float scale, void* out, void* part_ws, size_t part_bytes, const AttendPlan& pl, hipStream_t st,
                bool skip_merge = false) {
+  const AttendShape a = kernel_shape(call, pl);
   MlaParams prm{};
 #ifdef QD_STAMPS
   prm.stamps = g_mla_stamps;
@@ -2747,6 +2962,7 @@ int run_attend(const AttendShape& a, const void* q, const void* qr, const void* 
   prm.nk = a.nk;
   prm.causal = causal ? 1 : 0;
   prm.splits = pl.splits;
+  prm.fold = a.T == call.T ? 1 : call.T;
   prm.head_groups = pl.head_groups;
   prm.kch = pl.kch;
   prm.nht = pl.nht;
@@ -2756,11 +2972,11 @@ int run_attend(const AttendShape& a, const void* q, const void* qr, const void* 
   prm.num_blocks = num_blocks;
   const int64_t rows = static_cast<int64_t>(a.B) * a.T;
   prm.sl2 = scale * kLog2e;
-  const size_t need = attend_partial_bytes(a, pl);
+  const size_t need = attend_partial_bytes(call, pl);
   if (need > 0 && (part_bytes < need || !part_ws || !aligned16(part_ws)))
     return mla_fail(nullptr, 0, "workspace too small for the attention partials");
   if (pl.mfma) {
-    const PartialRefs pr = partial_refs(a, pl, part_ws);
+    const PartialRefs pr = partial_refs(call, pl, part_ws);
     prm.gtotal = pr.gtotal;
     prm.meta = pr.meta;
   }
@@ -2928,6 +3144,13 @@ DecodeLayout decode_layout(const AttendShape& a, const AttendPlan& pl) {
   return d;
 }
 
+// A pool of 2^31 rows or more (32-bit row lists do not reach it; its plans
+// need less workspace than the ones sized without num_blocks) keeps the
+// kernels before the shared-tile one for gathered rows.
+int gather_flags(int64_t num_blocks, int block_size, int flags) {
+  return num_blocks * block_size > 2147483647LL ? flags | kNoGather : flags;
+}
+
 bool attend_shape_ok(const AttendShape& a) {
   return a.B >= 0 && a.T >= 0 && a.H > 0 && a.Dc > 0 && a.Dc <= 512 && a.Dr > 0 && a.P > 0 && a.maxP > 0 &&
          a.nk >= -1 && float_dtype(a.dtype) && a.B <= 65535 && a.T <= 65535;
@@ -3081,7 +3304,7 @@ int qd_mla_attend(const void* q, const void* q_rope, const void* cache, const in
   if (static_cast<int64_t>(batch) * q_len == 0) return QD_OK;
   if (!q || !q_rope || !cache || !block_table || !lengths || !positions || !out)
     return mla_fail(nullptr, 0, "null tensor pointer");
-  AttendPlan pl = plan_attend(a, splits, flags);
+  AttendPlan pl = plan_attend(a, splits, gather_flags(num_blocks, block_size, flags));
   if (pl.mfma && !(aligned16(cache) && aligned16(out))) pl.mfma = false;
   return run_attend(a, q, q_rope, cache, block_table, lengths, positions, indices, causal, num_blocks, scale, out,
                     workspace, workspace_bytes, pl, static_cast<hipStream_t>(stream));
@@ -3151,7 +3374,7 @@ int qd_mla_decode(const void* q_nope, const void* q_rope, const void* cache, con
   if (rows == 0) return QD_OK;
   if (!q_nope || !q_rope || !cache || !block_table || !lengths || !positions || !w_uk || !w_uv || !out)
     return mla_fail(nullptr, 0, "null tensor pointer");
-  AttendPlan pl = plan_attend(a, splits, flags);
+  AttendPlan pl = plan_attend(a, splits, gather_flags(num_blocks, block_size, flags));
   const DecodeLayout lay = decode_layout(a, pl);
   if (!workspace || workspace_bytes < lay.total || !aligned16(workspace))
     return mla_fail(nullptr, 0, "workspace must hold qd_mla_decode_workspace_bytes() bytes, 16-byte aligned");
@@ -3165,7 +3388,7 @@ int qd_mla_decode(const void* q_nope, const void* q_rope, const void* cache, con
   // The merge of split rows folded into the value projection when it runs
   // the 16-row MFMA tiling (launch_project's choice for small batches).
   const int64_t fill = 2 * static_cast<int64_t>(device_cus());
-  const bool fuse = pl.mfma && half_partials(pl) && latent_dim == 512 && (flags & QD_FLAG_FORCE_GENERIC) == 0 &&
+  const bool fuse = pl.mfma && half_partials(pl) && pl.mode != kShFold && latent_dim == 512 && (flags & QD_FLAG_FORCE_GENERIC) == 0 &&
                     project_mfma_applies(rows, latent_dim, value_dim, dtype, latent, w_uv, out) &&
                     (rows < 64 || (value_dim + 127) / 128 * heads * ((rows + 63) / 64) < fill) &&
                     (rows + 15) / 16 <= 65535;

@@ -524,3 +524,93 @@ def test_mla_attend_fp16_partial_error_bound(gpu, heads, flags):
     bound = 4 * 2.0 ** -12 * bmax + 0.5 * ulp(one) + 0.5 * ulp(three) + 2.0 ** -24
     diff = (three - one).abs()
     assert torch.all(diff <= bound), f"max excess {(diff - bound).max().item():.3e}"
+
+
+def _attend(c, qa, scale, *, causal=True, indices=None, splits=0):
+    out = torch.full_like(qa, float("nan"))
+    rc = cabi.mla_attend(qa, c["q_rope"], c["cache"], c["table"], c["lens"], c["positions"], out, scale=scale,
+                         indices=indices, causal=causal, splits=splits)
+    assert rc == 0, cabi.error_string(rc)
+    torch.cuda.synchronize()
+    return out
+
+
+# (name, heads, q_len, page, K listed tokens per query or None, lengths)
+GATHER_SHAPES = [
+    ("h64-k100", 64, 1, 64, 100, [300, 5, 0, 129]),
+    ("h128-k33-t2", 128, 2, 16, 33, [40, 700, 1]),
+    ("h96-k1", 96, 1, 32, 1, [64, 2]),
+    ("h64-k2048", 64, 1, 64, 2048, [5000, 2047, 2049]),
+    ("h64-k32-page7", 64, 3, 7, 32, [50, 31, 200]),
+    ("h64-dense-page1", 64, 1, 1, None, [1, 31, 32, 33, 700, 0]),
+    ("h128-dense-page8-t2", 128, 2, 8, None, [2, 65, 1000]),
+]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+@pytest.mark.parametrize("shape", GATHER_SHAPES, ids=[s[0] for s in GATHER_SHAPES])
+def test_mla_gathered_rows_on_the_shared_tile_kernel(gpu, shape, dtype):
+    """Listed tokens, and pages that hold no whole 16-token groups, with 64 or
+    more heads: the shared-tile kernel takes them and matches the oracle whole
+    and with 1, 3 and 7 ranges, entries that are not visible ignored (whole
+    tiles and whole rows of them too), a repeated entry counted twice.  Cache
+    rows that no list names hold NaN."""
+    name, heads, q_len, page, k, lengths = shape
+    say(f"mla gathered rows {name} {dtype}")
+    c = _case(gpu, lengths=lengths, q_len=q_len, heads=heads, block_size=page, dtype=dtype, num_indices=k)
+    idx = c["indices"]
+    if idx is not None:
+        if k >= 33:
+            idx[0, 0, 1:k - 1:3] = -1
+            idx[-1, -1, :32] = torch.tensor([10_000] * 31 + [-5], dtype=torch.int32)   # a tile without a visible row
+            idx[0, 0, 0] = idx[0, 0, k - 1] = 3
+        idx[1, 0] = -1                                                                 # nothing listed
+        seen = torch.zeros(c["cache"].shape[:2], dtype=torch.bool)
+        for b, n in enumerate(lengths):
+            for t in range(q_len):
+                for tok in {int(x) for x in idx[b, t].tolist() if 0 <= x < n}:
+                    seen[int(c["table"][b, tok // page]), tok % page] = True
+        clean = c["cache"].clone()
+        c["cache"][~seen.to(gpu)] = float("nan")
+    kind = cabi.mla_attend_info(len(lengths), q_len, heads, 512, 64, page, c["table"].shape[1],
+                                nk=-1 if idx is None else k)[0]
+    assert kind == 3
+    qa = _absorbed(c, dtype).to(dtype).to(gpu)
+    scale = default_mla_scale(c["q_nope"].shape[-1], c["q_rope"].shape[-1])
+    outs = [_attend(c, qa, scale, indices=idx, splits=s) for s in (0, 1, 3, 7)]
+    if idx is not None:
+        c["cache"] = clean
+    ref = _oracle_attend(c, qa, scale, True, idx, dtype)
+    for out, s in zip(outs, (0, 1, 3, 7)):
+        _close(out, ref, dtype, f"{name} splits={s}")
+
+
+# (name, heads, q_len, page, lengths)
+FOLD_SHAPES = [
+    ("h16-t4", 16, 4, 64, [0, 3, 4, 40, 1031]),       # a query before the context starts
+    ("h20-t4", 20, 4, 32, [33, 500]),                 # 80 heads: a quarter of the second head group
+    ("h32-t2", 32, 2, 64, [1, 2, 63, 64, 65, 2500]),
+    ("h128-t3", 128, 3, 32, [31, 32, 34, 900]),
+]
+
+
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+@pytest.mark.parametrize("shape", FOLD_SHAPES, ids=[s[0] for s in FOLD_SHAPES])
+def test_mla_folded_queries(gpu, shape, dtype, causal):
+    """Several queries per sequence as heads of one row of the shared-tile
+    kernel: each query sees its own prefix (positions out of order and past
+    the end too), whole and with 1, 3 and 7 ranges."""
+    name, heads, q_len, page, lengths = shape
+    say(f"mla folded queries {name} {dtype} causal={causal}")
+    c = _case(gpu, lengths=lengths, q_len=q_len, heads=heads, block_size=page, dtype=dtype)
+    c["positions"][-1] = c["positions"][-1].flip(0)
+    c["positions"][-2, 0] = 2 ** 31 - 1
+    c["positions"][1, -1] = -3
+    kind = cabi.mla_attend_info(len(lengths), q_len, heads, 512, 64, page, c["table"].shape[1])[0]
+    assert kind == 3
+    qa = _absorbed(c, dtype).to(dtype).to(gpu)
+    scale = default_mla_scale(c["q_nope"].shape[-1], c["q_rope"].shape[-1])
+    ref = _oracle_attend(c, qa, scale, causal, None, dtype)
+    for s in (0, 1, 3, 7):
+        _close(_attend(c, qa, scale, causal=causal, splits=s), ref, dtype, f"{name} splits={s}")
