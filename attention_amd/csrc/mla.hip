@@ -2399,14 +2399,21 @@ __global__ __launch_bounds__(kShThreads) void mla_attend_shared_kernel(MlaParams
 // HALF: half-precision rows of the shared-tile and wave kernels
 // (kHalfHeader, Dc = 512); lane j folds columns 8 j .. 8 j + 7 (one 16-byte
 // load per row and one store).
-template <int DT, bool HALF>
+//
+// WIDE: a workgroup per (row, head), for rows split over many ranges: wave v
+// folds batches v, v + 4, ... and wave 0 then the four states in order, a
+// quarter of the dependent round trips (mla_decode at the same ranges, 16
+// heads: B1/L30000 61.8 -> 41.4 us, B16/L4000 46.5 -> 35.1; 128 heads B4/L16000
+// 67.5 -> 49.2).
+template <int DT, bool HALF, bool WIDE>
 __global__ __launch_bounds__(256) void mla_merge_sk_kernel(MlaParams p) {
   using E = Elem<DT>;
   using S = typename E::S;
   constexpr int kAcc = 8;
   constexpr int kBatch = 8;
   const int lane = threadIdx.x & 63;
-  const int64_t wid = static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
+  const int wv = static_cast<int>(threadIdx.x) >> 6;
+  const int64_t wid = WIDE ? static_cast<int64_t>(blockIdx.x) : static_cast<int64_t>(blockIdx.x) * 4 + wv;
   if (wid >= static_cast<int64_t>(p.B) * p.T * p.H) return;
   const int64_t r = wid / p.H;
   const int h = static_cast<int>(wid % p.H);
@@ -2426,7 +2433,7 @@ __global__ __launch_bounds__(256) void mla_merge_sk_kernel(MlaParams p) {
   float acc[kAcc];
 #pragma unroll
   for (int j = 0; j < kAcc; ++j) acc[j] = 0.f;
-  for (int c = 0; c < nwg; c += kBatch) {
+  for (int c = WIDE ? kBatch * wv : 0; c < nwg; c += WIDE ? 4 * kBatch : kBatch) {
     float ms[kBatch], ls[kBatch], v[kBatch][kAcc];
 #pragma unroll
     for (int t = 0; t < kBatch; ++t) {
@@ -2463,6 +2470,26 @@ __global__ __launch_bounds__(256) void mla_merge_sk_kernel(MlaParams p) {
     for (int t = 0; t < kBatch; ++t) {
       if (ls[t] == 0.f) continue;  // absent or empty partial
       lse_fold(M, L, acc, ms[t], ls[t], v[t]);
+    }
+  }
+  if constexpr (WIDE) {
+    __shared__ float sacc[4][kAcc][64];
+    __shared__ float sml[4][2];
+#pragma unroll
+    for (int j = 0; j < kAcc; ++j) sacc[wv][j][lane] = acc[j];
+    if (lane == 0) {
+      sml[wv][0] = M;
+      sml[wv][1] = L;
+    }
+    __syncthreads();
+    if (wv != 0) return;
+#pragma unroll
+    for (int u = 1; u < 4; ++u) {
+      if (sml[u][1] == 0.f) continue;
+      float v[kAcc];
+#pragma unroll
+      for (int j = 0; j < kAcc; ++j) v[j] = sacc[u][j][lane];
+      lse_fold(M, L, acc, sml[u][0], sml[u][1], v);
     }
   }
   S* orow = static_cast<S*>(p.out) + wid * p.Dc;
@@ -2706,21 +2733,28 @@ bool shared_fold_applies(int q_len, int heads) { return q_len * heads >= 32; }
 
 // Ranges (workgroups per head group) for `rows` rows of at most `tiles` tiles:
 // the CUs, but per row at most per_row * sqrt(tiles).  A row split over x
-// ranges takes tiles / x steps and then a fold of x partials, 8 per memory
-// round trip, so the best x grows with the square root of the tiles; one row
-// on every CU folded 256 of them.  The factors were swept from 0.25 to 8 over
-// 1-128 rows of 64-30000 tokens (graph replays, us per mla_decode, all CUs ->
-// now; full batches keep all CUs):
-//   wave kernel, 16 heads     B1/L500 56.4 -> 26.1, B1/L4000 125 -> 31.0, B1/L30000 220 -> 58.5,
-//                             B4/L4000 80.0 -> 40.0, B16/L4000 46.6 -> 40.9
-//   shared-tile, 128 heads    B1/L4000 81.2 -> 35.3, B1/L30000 132 -> 70.9, B4/L16000 75.8 -> 67.5
-//   staged, 16 heads, K 2048  B1 128 -> 42, B4 66.7 -> 43.9
-constexpr double kShRangesPerRow = 1.1, kWaveRangesPerRow = 0.6, kStagedRangesPerRow = 2.0;
+// ranges takes tiles / x steps and then a fold of x partials, so the best x
+// grows with the square root of the tiles; one row on every CU folded 256 of
+// them.  The factors were swept from 0.25 to 8 over 1-128 rows of 64-30000
+// tokens (graph replays, us per mla_decode: all CUs and 8 partials per round
+// trip -> now, with mla_merge_sk_kernel's WIDE; batches that fill the CUs
+// with a few ranges per row keep them all):
+//   wave kernel, 16 heads     B1/L500 56.4 -> 24.4, B1/L4000 125 -> 28.2, B1/L30000 220 -> 39.6,
+//                             B4/L4000 80.0 -> 31.6, B16/L4000 46.6 -> 35.1
+//   shared-tile, 128 heads    B1/L4000 81.2 -> 32.9, B1/L30000 132 -> 48.6, B4/L16000 75.8 -> 49.0
+//   staged, 16 heads, K 2048  B1 128 -> 33.1, B4 66.7 -> 35.1
+// The grid has whole octets of ranges (one per XCD) for every head group: with
+// a part octet beyond the CUs, workgroups waited for a second round while the
+// idle ones freed CUs of other XCDs (3 groups, B8 3 x 64 heads U[100, 2000]: 85
+// ranges 57.6 us, 80 ranges 39.1).
+constexpr double kShRangesPerRow = 2.0, kWaveRangesPerRow = 2.0, kStagedRangesPerRow = 3.0;
 
 int range_count(int64_t rows, int64_t tiles, int groups, double per_row) {
   const double per = std::ceil(per_row * std::sqrt(static_cast<double>(std::max<int64_t>(tiles, 1))));
-  const int64_t cap = rows * static_cast<int64_t>(per);
-  return static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(device_cus() / groups, cap)));
+  const int64_t most = rows * static_cast<int64_t>(per);
+  int64_t n = std::max<int64_t>(1, std::min<int64_t>(device_cus() / groups, most));
+  if (n > 8 && (n + 7) / 8 * 8 * groups > device_cus()) n = n / 8 * 8;
+  return static_cast<int>(n);
 }
 
 AttendPlan plan_attend(const AttendShape& a, int forced, int flags) {
@@ -2835,6 +2869,14 @@ AttendShape kernel_shape(const AttendShape& a, const AttendPlan& pl) {
 }
 int partial_stride(const AttendShape& a, const AttendPlan& pl) {
   return half_partials(pl) ? kHalfPst : a.Dc + 2;
+}
+
+// Rows split over many ranges are merged by a workgroup per (row, head); the
+// value projection of mla_decode then takes whole rows (its own fold walks a
+// row's partials 8 per round trip, as the other merge does).
+constexpr int64_t kWideMergeRanges = 8;
+bool wide_merge(const AttendShape& kernel_shape, const AttendPlan& pl) {
+  return pl.wgs > kWideMergeRanges * kernel_shape.B * kernel_shape.T;
 }
 
 size_t attend_partial_bytes(const AttendShape& call, const AttendPlan& pl) {
@@ -3026,11 +3068,16 @@ int run_attend(const AttendShape& call, const void* q, const void* qr, const voi
   if (pl.mfma) {
     using MergeFn = void (*)(MlaParams);
     MergeFn fn = nullptr;
-    if (a.dtype == QD_DTYPE_BF16)
-      fn = half_partials(pl) ? mla_merge_sk_kernel<QD_DTYPE_BF16, true> : mla_merge_sk_kernel<QD_DTYPE_BF16, false>;
+    const bool wide = wide_merge(a, pl);
+    if (half_partials(pl))
+      fn = a.dtype == QD_DTYPE_BF16
+               ? (wide ? mla_merge_sk_kernel<QD_DTYPE_BF16, true, true> : mla_merge_sk_kernel<QD_DTYPE_BF16, true, false>)
+               : (wide ? mla_merge_sk_kernel<QD_DTYPE_F16, true, true> : mla_merge_sk_kernel<QD_DTYPE_F16, true, false>);
     else
-      fn = half_partials(pl) ? mla_merge_sk_kernel<QD_DTYPE_F16, true> : mla_merge_sk_kernel<QD_DTYPE_F16, false>;
-    hipLaunchKernelGGL(fn, dim3(mgrid), dim3(256), 0, st, prm);
+      fn = a.dtype == QD_DTYPE_BF16
+               ? (wide ? mla_merge_sk_kernel<QD_DTYPE_BF16, false, true> : mla_merge_sk_kernel<QD_DTYPE_BF16, false, false>)
+               : (wide ? mla_merge_sk_kernel<QD_DTYPE_F16, false, true> : mla_merge_sk_kernel<QD_DTYPE_F16, false, false>);
+    hipLaunchKernelGGL(fn, dim3(static_cast<unsigned>(wide ? rows * a.H : mgrid)), dim3(256), 0, st, prm);
     return launch_status("mla_attend merge");
   }
   switch (a.dtype) {
@@ -3388,7 +3435,7 @@ int qd_mla_decode(const void* q_nope, const void* q_rope, const void* cache, con
   // The merge of split rows folded into the value projection when it runs
   // the 16-row MFMA tiling (launch_project's choice for small batches).
   const int64_t fill = 2 * static_cast<int64_t>(device_cus());
-  const bool fuse = pl.mfma && half_partials(pl) && pl.mode != kShFold && latent_dim == 512 && (flags & QD_FLAG_FORCE_GENERIC) == 0 &&
+  const bool fuse = pl.mfma && half_partials(pl) && pl.mode != kShFold && !wide_merge(a, pl) && latent_dim == 512 && (flags & QD_FLAG_FORCE_GENERIC) == 0 &&
                     project_mfma_applies(rows, latent_dim, value_dim, dtype, latent, w_uv, out) &&
                     (rows < 64 || (value_dim + 127) / 128 * heads * ((rows + 63) / 64) < fill) &&
                     (rows + 15) / 16 <= 65535;
