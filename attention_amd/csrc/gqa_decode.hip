@@ -1141,12 +1141,14 @@ struct GenWave : MfmaWave<VD, DT, PF, 1> {
   int krow[KCG];     // K load c of this lane: row of the group ...
   int kcol[KCG];     // ... and byte offset in the row
   int voff;          // byte offset of this lane's V piece
+  int tok0;          // token of group 0 (a split may start at any page)
   int32_t* win;      // this wave's table window
 
   __device__ void init_lane_gen(const DecodeParams& p, char* ktile, int32_t* window) {
     Base::init_lane();
     dm = p.D;
     win = window;
+    tok0 = 0;
     const int per_row = dm >> 3;  // 16-byte pieces of a K row
 #pragma unroll
     for (int c = 0; c < KCG; ++c) {
@@ -1168,7 +1170,7 @@ struct GenWave : MfmaWave<VD, DT, PF, 1> {
   }
 
   __device__ int pages_to(const DecodeParams& p, int gb, int first) const {
-    const uint32_t last = min(16u * static_cast<uint32_t>(gb), static_cast<uint32_t>(this->len)) - 1u;
+    const uint32_t last = min(tok0 + 16u * static_cast<uint32_t>(gb), static_cast<uint32_t>(this->len)) - 1u;
     return page_of(p, static_cast<int>(last)) - first + 1;
   }
 
@@ -1177,7 +1179,7 @@ struct GenWave : MfmaWave<VD, DT, PF, 1> {
     const bool head_ok = this->r16 < this->hcount;
     this->trow = p.table + static_cast<int64_t>(b) * p.maxP;
     this->len = valid_tokens;
-    const int first = page_of(p, 16 * ga);
+    const int first = page_of(p, tok0 + 16 * ga);
     load_window(p, first, pages_to(p, gb, first));
     const char* qp = static_cast<const char*>(p.q) +
                      (static_cast<int64_t>(b) * p.Hq + vhead_base(p, kvh) + (head_ok ? this->r16 : 0)) * dm * 2;
@@ -1198,7 +1200,7 @@ struct GenWave : MfmaWave<VD, DT, PF, 1> {
   }
 
   __device__ void issue(const DecodeParams& p, Buf& buf, int gi) {
-    const int tg = 16 * gi;
+    const int tg = tok0 + 16 * gi;
     buf.tg = tg;
     // Pool row of token r16 (tokens at or past the end re-read the last one);
     // num_blocks * P < 2^31 (host check).
@@ -1264,10 +1266,10 @@ struct GenWave : MfmaWave<VD, DT, PF, 1> {
   __device__ void run(const DecodeParams& p, int ga, int gb, char* ktile, bool lockstep = false) {
     for (int g_lo = ga; g_lo < gb;) {
       if (g_lo != ga) {  // the first window came with begin_item_gen
-        const int first = page_of(p, 16 * g_lo);
+        const int first = page_of(p, tok0 + 16 * g_lo);
         load_window(p, first, pages_to(p, gb, first));
       }
-      const int64_t whole = static_cast<int64_t>(this->wbase + kWinPages) * p.P >> 4;  // groups inside the window
+      const int64_t whole = (static_cast<int64_t>(this->wbase + kWinPages) * p.P - tok0) >> 4;  // groups inside the window
       const int g_hi = whole < gb && page_of(p, this->len - 1) >= this->wbase + kWinPages ? static_cast<int>(whole) : gb;
       const int n = g_hi - g_lo;
       Buf buf[PF];
@@ -1774,8 +1776,11 @@ __global__ __launch_bounds__((64 * sk_max_waves<D, 1, 0, PF, DT>())) void decode
   else
     wv.init_lane();
 
-  const int ga = ci.tb >> 4;  // tb is 0 or a multiple of a page of whole groups
-  const int n = ((ci.te + 15) >> 4) - ga;
+  // Groups of the split: from its first token in the general layout, else of
+  // the sequence (tb lies on whole groups).
+  const int ga = kGen ? 0 : ci.tb >> 4;
+  const int n = kGen ? (ci.te - ci.tb + 15) >> 4 : ((ci.te + 15) >> 4) - ga;
+  if constexpr (kGen) wv.tok0 = ci.tb;
   const int per = (n + p.wg_waves - 1) / p.wg_waves;
   const int act = per > 0 ? (n + per - 1) / per : 0;  // waves with groups: the first `act`
   const int g0 = ga + wid * per;
@@ -3332,6 +3337,15 @@ DecodeParams make_params(const void* q, const void* k_cache, const void* v_cache
   return prm;
 }
 
+// Serves each kv-head as c chunks of its q-heads (kv_split_for).
+void use_kv_chunks(DecodeParams* prm, int q_heads, int kv_heads, int c) {
+  prm->Hkv = kv_heads * c;
+  prm->g = kv_chunk_heads(q_heads, kv_heads, c);
+  prm->kv_split = c;
+  prm->kv_rows = kv_heads;
+  prm->kv_g = q_heads / kv_heads;
+}
+
 // Scratch bytes the automatic path needs for these shapes: the larger of
 // the aligned and unaligned plans, so that the size does not depend on
 // pointer alignment (QD_STAGE_VALU's plan runs on the same grid and fits).
@@ -3546,12 +3560,22 @@ int qd_gqa_decode_launch(const void* q, const void* k_cache, const void* v_cache
   const bool use_mfma = qd_gqa_decode_kernel_kind(q_heads, kv_heads, head_dim, block_size, dtype, flags) &&
                         aligned16(q) && aligned16(k_cache) && aligned16(v_cache) && aligned16(out) &&
                         (splits <= 1 || (reinterpret_cast<uintptr_t>(workspace) & 7u) == 0);
+  // The general layout where the exact one does not apply, with groups above
+  // kMfmaHeads in chunks as on the balanced path (reported as kind 0 by
+  // qd_gqa_decode_kernel_kind, like the VALU kernel).
+  const int split_kv = kv_split_for(q_heads, kv_heads);
+  const bool general = !use_mfma && (flags & QD_FLAG_FORCE_GENERIC) == 0 && general_applies(head_dim, dtype) &&
+                       split_kv > 0 && static_cast<int64_t>(kv_heads) * split_kv <= 65535 &&
+                       num_blocks * block_size <= 2147483647LL && aligned16(q) && aligned16(k_cache) &&
+                       aligned16(v_cache) && aligned16(out) &&
+                       (splits <= 1 || (reinterpret_cast<uintptr_t>(workspace) & 7u) == 0);
   (void)hipGetLastError();  // start from a clean error state
-  if (use_mfma) {
+  if (use_mfma || general) {
     const int cp = chunk_pages > 0 ? chunk_pages : (max_pages + splits - 1) / splits;
-    prm.wg_waves = wg_waves_for(static_cast<int64_t>(splits) * kv_heads * batch,
+    if (general && split_kv > 1) use_kv_chunks(&prm, q_heads, kv_heads, split_kv);
+    prm.wg_waves = wg_waves_for(static_cast<int64_t>(splits) * prm.Hkv * batch,
                                 (static_cast<int64_t>(cp) * block_size + 15) / 16, dtype, head_dim);
-    st = launch_wg(prm, dtype, head_dim, false, splits, kv_heads, batch, stm);
+    st = launch_wg(prm, dtype, head_dim, general, splits, prm.Hkv, batch, stm);
     if (st != QD_OK) return st;
   } else {
     KernelFn fn;
@@ -3639,13 +3663,7 @@ int qd_gqa_decode_auto_stages(const void* q, const void* k_cache, const void* v_
   prm.wg_waves = ap.wg_waves;
   prm.kv_slices = fused ? 1 : ap.kv_slices;
   prm.stage_bytes = ap.stage_bytes ? static_cast<int>(ap.stage_bytes / ap.wg_waves) : 0;
-  if (ap.kv_split > 1) {
-    prm.Hkv = kv_heads * ap.kv_split;
-    prm.g = kv_chunk_heads(q_heads, kv_heads, ap.kv_split);
-    prm.kv_split = ap.kv_split;
-    prm.kv_rows = kv_heads;
-    prm.kv_g = q_heads / kv_heads;
-  }
+  if (ap.kv_split > 1) use_kv_chunks(&prm, q_heads, kv_heads, ap.kv_split);
   hipStream_t stm = static_cast<hipStream_t>(stream);
   (void)hipGetLastError();
   if (single) {

@@ -136,7 +136,11 @@ int qd_gqa_decode_launch(const void* q, const void* k_cache, const void* v_cache
                          int chunk_pages, int flags, void* stream);
 
 /* Which kernel qd_gqa_decode_launch would run for these shapes:
- * 1 = MFMA kernel, 0 = portable VALU kernel. */
+ * 1 = the MFMA kernel for head_dim 64/96/128/256, whole 16-token groups per
+ * page and groups of at most 16 q-heads, 0 = the others: the general MFMA
+ * layout (16-bit, head_dim a multiple of 8 up to 128 or of 16 up to 256,
+ * groups up to 128, not with QD_FLAG_FORCE_GENERIC) or the portable VALU
+ * kernel. */
 int qd_gqa_decode_kernel_kind(int q_heads, int kv_heads, int head_dim, int block_size,
                               int dtype, int flags);
 
@@ -227,7 +231,8 @@ int qd_gqa_decode_auto_stages(const void* q, const void* k_cache, const void* v_
  * file-scope device array of qd_gqa_decode_noalloc_scratch_bytes() bytes
  * (16 MiB) per GPU, held until the process ends; shapes whose
  * qd_gqa_decode_auto_workspace_bytes() exceed it are rejected with
- * QD_ERR_INVALID_VALUE before anything is enqueued.  Nothing is allocated
+ * QD_ERR_INVALID_VALUE before anything is enqueued (shapes of the general
+ * kernel, only where the split layout's partials exceed it too).  Nothing is allocated
  * (the array's address is looked up once per device).  Every call on a GPU
  * uses that GPU's one array: calls that may overlap on one GPU (different
  * streams, host threads) race and must be serialized by the caller. */
@@ -241,7 +246,11 @@ int qd_gqa_decode_auto_noalloc(const void* q, const void* k_cache, const void* v
 /* Describes the automatic path's choice (assuming aligned pointers):
  * returns 2 for the balanced MFMA path with the fused merge, 1 for it with
  * the separate merge kernel (*waves = its total wave count), 0 for the split
- * path (*splits, *chunk_pages), -1 for invalid shapes.  Any output pointer
+ * path (*splits, *chunk_pages), -1 for invalid shapes.  Whole calls whose
+ * shape is reported as 0 may run the balanced kernels all the same (the
+ * general layout, fp32 from 16384 tokens of capacity), and short contexts of
+ * any kind run in one launch; what is reported is what stages, or a
+ * workspace of the split layout's size, get.  Any output pointer
  * may be NULL. */
 int qd_gqa_decode_auto_info(int batch, int q_heads, int kv_heads, int head_dim, int block_size,
                             int max_pages, int dtype, int* waves, int* splits, int* chunk_pages);

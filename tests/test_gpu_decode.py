@@ -1205,3 +1205,25 @@ def test_one_launch_short_contexts(gpu, shape):
     assert torch.equal(merged, torch.full_like(q, 7.0))
     out = run(cabi.QD_STAGE_ALL | cabi.QD_STAGE_UNFUSED, torch.full_like(q, float("nan")))
     assert_close(out, ref, DT_NAME[dtype], rows, "balanced")
+
+
+@pytest.mark.parametrize("shape", GENERAL_SHAPES[:16],
+                         ids=lambda s: f"{DT_NAME[s[0]]}-Hq{s[1]}-Hkv{s[2]}-D{s[3]}-P{s[4]}-B{len(s[5])}")
+def test_general_layout_explicit_splits(gpu, shape):
+    """The general layout on caller-given splits, which start at any page (so
+    inside a 16-token group): every row matches the oracle, and the VALU
+    kernel of the same call."""
+    dtype, hq, hkv, d, p, lengths = shape
+    say(f"general splits {DT_NAME[dtype]} Hq{hq} Hkv{hkv} D{d} P{p}")
+    q, k, v, table, lens = to_dev(make_decode_case(lengths=lengths, q_heads=hq, kv_heads=hkv, head_dim=d, block_size=p,
+                                                   dtype=dtype, seed=145), gpu)
+    ref, rows = oracle_rows((q, k, v, table, lens))
+    for splits, chunk in [(1, 0), (3, 0), (7, 0), (-(-table.shape[1] // 2), 2)]:
+        ws = torch.full((max(1, q.shape[0] * hq * splits * (d + 2)),), float("nan"), device=gpu, dtype=torch.float32)
+        for flags in (0, cabi.QD_FLAG_FORCE_GENERIC):
+            out = torch.full_like(q, float("nan"))
+            rc = cabi.launch(q, k, v, table, lens, out, scale=1 / math.sqrt(d), splits=splits, chunk_pages=chunk,
+                             workspace=ws if splits > 1 else None, flags=flags)
+            assert rc == 0, cabi.error_string(rc)
+            torch.cuda.synchronize()
+            assert_close(out, ref, DT_NAME[dtype], rows, f"splits={splits} chunk={chunk} flags={flags}")
