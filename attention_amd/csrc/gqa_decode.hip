@@ -1103,7 +1103,7 @@ constexpr int kGenWinPages = 512;  // page-table window of the general layout (L
 // One wave's decode state for one kv-head in the general layout: 16-bit
 // caches with any block_size and any head_dim Dm = p.D that is a multiple of
 // 8 up to 128 or of 16 up to 256 (VD = 64, 128 or 256 is the next V layout,
-// KC = 32-wide QK chunks covering Dm).  MfmaWave's lane layouts with two
+// KCG = 64-byte chunks covering a K row), and fp32 caches alike.  MfmaWave's lane layouts with two
 // changes:
 //   rows   a 16-token group may span pages, so lane r16 finds the pool row of
 //          token r16 (its page from a window of the table row in LDS, the
@@ -1127,13 +1127,16 @@ struct GenWave : MfmaWave<VD, DT, PF, 1> {
   using Base = MfmaWave<VD, DT, PF, 1>;
   using Ops = MfmaOps<DT>;
   using S = typename Elem<DT>::S;
+  static constexpr bool kF32 = DT == QD_DTYPE_F32;
+  static constexpr int ES = kF32 ? 4 : 2;           // bytes per element
+  using VR = VRow<VD * ES / 2>;                     // a lane's EV elements of a V row
   static constexpr int EV = VD / 16;                // V elements per lane and row
   static constexpr int kStride = 64 * KCG + 32;     // LDS bytes per K row
   static constexpr int kTileBytes = 16 * kStride;
   static constexpr int kWinPages = kGenWinPages;
   struct Buf {
     u32x4 k[KCG];
-    VRow<VD> v[4];
+    VR v[4];
     int tg;
   };
   u32x4 qg[KCG];
@@ -1149,14 +1152,14 @@ struct GenWave : MfmaWave<VD, DT, PF, 1> {
     dm = p.D;
     win = window;
     tok0 = 0;
-    const int per_row = dm >> 3;  // 16-byte pieces of a K row
+    const int per_row = dm * ES >> 4;  // 16-byte pieces of a K row
 #pragma unroll
     for (int c = 0; c < KCG; ++c) {
       const int piece = min(64 * c + this->lane, 16 * per_row - 1);
       krow[c] = piece / per_row;
       kcol[c] = 16 * (piece - krow[c] * per_row);
     }
-    voff = 2 * min(EV * this->r16, dm - EV);
+    voff = ES * min(EV * this->r16, dm - EV);
     for (int o = 16 * this->lane; o < kTileBytes; o += 1024)
       *reinterpret_cast<u32x4*>(ktile + o) = u32x4{0u, 0u, 0u, 0u};
   }
@@ -1182,21 +1185,21 @@ struct GenWave : MfmaWave<VD, DT, PF, 1> {
     const int first = page_of(p, tok0 + 16 * ga);
     load_window(p, first, pages_to(p, gb, first));
     const char* qp = static_cast<const char*>(p.q) +
-                     (static_cast<int64_t>(b) * p.Hq + vhead_base(p, kvh) + (head_ok ? this->r16 : 0)) * dm * 2;
+                     (static_cast<int64_t>(b) * p.Hq + vhead_base(p, kvh) + (head_ok ? this->r16 : 0)) * dm * ES;
 #pragma unroll
     for (int c = 0; c < KCG; ++c) {
-      const int e = 32 * c + 8 * this->q4;
-      const u32x4 x = *reinterpret_cast<const u32x4*>(qp + 2 * min(e, dm - 8));
+      const int at = 64 * c + 16 * this->q4;
+      const u32x4 x = *reinterpret_cast<const u32x4*>(qp + min(at, dm * ES - 16));
       const u32x4 zero = {0u, 0u, 0u, 0u};
-      qg[c] = head_ok && e < dm ? x : zero;
+      qg[c] = head_ok && at < dm * ES ? x : zero;
     }
     this->m_run[0] = -INFINITY;
     this->l_run[0] = 0.f;
 #pragma unroll
     for (int d = 0; d < EV; ++d) this->acc[0][d] = f32x4{0.f, 0.f, 0.f, 0.f};
     const int64_t col = p.kv_split > 1 ? kvh / p.kv_split : kvh;
-    this->kbase = static_cast<const char*>(p.k) + col * dm * 2;
-    this->vbase = static_cast<const char*>(p.v) + col * dm * 2;
+    this->kbase = static_cast<const char*>(p.k) + col * dm * ES;
+    this->vbase = static_cast<const char*>(p.v) + col * dm * ES;
   }
 
   __device__ void issue(const DecodeParams& p, Buf& buf, int gi) {
@@ -1207,7 +1210,7 @@ struct GenWave : MfmaWave<VD, DT, PF, 1> {
     const int t = static_cast<int>(min(static_cast<uint32_t>(tg + this->r16), static_cast<uint32_t>(this->len - 1)));
     const int page = page_of(p, t);
     const int row = clamp_page(win[page - this->wbase], p.num_blocks) * p.P + (t - page * p.P);
-    const int64_t row_bytes = static_cast<int64_t>(p.kv_rows) * dm * 2;
+    const int64_t row_bytes = static_cast<int64_t>(p.kv_rows) * dm * ES;
 #pragma unroll
     for (int c = 0; c < KCG; ++c) {
       const int64_t r = __builtin_amdgcn_ds_bpermute(4 * krow[c], row);
@@ -1216,7 +1219,7 @@ struct GenWave : MfmaWave<VD, DT, PF, 1> {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int64_t r = __builtin_amdgcn_ds_bpermute(4 * (4 * this->q4 + i), row);
-      buf.v[i] = load_vrow<VD>(this->vbase + r * row_bytes + voff);
+      buf.v[i] = load_vrow<VD * ES / 2>(this->vbase + r * row_bytes + voff);
     }
     __builtin_amdgcn_sched_barrier(0);
   }
@@ -1231,7 +1234,15 @@ struct GenWave : MfmaWave<VD, DT, PF, 1> {
       ka[c] = *reinterpret_cast<const u32x4*>(ktile + this->r16 * kStride + 64 * c + 16 * this->q4);
     f32x4 s = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int c = 0; c < KCG; ++c) s = Ops::qk(ka[c], qg[c], s);
+    for (int c = 0; c < KCG; ++c) {
+      if constexpr (kF32) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          s = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(ka[c][e]), __uint_as_float(qg[c][e]), s, 0, 0, 0);
+      } else {
+        s = Ops::qk(ka[c], qg[c], s);
+      }
+    }
     float x[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) x[i] = (4 * this->q4 + i <= last) ? s[i] : -INFINITY;
@@ -1250,14 +1261,23 @@ struct GenWave : MfmaWave<VD, DT, PF, 1> {
 #pragma unroll
       for (int d = 0; d < EV; ++d) this->acc[0][d] *= alpha;
     }
-    const u32x2 hi = {Ops::pack2(pr[0], pr[1]), Ops::pack2(pr[2], pr[3])};
-    const u32x4 w = {hi[0], hi[1], Ops::rest2(pr[0], pr[1], hi[0]), Ops::rest2(pr[2], pr[3], hi[1])};
+    if constexpr (kF32) {
 #pragma unroll
-    for (int d = 0; d < EV; ++d) {
-      const uint32_t sel = (d & 1) ? 0x07060302u : 0x05040100u;
-      const uint32_t a0 = __builtin_amdgcn_perm(buf.v[1].w[d >> 1], buf.v[0].w[d >> 1], sel);
-      const uint32_t a1 = __builtin_amdgcn_perm(buf.v[3].w[d >> 1], buf.v[2].w[d >> 1], sel);
-      this->acc[0][d] = Ops::mma32(u32x4{a0, a1, a0, a1}, w, this->acc[0][d]);
+      for (int d = 0; d < EV; ++d)
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+          this->acc[0][d] = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(buf.v[c].w[d]), pr[c],
+                                                                 this->acc[0][d], 0, 0, 0);
+    } else {
+      const u32x2 hi = {Ops::pack2(pr[0], pr[1]), Ops::pack2(pr[2], pr[3])};
+      const u32x4 w = {hi[0], hi[1], Ops::rest2(pr[0], pr[1], hi[0]), Ops::rest2(pr[2], pr[3], hi[1])};
+#pragma unroll
+      for (int d = 0; d < EV; ++d) {
+        const uint32_t sel = (d & 1) ? 0x07060302u : 0x05040100u;
+        const uint32_t a0 = __builtin_amdgcn_perm(buf.v[1].w[d >> 1], buf.v[0].w[d >> 1], sel);
+        const uint32_t a1 = __builtin_amdgcn_perm(buf.v[3].w[d >> 1], buf.v[2].w[d >> 1], sel);
+        this->acc[0][d] = Ops::mma32(u32x4{a0, a1, a0, a1}, w, this->acc[0][d]);
+      }
     }
     __builtin_amdgcn_sched_barrier(0);
   }
@@ -1310,12 +1330,16 @@ struct GenWave : MfmaWave<VD, DT, PF, 1> {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       if (!block_ok(i)) continue;
-      uint32_t wv[EV / 2];
+      uint32_t wv[EV * ES / 4];
 #pragma unroll
-      for (int j = 0; j < EV; j += 2)
-        wv[j / 2] = Ops::pack2(l_tot > 0.f ? this->acc[0][j][i] * inv : 0.f,
-                               l_tot > 0.f ? this->acc[0][j + 1][i] * inv : 0.f);
-      store_words<EV / 2>(row + 2 * EV * (4 * this->q4 + i), wv);
+      for (int j = 0; j < EV; j += 4 / ES) {
+        const float x = l_tot > 0.f ? this->acc[0][j][i] * inv : 0.f;
+        if constexpr (kF32)
+          wv[j] = __float_as_uint(x);
+        else
+          wv[j / 2] = Ops::pack2(x, l_tot > 0.f ? this->acc[0][j + 1][i] * inv : 0.f);
+      }
+      store_words<EV * ES / 4>(row + ES * EV * (4 * this->q4 + i), wv);
     }
   }
 
@@ -1339,7 +1363,7 @@ struct GenWave : MfmaWave<VD, DT, PF, 1> {
             l_tot);
   }
   __device__ void stage_direct(const DecodeParams&, char* area, int, float l_tot) {
-    if (this->r16 < this->hcount) put_row(area + this->r16 * dm * 2, l_tot);
+    if (this->r16 < this->hcount) put_row(area + this->r16 * dm * ES, l_tot);
   }
   __device__ void store_partial(const DecodeParams&, int, float* w, int64_t head_stride, float l_tot) {
     if (this->r16 < this->hcount) put_partial(w + this->r16 * head_stride, l_tot);
@@ -1767,8 +1791,9 @@ __global__ __launch_bounds__((64 * sk_max_waves<D, 1, 0, PF, DT>())) void decode
   const int wid = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
   const int dm = kGen ? p.D : D;
   using Wave = std::conditional_t<
-      DT == QD_DTYPE_F32, MfmaWaveF32<D, PF>,
-      std::conditional_t<kGen, GenWave<D, kGen ? KCG : 1, DT, PF>, MfmaWave<D, DT, PF, 1>>>;
+      kGen, GenWave<D, kGen ? KCG : 1, DT, PF>,
+      std::conditional_t<DT == QD_DTYPE_F32, MfmaWaveF32<(DT == QD_DTYPE_F32 && !kGen) ? D : 64, PF>,
+                         MfmaWave<D, DT, PF, 1>>>;
   Wave wv;
   char* tile = wg_lds + wid * kTile;
   if constexpr (kGen)
@@ -2022,7 +2047,7 @@ __global__ __launch_bounds__((64 * sk_max_waves<D, NKV, GV, PF, DT>())) void dec
   const int kv_slices = FUSED ? 1 : p.kv_slices;
   static_assert(DT != QD_DTYPE_F32 || (NKV == 1 && GV == 0 && !FUSED), "fp32 caches: one kv-head per wave, merge kernel");
   constexpr bool kGen = KCG > 0;
-  static_assert(!kGen || (NKV == 1 && GV == 0 && !FUSED && DT != QD_DTYPE_F32), "general layout: one kv-head per wave");
+  static_assert(!kGen || (NKV == 1 && GV == 0 && !FUSED), "general layout: one kv-head per wave");
   constexpr int kTileBytes = kGen ? 16 * (64 * KCG + 32) : KTile<D, DT == QD_DTYPE_F32 ? 4 : 2>::kBytes;
   __shared__ __align__(16) char ktile[sk_max_waves<D, NKV, GV, PF, DT>()][kTileBytes];
   const int dm = kGen ? p.D : D;  // head_dim in memory
@@ -2140,8 +2165,9 @@ __global__ __launch_bounds__((64 * sk_max_waves<D, NKV, GV, PF, DT>())) void dec
   // GV > 0: the VALU comparison variant (ValuWave, GV heads per group).
   using Wave = std::conditional_t<
       GV == 0,
-      std::conditional_t<DT == QD_DTYPE_F32, MfmaWaveF32<D, PF>,
-                         std::conditional_t<kGen, GenWave<D, kGen ? KCG : 1, DT, PF>, MfmaWave<D, DT, PF, NKV>>>,
+      std::conditional_t<kGen, GenWave<D, kGen ? KCG : 1, DT, PF>,
+                         std::conditional_t<DT == QD_DTYPE_F32, MfmaWaveF32<(DT == QD_DTYPE_F32 && !kGen) ? D : 64, PF>,
+                                            MfmaWave<D, DT, PF, NKV>>>,
       ValuWave<D, DT, PF, (GV > 0 ? GV : 4)>>;
   Wave wv;
   if constexpr (kGen) {
@@ -2543,11 +2569,6 @@ bool f32_mfma_applies(int q_heads, int kv_heads, int head_dim, int block_size, i
 // B40 U[300, 1000] 25.4 -> 16.8; B4/L1024 16.5 -> 16.4, B1/L1024 11.9 -> 14.1).
 constexpr int64_t kF32GeneralTokens = 16384;
 
-bool f32_general_applies(int batch, int q_heads, int kv_heads, int head_dim, int block_size, int max_pages, int dtype) {
-  return f32_mfma_applies(q_heads, kv_heads, head_dim, block_size, dtype) &&
-         static_cast<int64_t>(batch) * max_pages * block_size >= kF32GeneralTokens;
-}
-
 bool f32_sk_applies(int batch, int q_heads, int kv_heads, int head_dim, int block_size, int max_pages, int dtype) {
   return f32_mfma_applies(q_heads, kv_heads, head_dim, block_size, dtype) &&
          static_cast<int64_t>(batch) * max_pages * block_size >= kF32SkTokens;
@@ -2615,9 +2636,11 @@ using KernelFn = void (*)(DecodeParams);
 // layout's VALU kernel (us per call, bf16/fp16): B64 Hq32/Hkv8 D72 P16 196.1 ->
 // 26.8, B16 D160 P32 327.3 -> 45.4, B16 D256 P8 136.0 -> 55.6, B16 D128 P1
 // U[1000, 6000] 89.7 -> 47.0, B64 Hq8/Hkv2 D32 28.9 -> 15.5, B1 Hq8/Hkv1 D16
-// 11.3 -> 9.4.
+// 11.3 -> 9.4; fp32, from kF32GeneralTokens of capacity: Hq32/Hkv4 D72
+// B3/L14328 91.5 -> 36.1, Hq16/Hkv2 D192 B30 107.5 -> 36.8, Hq32/Hkv8 D256 B16
+// 90.0 -> 70.2 (two rows of registers spill there).
 bool general_applies(int head_dim, int dtype) {
-  return (dtype == QD_DTYPE_F16 || dtype == QD_DTYPE_BF16) &&
+  return (dtype == QD_DTYPE_F16 || dtype == QD_DTYPE_BF16 || dtype == QD_DTYPE_F32) &&
          (head_dim <= 128 ? head_dim % 8 == 0 : head_dim % 16 == 0 && head_dim <= 256);
 }
 
@@ -2635,7 +2658,17 @@ KernelFn pick_general_sk(int head_dim) {
   return decode_mfma_sk_kernel<256, DT, 2, 1, 0, false, false, 8>;
 }
 
+// fp32: rows are stored after each item (one wave per SIMD above head_dim 64).
+KernelFn pick_general_sk_f32(int head_dim) {
+  if (head_dim <= 64) return decode_mfma_sk_kernel<64, QD_DTYPE_F32, 2, 1, 0, false, false, 4>;
+  if (head_dim <= 96) return decode_mfma_sk_kernel<128, QD_DTYPE_F32, 2, 1, 0, false, false, 6>;
+  if (head_dim <= 128) return decode_mfma_sk_kernel<128, QD_DTYPE_F32, 2, 1, 0, false, false, 8>;
+  if (head_dim <= 192) return decode_mfma_sk_kernel<256, QD_DTYPE_F32, 1, 1, 0, false, false, 12>;
+  return decode_mfma_sk_kernel<256, QD_DTYPE_F32, 1, 1, 0, false, false, 16>;
+}
+
 KernelFn pick_general_sk_dt(int dtype, int head_dim, bool hold) {
+  if (dtype == QD_DTYPE_F32) return pick_general_sk_f32(head_dim);
   if (dtype == QD_DTYPE_F16)
     return hold ? pick_general_sk<QD_DTYPE_F16, true>(head_dim) : pick_general_sk<QD_DTYPE_F16, false>(head_dim);
   return hold ? pick_general_sk<QD_DTYPE_BF16, true>(head_dim) : pick_general_sk<QD_DTYPE_BF16, false>(head_dim);
@@ -2651,6 +2684,8 @@ KernelFn pick_general_merge(int head_dim) {
 }
 
 KernelFn pick_general_merge_dt(int dtype, int head_dim, bool one_head) {
+  if (dtype == QD_DTYPE_F32)
+    return one_head ? pick_general_merge<QD_DTYPE_F32, 16, 4>(head_dim) : pick_general_merge<QD_DTYPE_F32, 8, 1>(head_dim);
   if (dtype == QD_DTYPE_F16)
     return one_head ? pick_general_merge<QD_DTYPE_F16, 16, 4>(head_dim) : pick_general_merge<QD_DTYPE_F16, 8, 1>(head_dim);
   return one_head ? pick_general_merge<QD_DTYPE_BF16, 16, 4>(head_dim) : pick_general_merge<QD_DTYPE_BF16, 8, 1>(head_dim);
@@ -2676,7 +2711,16 @@ KernelFn pick_wg_general(int D) {
   return decode_wg_kernel<256, DT, 2, 8>;
 }
 
+KernelFn pick_wg_general_f32(int D) {
+  if (D <= 64) return decode_wg_kernel<64, QD_DTYPE_F32, 2, 4>;
+  if (D <= 96) return decode_wg_kernel<128, QD_DTYPE_F32, 2, 6>;
+  if (D <= 128) return decode_wg_kernel<128, QD_DTYPE_F32, 2, 8>;
+  if (D <= 192) return decode_wg_kernel<256, QD_DTYPE_F32, 1, 12>;
+  return decode_wg_kernel<256, QD_DTYPE_F32, 1, 16>;
+}
+
 KernelFn pick_wg_dt(int dtype, int D, bool general) {
+  if (dtype == QD_DTYPE_F32 && general) return pick_wg_general_f32(D);
   if (dtype == QD_DTYPE_F32)
     return D == 64 ? decode_wg_kernel<64, QD_DTYPE_F32, kPrefetch> : decode_wg_kernel<128, QD_DTYPE_F32, kPrefetch>;
   if (dtype == QD_DTYPE_F16) return general ? pick_wg_general<QD_DTYPE_F16>(D) : pick_wg<QD_DTYPE_F16>(D);
@@ -2687,7 +2731,7 @@ KernelFn pick_wg_dt(int dtype, int D, bool general) {
 size_t wg_lds_bytes(int dtype, int D, bool general, int nw) {
   const int vd = general ? general_vd(D) : D;
   const int es = dtype == QD_DTYPE_F32 ? 4 : 2;
-  const int kc = D <= 64 ? 2 : D <= 96 ? 3 : D <= 128 ? 4 : D <= 192 ? 6 : 8;
+  const int kc = (D <= 64 ? 2 : D <= 96 ? 3 : D <= 128 ? 4 : D <= 192 ? 6 : 8) * (es / 2);
   const int tile = general ? 16 * (64 * kc + 32) + 2048 : 16 * (es * D + 32);
   return static_cast<size_t>(nw) * std::max(tile, wg_wave_merge_bytes(vd));
 }
@@ -3012,8 +3056,9 @@ constexpr int64_t kFusedMaxTrips = 2;
 // issue slots, and a CU its load path: 8 waves were level with 4 or slower
 // except on long runs of head_dim 64), no more than there are groups.  Many
 // workgroups of few groups run single waves (bf16 Hq32/Hkv8 D128 B256/L64 19.5
-// us against 22.2 with 4 waves), fp32 head_dim 128 ones two (B64/L512 48.9
-// against 53.2), and head_dim 256 splits stay single waves unless they are
+// us against 22.2 with 4 waves), fp32 ones above head_dim 64 two (D128 B64/L512
+// 48.9 against 53.2) or, from 1024 workgroups, one (D96 B64 8 splits 23.1 against
+// 28.9), and head_dim 256 splits stay single waves unless they are
 // too few for the CUs (B8, 8 splits: 42.4 against 45.6).  With caller-given
 // splits, us per call with 1 -> 4 waves (graph replays): B4 U[2048, 4096] 4
 // splits 43.0 -> 20.5, 16 splits 18.7 -> 18.2; B1/L16000 16 splits 44.5 -> 21.6;
@@ -3022,7 +3067,7 @@ int wg_waves_for(int64_t wgs, int64_t groups, int dtype, int head_dim) {
   if (wgs > 1024 && groups <= 8) return 1;
   int cap = 4;
   if (dtype == QD_DTYPE_F32) {
-    if (head_dim > 64 && wgs >= 512) cap = 2;
+    if (head_dim > 64 && wgs >= 512) cap = wgs >= 1024 ? 1 : 2;
   } else if (head_dim <= 64) {
     if (groups >= 64) cap = 8;
   } else if (head_dim > 128 && wgs >= 256) {
@@ -3053,6 +3098,7 @@ bool wg_single_applies(int64_t wgs, int64_t groups, int dtype, int head_dim, boo
   int64_t most = 32, work = 32768;
   if (dtype == QD_DTYPE_F32) {
     most = wgs >= 512 ? 64 : wgs >= 128 ? (head_dim <= 64 ? 64 : 16) : (head_dim <= 64 ? 16 : 8);
+    if (general) most = std::min<int64_t>(most, 32);
   } else if (head_dim > 128) {
     most = 16;
   } else if (general) {
@@ -3089,6 +3135,8 @@ struct AutoPlan {
   int kv_split;     // stream-K: virtual kv-heads per kv-head (DecodeParams::kv_split)
   bool general;     // stream-K: the general layout (general_applies)
   int kv_slices;    // stream-K: workgroups per range (DecodeParams::kv_slices)
+  bool gen_wave;    // with general: GenWave (else MfmaWaveF32)
+  bool single_gen;  // with wg_single: GenWave
   int wg_single;    // whole call in one launch of decode_wg_kernel: waves per workgroup, else 0
 };
 
@@ -3140,7 +3188,7 @@ bool fused_applies(int batch, int q_heads, int kv_heads, int head_dim, int nkv, 
 // whether q/k/v/out are 16-byte aligned (the MFMA kernels' vector loads).
 int auto_plan(int batch, int q_heads, int kv_heads, int head_dim, int block_size, int max_pages,
               int dtype, bool aligned, AutoPlan* ap, bool valu = false, bool allow_general = true) {
-  *ap = AutoPlan{false, 0, 1, 1, false, false, 0, 0, 1, 0, kCounterBytes, 0, 1, false, 1, 0};
+  *ap = AutoPlan{false, 0, 1, 1, false, false, 0, 0, 1, 0, kCounterBytes, 0, 1, false, 1, false, false, 0};
   if (batch <= 0) return QD_OK;
   const int split = kv_split_for(q_heads, kv_heads);
   const int vkv = kv_heads * (split > 0 ? split : 1);  // kv-heads as the stream-K kernel serves them
@@ -3152,17 +3200,23 @@ int auto_plan(int batch, int q_heads, int kv_heads, int head_dim, int block_size
   const int64_t gmax = static_cast<int64_t>(batch) * groups;
   const bool general =
       !exact && !valu && allow_general &&
-      (f32 ? f32_general_applies(batch, q_heads, kv_heads, head_dim, block_size, max_pages, dtype)
-           : general_applies(head_dim, dtype));
-  if (aligned && split > 0 && !valu && (exact || general || f32_mfma_applies(q_heads, kv_heads, head_dim, block_size, dtype)))
-    ap->wg_single = vkv <= 65535 && wg_single_applies(static_cast<int64_t>(batch) * vkv, groups, dtype, head_dim, general && !f32)
+      general_applies(head_dim, dtype) &&
+      (!f32 || static_cast<int64_t>(batch) * max_pages * block_size >= kF32GeneralTokens);
+  // (fp32 head_dim 64 and 128 on whole-group pages keep MfmaWaveF32.)
+  const bool gen_wave = general && !f32_mfma_applies(q_heads, kv_heads, head_dim, block_size, dtype);
+  const bool f32_wave = f32_mfma_applies(q_heads, kv_heads, head_dim, block_size, dtype);
+  const bool single_gen = !exact && !f32_wave && allow_general && general_applies(head_dim, dtype);
+  if (aligned && split > 0 && !valu && (exact || f32_wave || single_gen)) {
+    ap->wg_single = vkv <= 65535 && wg_single_applies(static_cast<int64_t>(batch) * vkv, groups, dtype, head_dim, single_gen)
                         ? wg_waves_for(static_cast<int64_t>(batch) * vkv, groups, dtype, head_dim)
                         : 0;
+    ap->single_gen = single_gen;
+  }
   if (aligned && split > 0 && (split == 1 || !valu) && (exact || general) && batch <= kSkMaxBatch) {
     int nkv = 1;
     const bool wide = !valu && !f32 && !general && sk_wide_applies(vkv, head_dim);
     auto pick = [&](bool hold) {
-      return general && !f32 ? pick_general_sk_dt(dtype, head_dim, hold)
+      return gen_wave ? pick_general_sk_dt(dtype, head_dim, hold)
                      : pick_mfma_sk_dt(dtype, head_dim, nkv, wide && nkv == 1, false, hold);
     };
     // fp32 at head_dim 128 holds 64 KB of K/V per group in flight: one wave
@@ -3209,7 +3263,7 @@ int auto_plan(int batch, int q_heads, int kv_heads, int head_dim, int block_size
     // U[500, 1500] Hkv8 D256 179.4 held, 165.8 us stored; fp32 D128 199.7 and
     // 171.6; Qwen2.5-7B's shape at B128/L1024 51.5 and 47.2), while with two
     // kv-heads per wave (Gemma-2-9B's shape) holding was level.
-    const bool one_per_simd = nkv == 1 && (wide || head_dim > 128 || (f32 && head_dim > 64));
+    const bool one_per_simd = nkv == 1 && (wide || head_dim > 128 || (f32 && (head_dim > 64 || gen_wave)));
     if (!valu && !one_per_simd && hold_results(batch, w)) {
       const KernelFn hfn = pick(true);
       ap->stage_bytes = stage_lds_bytes(g, head_dim, nkv, nw);
@@ -3227,6 +3281,7 @@ int auto_plan(int batch, int q_heads, int kv_heads, int head_dim, int block_size
     }
     ap->stream_k = true;
     ap->general = general;
+    ap->gen_wave = gen_wave;
     ap->kv_split = split;
     ap->wgs = static_cast<int>(w);
     ap->wg_waves = nw;
@@ -3528,6 +3583,13 @@ int qd_gqa_decode_kernel_kind(int q_heads, int kv_heads, int head_dim, int block
   return mfma_applies(q_heads, kv_heads, head_dim, block_size, dtype) ? 1 : 0;
 }
 
+// fp32 above head_dim 96 holds one wave per SIMD (the VALU kernel three), so
+// many short splits are left to the VALU kernel (us per call, VALU -> MFMA;
+// Hkv8 D128: 512 splits in all, B4 U[2000, 4096] 40.7 -> 29.4, B32 U[100, 1000]
+// 72.0 -> 41.5; 1008, B2 U[1000, 3000] 17.1 -> 24.1; D256: 157, B1/L5000 35.9 ->
+// 22.6; 1032, B3 31.4 -> 40.7).
+static constexpr int64_t kF32WideSplits = 512;
+
 int qd_gqa_decode_launch(const void* q, const void* k_cache, const void* v_cache,
                          const int32_t* block_table, const int32_t* context_lens, void* out,
                          float* workspace, size_t workspace_bytes, int batch, int q_heads,
@@ -3566,6 +3628,8 @@ int qd_gqa_decode_launch(const void* q, const void* k_cache, const void* v_cache
   const int split_kv = kv_split_for(q_heads, kv_heads);
   const bool general = !use_mfma && (flags & QD_FLAG_FORCE_GENERIC) == 0 && general_applies(head_dim, dtype) &&
                        split_kv > 0 && static_cast<int64_t>(kv_heads) * split_kv <= 65535 &&
+                       (dtype != QD_DTYPE_F32 || head_dim <= 96 ||
+                        static_cast<int64_t>(splits) * kv_heads * split_kv * batch <= kF32WideSplits) &&
                        num_blocks * block_size <= 2147483647LL && aligned16(q) && aligned16(k_cache) &&
                        aligned16(v_cache) && aligned16(out) &&
                        (splits <= 1 || (reinterpret_cast<uintptr_t>(workspace) & 7u) == 0);
@@ -3671,12 +3735,12 @@ int qd_gqa_decode_auto_stages(const void* q, const void* k_cache, const void* v_
     prm.wg_waves = ap.wg_single;
     prm.splits = 1;
     if (stages & QD_STAGE_DECODE) {
-      st = launch_wg(prm, dtype, head_dim, ap.general, 1, prm.Hkv, batch, stm);
+      st = launch_wg(prm, dtype, head_dim, ap.single_gen, 1, prm.Hkv, batch, stm);
       if (st != QD_OK) return st;
     }
     return launch_error();
   }
-  if (ap.general && dtype != QD_DTYPE_F32) {
+  if (ap.gen_wave) {
     hipLaunchKernelGGL(pick_general_sk_dt(dtype, head_dim, ap.stage_bytes > 0), dim3(ap.wgs, ap.kv_slices), dim3(64 * ap.wg_waves),
                        ap.stage_bytes, stm, prm);
     const bool one_head = merge_one_head_per_wave(batch, q_heads);

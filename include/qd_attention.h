@@ -138,9 +138,9 @@ int qd_gqa_decode_launch(const void* q, const void* k_cache, const void* v_cache
 /* Which kernel qd_gqa_decode_launch would run for these shapes:
  * 1 = the MFMA kernel for head_dim 64/96/128/256, whole 16-token groups per
  * page and groups of at most 16 q-heads, 0 = the others: the general MFMA
- * layout (16-bit, head_dim a multiple of 8 up to 128 or of 16 up to 256,
- * groups up to 128, not with QD_FLAG_FORCE_GENERIC) or the portable VALU
- * kernel. */
+ * layout (head_dim a multiple of 8 up to 128 or of 16 up to 256, groups up to
+ * 128, not with QD_FLAG_FORCE_GENERIC; fp32 above head_dim 96 only for at most
+ * 512 workgroups) or the portable VALU kernel. */
 int qd_gqa_decode_kernel_kind(int q_heads, int kv_heads, int head_dim, int block_size,
                               int dtype, int flags);
 
@@ -162,10 +162,11 @@ int qd_gqa_decode_kernel_kind(int q_heads, int kv_heads, int head_dim, int block
  *     workgroup to finish a piece of it (the fused merge, when the merge is
  *     short: see qd_gqa_decode_auto_info) or by a second kernel on the same
  *     stream;
- *   - 16-bit caches with any other block_size, or a head_dim that is another
- *     multiple of 8 up to 128 or of 16 up to 256 (same groups and batch,
- *     num_blocks * block_size < 2^31): the same partition with the general
- *     kernel, merged by a second kernel.  It serves whole calls only and is
+ *   - caches with any other block_size, or a head_dim that is another multiple
+ *     of 8 up to 128 or of 16 up to 256 (same groups and batch, num_blocks *
+ *     block_size < 2^31), and in fp32 any of these from 16384 tokens of
+ *     capacity: the same partition with the general kernel (fp32 head_dim
+ *     64/128 with its own), merged by a second kernel.  It serves whole calls only and is
  *     reported as kind 0 by qd_gqa_decode_auto_info; with a workspace that
  *     holds only the split layout's partials the split layout runs instead;
  *   - short contexts (wg_single_applies in gqa_decode.hip: by max_pages *

@@ -1227,3 +1227,55 @@ def test_general_layout_explicit_splits(gpu, shape):
             assert rc == 0, cabi.error_string(rc)
             torch.cuda.synchronize()
             assert_close(out, ref, DT_NAME[dtype], rows, f"splits={splits} chunk={chunk} flags={flags}")
+
+
+# (Hq, Hkv, D, P, lengths): fp32 on the general layout, as splits, in one launch and
+# balanced (16384 tokens of capacity).
+GENERAL_F32_SHAPES = [
+    (32, 8, 80, 16, [17, 1000, 0, 33]),
+    (8, 2, 64, 1, [1, 600, 513, 16]),
+    (28, 4, 128, 3, [1537, 5, 700]),
+    (6, 3, 72, 12, [100, 1, 0, 999]),
+    (48, 1, 96, 8, [129, 700]),                       # 3 x 16 q-heads
+    (8, 4, 160, 16, [65, 900, 2]),
+    (16, 2, 192, 7, [6, 7, 8, 300]),
+    (4, 2, 256, 16, [1, 250, 33]),
+    (8, 1, 40, 16, [300, 31]),
+    (8, 8, 80, 16, [4500, 1, 0, 900]),                # balanced
+    (8, 2, 64, 8, [3000] + _fused_lengths(69, 1, 500, 146)),
+    (16, 4, 128, 20, [6000, 17, 2999]),
+]
+
+
+@pytest.mark.parametrize("shape", GENERAL_F32_SHAPES, ids=lambda s: f"Hq{s[0]}-Hkv{s[1]}-D{s[2]}-P{s[3]}-B{len(s[4])}")
+def test_general_layout_f32(gpu, shape):
+    """fp32 caches on the general layout at the fp32 bar: the automatic path
+    on a NaN-filled workspace and with the rest of the pool poisoned, and
+    caller-given splits."""
+    hq, hkv, d, p, lengths = shape
+    say(f"general fp32 Hq{hq} Hkv{hkv} D{d} P{p} B{len(lengths)}")
+    q, k, v, table, lens = to_dev(make_decode_case(lengths=lengths, q_heads=hq, kv_heads=hkv, head_dim=d, block_size=p,
+                                                   dtype=torch.float32, seed=147), gpu)
+    ref, rows = oracle_rows((q, k, v, table, lens))
+    used = torch.zeros(k.shape[0], dtype=torch.bool)
+    for b, n in enumerate(lengths):
+        used[table[b, :-(-n // p)].long().cpu()] = True
+        if n % p:
+            k[int(table[b, n // p]), n % p:] = float("nan")
+            v[int(table[b, n // p]), n % p:] = float("inf")
+    k[~used.to(gpu)] = float("inf")
+    v[~used.to(gpu)] = float("nan")
+    ws = cabi.auto_workspace(len(lengths), hq, hkv, d, p, table.shape[1], cabi.DTYPE[q.dtype], gpu, fill=0xFF)
+    out = torch.full_like(q, float("nan"))
+    rc = cabi.auto_launch(q, k, v, table, lens, out, scale=1 / math.sqrt(d), workspace=ws)
+    assert rc == 0, cabi.error_string(rc)
+    torch.cuda.synchronize()
+    assert_close(out, ref, "f32", rows, "general fp32")
+    for splits in (1, 3):
+        parts = torch.full((max(1, q.shape[0] * hq * splits * (d + 2)),), float("nan"), device=gpu)
+        out = torch.full_like(q, float("nan"))
+        rc = cabi.launch(q, k, v, table, lens, out, scale=1 / math.sqrt(d), splits=splits, chunk_pages=0,
+                         workspace=parts if splits > 1 else None, flags=0)
+        assert rc == 0, cabi.error_string(rc)
+        torch.cuda.synchronize()
+        assert_close(out, ref, "f32", rows, f"general fp32 splits={splits}")
