@@ -69,17 +69,26 @@ struct LatentWriteParams {
 // grid n, block 64: row t -> cache row slots[t] (skipped when out of range).
 __global__ __launch_bounds__(64) void latent_write_vec16_kernel(LatentWriteParams p) {
   const int64_t t = blockIdx.x;
-  const int64_t s = p.slots[t];
-  if (s < 0 || s >= p.rows) return;
-  char* dst = p.cache + s * p.row_bytes;
   const char* la = p.latent + t * p.lat_bytes;
   const char* ro = p.rope + t * p.rope_bytes;
   const int64_t nl = p.lat_bytes >> 4, nr = p.rope_bytes >> 4;
-  for (int64_t i = threadIdx.x; i < nl + nr; i += 64) {
-    const u32x4 v = i < nl ? *reinterpret_cast<const u32x4*>(la + 16 * i)
-                           : *reinterpret_cast<const u32x4*>(ro + 16 * (i - nl));
-    *reinterpret_cast<u32x4*>(dst + 16 * i) = v;
-  }
+  auto piece = [&](int64_t i) {
+    return i < nl ? *reinterpret_cast<const u32x4*>(la + 16 * i) : *reinterpret_cast<const u32x4*>(ro + 16 * (i - nl));
+  };
+  // The first 2 KB are loaded with the slot that says where they go (96 rows:
+  // 4.8 -> 3.9 us in the trace; the same order in kv_append changed nothing).
+  constexpr int kAhead = 2;
+  u32x4 ahead[kAhead];
+#pragma unroll
+  for (int j = 0; j < kAhead; ++j)
+    if (threadIdx.x + 64 * j < nl + nr) ahead[j] = piece(threadIdx.x + 64 * j);
+  const int64_t s = p.slots[t];
+  if (s < 0 || s >= p.rows) return;
+  char* dst = p.cache + s * p.row_bytes;
+#pragma unroll
+  for (int j = 0; j < kAhead; ++j)
+    if (threadIdx.x + 64 * j < nl + nr) *reinterpret_cast<u32x4*>(dst + 16 * (threadIdx.x + 64 * j)) = ahead[j];
+  for (int64_t i = threadIdx.x + 64 * kAhead; i < nl + nr; i += 64) *reinterpret_cast<u32x4*>(dst + 16 * i) = piece(i);
 }
 
 template <typename E>
