@@ -3200,9 +3200,9 @@ DecodeLayout decode_layout(const AttendShape& a, const AttendPlan& pl) {
   return d;
 }
 
-// A pool of 2^31 rows or more (32-bit row lists do not reach it; its plans
-// need less workspace than the ones sized without num_blocks) keeps the
-// kernels before the shared-tile one for gathered rows.
+// A pool of 2^31 rows or more, which 32-bit row lists do not reach, keeps the
+// staged kernel (its 2.4 TB would not fit the card: the guard only keeps an
+// inconsistent num_blocks from wrapping).
 int gather_flags(int64_t num_blocks, int block_size, int flags) {
   return num_blocks * block_size > 2147483647LL ? flags | kNoGather : flags;
 }

@@ -1092,7 +1092,7 @@ def main() -> None:
     if args.kernel == "auto" and args.splits == 0 and auto_kind == 1:
         kname, kernels = "decode_mfma_sk_kernel", "decode_mfma_sk_kernel+merge_sk_kernel"
     else:
-        kname = "decode_mfma_kernel" if kind == 1 else "decode_generic_kernel"
+        kname = "decode_wg_kernel" if kind == 1 else "decode_generic_kernel"
         kernels = kname + ("+combine_kernel" if splits > 1 else "")
     log(f"path: {path}; kernels {kernels}; waves={auto_waves} splits={splits} chunk_pages={chunk}; "
         f"warmup {args.warmup}, {SAMPLES} samples of {args.steps} steps")

@@ -370,9 +370,11 @@ size_t qd_mla_attend_workspace_bytes(int batch, int q_len, int heads, int latent
                                      int flags);
 
 /* The plan qd_mla_attend would use: returns 3 for the shared-tile MFMA
- * kernel (dense rows, latent 512, rope 64, 32-token pages, 64 heads or more),
- * 2 for the wave-streamed MFMA kernel (dense rows, latent 512, rope 64,
- * 16-token pages, other head counts), 1 for the
+ * kernel (latent 512, rope 64: 64 heads or more on listed tokens, on pages of
+ * a multiple of 32 tokens or of no multiple of 16, or q_len * heads >= 32 with
+ * q_len > 1 on dense pages of a multiple of 32 tokens), 2 for the
+ * wave-streamed MFMA kernel (latent 512, rope 64, the other dense rows on
+ * pages of a multiple of 16 tokens), 1 for the
  * workgroup-staged MFMA kernel (*out_splits = stream-K workgroups per head
  * group, *head_groups = head groups for both), 0 for the VALU kernel
  * (*out_splits = context splits per row, *head_groups = 0), -1 for invalid
