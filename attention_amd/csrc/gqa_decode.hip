@@ -2567,6 +2567,9 @@ bool f32_mfma_applies(int q_heads, int kv_heads, int head_dim, int block_size, i
 // capacity on (Hq32/Hkv8 D128, us per call, split layout -> balanced: B16
 // U[64, 1024] 24.5 -> 20.4, B16/L1024 33.8 -> 32.4, B4/L4096 33.9 -> 32.2, Hkv1
 // B40 U[300, 1000] 25.4 -> 16.8; B4/L1024 16.5 -> 16.4, B1/L1024 11.9 -> 14.1).
+// Those read fresh inputs; repeated over one 134 MB input that the Infinity
+// Cache holds, the split layout keeps 29.6 against 32 us at B4/L4096 and
+// B16/L1024.
 constexpr int64_t kF32GeneralTokens = 16384;
 
 bool f32_sk_applies(int batch, int q_heads, int kv_heads, int head_dim, int block_size, int max_pages, int dtype) {
