@@ -3115,6 +3115,8 @@ bool wg_single_applies(int64_t wgs, int64_t groups, int dtype, int head_dim, boo
 // Enqueues decode_wg_kernel with prm.wg_waves waves per workgroup.
 int launch_wg(const DecodeParams& prm, int dtype, int head_dim, bool general, int splits, int kv_heads, int batch,
               hipStream_t st) {
+  // A wave's lanes hold kMfmaHeads q-heads; larger groups come in chunks (use_kv_chunks).
+  if (prm.g > kMfmaHeads) return fail(QD_ERR_INVALID_VALUE, "more than 16 q-heads per (virtual) kv-head");
   const KernelFn fn = pick_wg_dt(dtype, head_dim, general);
   if (!allow_dyn_lds(fn)) return fail(QD_ERR_INVALID_VALUE, "dynamic LDS limit not raised");
   hipLaunchKernelGGL(fn, dim3(splits, kv_heads, batch), dim3(64 * prm.wg_waves),
@@ -3135,7 +3137,7 @@ struct AutoPlan {
   int chunk_pages;
   size_t ws_bytes;  // scratch bytes (kCounterBytes of counters first)
   size_t meta_offset;  // stream-K: byte offset of the meta table in the scratch
-  int kv_split;     // stream-K: virtual kv-heads per kv-head (DecodeParams::kv_split)
+  int kv_split;     // stream-K and one launch: virtual kv-heads per kv-head (DecodeParams::kv_split)
   bool general;     // stream-K: the general layout (general_applies)
   int kv_slices;    // stream-K: workgroups per range (DecodeParams::kv_slices)
   bool gen_wave;    // with general: GenWave (else MfmaWaveF32)
@@ -3214,6 +3216,7 @@ int auto_plan(int batch, int q_heads, int kv_heads, int head_dim, int block_size
                         ? wg_waves_for(static_cast<int64_t>(batch) * vkv, groups, dtype, head_dim)
                         : 0;
     ap->single_gen = single_gen;
+    ap->kv_split = split;  // also where no balanced plan follows
   }
   if (aligned && split > 0 && (split == 1 || !valu) && (exact || general) && batch <= kSkMaxBatch) {
     int nkv = 1;

@@ -1167,6 +1167,17 @@ ONE_LAUNCH_SHAPES = [
     (torch.float32, 16, 4, 64, 32, [1, 33, 200, 256]),
     (torch.float32, 8, 8, 128, 16, _fused_lengths(70, 1, 512, 152)),          # 2 waves
     (torch.bfloat16, 32, 8, 128, 16, _fused_lengths(300, 0, 64, 153)),        # single waves
+    # More than 16 q-heads per kv-head where no balanced plan exists: fp32
+    # below 16384 tokens of capacity, and batches above 4096.
+    (torch.float32, 32, 1, 128, 16, [1, 17, 0, 128]),                         # 2 x 16 q-heads
+    (torch.float32, 17, 1, 128, 16, [100, 16]),                               # 9 + 8
+    (torch.float32, 71, 1, 64, 16, [1, 130, 256]),                            # 4 x 15 + 11
+    (torch.float32, 256, 2, 80, 16, [1, 33, 120]),                            # 8 x 16, the largest group
+    (torch.float32, 64, 2, 256, 16, [1, 17, 128]),
+    (torch.float32, 48, 1, 40, 5, [4, 5, 6, 100]),
+    (torch.bfloat16, 32, 1, 64, 16, _fused_lengths(4097, 0, 32, 155)),
+    (torch.float16, 40, 1, 80, 8, _fused_lengths(4097, 0, 8, 156)),
+    (torch.float32, 20, 1, 64, 16, _fused_lengths(4097, 0, 32, 157)),
 ]
 
 
