@@ -103,6 +103,9 @@ def lib():
         L.qd_gqa_decode_auto_counter_bytes.restype = ctypes.c_size_t
         L.qd_gqa_decode_auto_counter_bytes.argtypes = []
         L.qd_gqa_decode_auto_info.argtypes = [ctypes.c_int] * 7 + [ctypes.POINTER(ctypes.c_int)] * 3
+        L.qd_gqa_decode_auto_path.restype = ctypes.c_int
+        L.qd_gqa_decode_auto_path.argtypes = ([ctypes.c_int] * 6 + [ctypes.c_int64, ctypes.c_int]
+                                              + [ctypes.POINTER(ctypes.c_int)] * 4)
         V, I, I64, F = ctypes.c_void_p, ctypes.c_int, ctypes.c_int64, ctypes.c_float
         MSG = [ctypes.c_char_p, ctypes.c_size_t]
         L.qd_latent_kv_write_validate.restype = I
@@ -202,6 +205,21 @@ def auto_info(batch, q_heads, kv_heads, head_dim, block_size, max_pages, dtype=2
     kind = lib().qd_gqa_decode_auto_info(batch, q_heads, kv_heads, head_dim, block_size, max_pages,
                                          dtype, ctypes.byref(w), ctypes.byref(s), ctypes.byref(c))
     return kind, w.value, s.value, c.value
+
+
+QD_PATHS = ("split", "balanced", "fused", "one launch")
+QD_LAYOUTS = ("valu", "exact", "general")
+
+
+def auto_path(batch, q_heads, kv_heads, head_dim, block_size, max_pages, num_blocks, dtype=2):
+    """What a whole call runs: (path of QD_PATHS, layout of QD_LAYOUTS, q-head
+    chunks per kv-head, workgroups, waves per workgroup), or None for invalid
+    shapes."""
+    layout, chunks, wgs, waves = (ctypes.c_int() for _ in range(4))
+    path = lib().qd_gqa_decode_auto_path(batch, q_heads, kv_heads, head_dim, block_size, max_pages, num_blocks, dtype,
+                                         ctypes.byref(layout), ctypes.byref(chunks), ctypes.byref(wgs),
+                                         ctypes.byref(waves))
+    return None if path < 0 else (QD_PATHS[path], QD_LAYOUTS[layout.value], chunks.value, wgs.value, waves.value)
 
 
 def auto_launch(q, k, v, table, lens, out, *, scale, workspace=None, stream=None, stages=QD_STAGE_ALL):

@@ -2647,6 +2647,10 @@ bool general_applies(int head_dim, int dtype) {
          (head_dim <= 128 ? head_dim % 8 == 0 : head_dim % 16 == 0 && head_dim <= 256);
 }
 
+// Whether the general layout's 32-bit pool rows (GenWave::issue) reach every
+// token slot of the pool.
+bool pool_rows_fit(int64_t num_blocks, int block_size) { return num_blocks <= 2147483647LL / block_size; }
+
 // V layout (64, 128 or 256 columns) and 32-wide QK chunks of the general
 // kernel serving a head_dim.
 int general_vd(int head_dim) { return head_dim <= 64 ? 64 : head_dim <= 128 ? 128 : 256; }
@@ -3319,6 +3323,42 @@ int auto_plan(int batch, int q_heads, int kv_heads, int head_dim, int block_size
   return QD_OK;
 }
 
+// fp32 above head_dim 96 holds one wave per SIMD (the VALU kernel three), so
+// many short splits are left to the VALU kernel (us per call, VALU -> MFMA;
+// Hkv8 D128: 512 splits in all, B4 U[2000, 4096] 40.7 -> 29.4, B32 U[100, 1000]
+// 72.0 -> 41.5; 1008, B2 U[1000, 3000] 17.1 -> 24.1; D256: 157, B1/L5000 35.9 ->
+// 22.6; 1032, B3 31.4 -> 40.7).
+constexpr int64_t kF32WideSplits = 512;
+
+// Kernel of the explicit split layout: the exact MFMA layout, the general one
+// where that does not apply (groups above kMfmaHeads in chunks as on the
+// balanced path), else the VALU kernel.
+enum class SplitKernel { kValu, kExact, kGeneral };
+
+SplitKernel split_kernel(int batch, int q_heads, int kv_heads, int head_dim, int block_size, int64_t num_blocks,
+                         int dtype, int splits, int flags, bool aligned) {
+  if (!aligned || (flags & QD_FLAG_FORCE_GENERIC) != 0) return SplitKernel::kValu;
+  if (mfma_applies(q_heads, kv_heads, head_dim, block_size, dtype)) return SplitKernel::kExact;
+  const int64_t chunks = static_cast<int64_t>(kv_heads) * kv_split_for(q_heads, kv_heads);
+  const bool general = general_applies(head_dim, dtype) && chunks > 0 && chunks <= 65535 &&
+                       (dtype != QD_DTYPE_F32 || head_dim <= 96 ||
+                        static_cast<int64_t>(splits) * chunks * batch <= kF32WideSplits) &&
+                       pool_rows_fit(num_blocks, block_size);
+  return general ? SplitKernel::kGeneral : SplitKernel::kValu;
+}
+
+// Plan of a call through the automatic path.  The general layout takes whole
+// calls, 32-bit pool rows, and a workspace of its plan's size; the split
+// layout serves the rest.
+int plan_call(int batch, int q_heads, int kv_heads, int head_dim, int block_size, int max_pages, int64_t num_blocks,
+              int dtype, bool aligned, bool valu, int stages, size_t workspace_bytes, AutoPlan* ap) {
+  const int st = auto_plan(batch, q_heads, kv_heads, head_dim, block_size, max_pages, dtype, aligned, ap, valu);
+  if (st != QD_OK) return st;
+  if (ap->general && (stages != QD_STAGE_ALL || !pool_rows_fit(num_blocks, block_size) || workspace_bytes < ap->ws_bytes))
+    return auto_plan(batch, q_heads, kv_heads, head_dim, block_size, max_pages, dtype, aligned, ap, valu, false);
+  return QD_OK;
+}
+
 int check_launch_shapes(int batch, int q_heads, int kv_heads, int head_dim, int block_size,
                         int max_pages, int64_t num_blocks, int dtype, float scale) {
   if (batch < 0) return fail(QD_ERR_INVALID_VALUE, "batch must be >= 0");
@@ -3589,13 +3629,6 @@ int qd_gqa_decode_kernel_kind(int q_heads, int kv_heads, int head_dim, int block
   return mfma_applies(q_heads, kv_heads, head_dim, block_size, dtype) ? 1 : 0;
 }
 
-// fp32 above head_dim 96 holds one wave per SIMD (the VALU kernel three), so
-// many short splits are left to the VALU kernel (us per call, VALU -> MFMA;
-// Hkv8 D128: 512 splits in all, B4 U[2000, 4096] 40.7 -> 29.4, B32 U[100, 1000]
-// 72.0 -> 41.5; 1008, B2 U[1000, 3000] 17.1 -> 24.1; D256: 157, B1/L5000 35.9 ->
-// 22.6; 1032, B3 31.4 -> 40.7).
-static constexpr int64_t kF32WideSplits = 512;
-
 int qd_gqa_decode_launch(const void* q, const void* k_cache, const void* v_cache,
                          const int32_t* block_table, const int32_t* context_lens, void* out,
                          float* workspace, size_t workspace_bytes, int batch, int q_heads,
@@ -3622,25 +3655,17 @@ int qd_gqa_decode_launch(const void* q, const void* k_cache, const void* v_cache
                                  q_heads, kv_heads, head_dim, block_size, max_pages, num_blocks, scale,
                                  splits, chunk_pages);
   hipStream_t stm = static_cast<hipStream_t>(stream);
-  // The MFMA kernel's vector loads and stores need 16-byte aligned tensors
-  // and an 8-byte aligned workspace (its partials are stored in float pairs);
-  // the generic kernel stores single elements.
-  const bool use_mfma = qd_gqa_decode_kernel_kind(q_heads, kv_heads, head_dim, block_size, dtype, flags) &&
-                        aligned16(q) && aligned16(k_cache) && aligned16(v_cache) && aligned16(out) &&
-                        (splits <= 1 || (reinterpret_cast<uintptr_t>(workspace) & 7u) == 0);
-  // The general layout where the exact one does not apply, with groups above
-  // kMfmaHeads in chunks as on the balanced path (reported as kind 0 by
-  // qd_gqa_decode_kernel_kind, like the VALU kernel).
-  const int split_kv = kv_split_for(q_heads, kv_heads);
-  const bool general = !use_mfma && (flags & QD_FLAG_FORCE_GENERIC) == 0 && general_applies(head_dim, dtype) &&
-                       split_kv > 0 && static_cast<int64_t>(kv_heads) * split_kv <= 65535 &&
-                       (dtype != QD_DTYPE_F32 || head_dim <= 96 ||
-                        static_cast<int64_t>(splits) * kv_heads * split_kv * batch <= kF32WideSplits) &&
-                       num_blocks * block_size <= 2147483647LL && aligned16(q) && aligned16(k_cache) &&
-                       aligned16(v_cache) && aligned16(out) &&
+  // The MFMA kernels' vector loads and stores need 16-byte aligned tensors
+  // and an 8-byte aligned workspace (their partials are stored in float
+  // pairs); the VALU kernel stores single elements.
+  const bool aligned = aligned16(q) && aligned16(k_cache) && aligned16(v_cache) && aligned16(out) &&
                        (splits <= 1 || (reinterpret_cast<uintptr_t>(workspace) & 7u) == 0);
+  const SplitKernel kernel =
+      split_kernel(batch, q_heads, kv_heads, head_dim, block_size, num_blocks, dtype, splits, flags, aligned);
   (void)hipGetLastError();  // start from a clean error state
-  if (use_mfma || general) {
+  if (kernel != SplitKernel::kValu) {
+    const bool general = kernel == SplitKernel::kGeneral;
+    const int split_kv = kv_split_for(q_heads, kv_heads);
     const int cp = chunk_pages > 0 ? chunk_pages : (max_pages + splits - 1) / splits;
     if (general && split_kv > 1) use_kv_chunks(&prm, q_heads, kv_heads, split_kv);
     prm.wg_waves = wg_waves_for(static_cast<int64_t>(splits) * prm.Hkv * batch,
@@ -3694,14 +3719,9 @@ int qd_gqa_decode_auto_stages(const void* q, const void* k_cache, const void* v_
                 mfma_applies(q_heads, kv_heads, head_dim, block_size, dtype) && batch <= kSkMaxBatch))
     return fail(QD_ERR_INVALID_VALUE, "QD_STAGE_VALU needs the balanced path with head_dim 128 and group size <= 8");
   AutoPlan ap;
-  st = auto_plan(batch, q_heads, kv_heads, head_dim, block_size, max_pages, dtype, aligned, &ap, valu);
+  st = plan_call(batch, q_heads, kv_heads, head_dim, block_size, max_pages, num_blocks, dtype, aligned, valu, stages,
+                 workspace_bytes, &ap);
   if (st != QD_OK) return st;
-  // The general layout takes whole calls, 32-bit pool rows, and a workspace
-  // of its plan's size; the split layout serves the rest.
-  if (ap.general && (stages != QD_STAGE_ALL || num_blocks * block_size > 2147483647LL || workspace_bytes < ap.ws_bytes)) {
-    st = auto_plan(batch, q_heads, kv_heads, head_dim, block_size, max_pages, dtype, aligned, &ap, valu, false);
-    if (st != QD_OK) return st;
-  }
   if (!workspace || workspace_bytes < ap.ws_bytes || !aligned16(workspace))
     return fail(QD_ERR_INVALID_VALUE, "workspace smaller than qd_gqa_decode_auto_workspace_bytes()");
   char* scratch = static_cast<char*>(workspace);
@@ -3822,6 +3842,47 @@ int qd_gqa_decode_auto_info(int batch, int q_heads, int kv_heads, int head_dim, 
   if (splits) *splits = ap.splits;
   if (chunk_pages) *chunk_pages = ap.chunk_pages;
   return ap.stream_k ? (ap.fused ? 2 : 1) : 0;
+}
+
+int qd_gqa_decode_auto_path(int batch, int q_heads, int kv_heads, int head_dim, int block_size, int max_pages,
+                            int64_t num_blocks, int dtype, int* layout, int* chunks, int* workgroups, int* waves) {
+  if (check_launch_shapes(batch, q_heads, kv_heads, head_dim, block_size, max_pages, num_blocks, dtype, 1.f) != QD_OK)
+    return -1;
+  AutoPlan ap;
+  if (plan_call(batch, q_heads, kv_heads, head_dim, block_size, max_pages, num_blocks, dtype, true, false,
+                QD_STAGE_ALL, ~size_t{0}, &ap) != QD_OK)
+    return -1;
+  int path = QD_PATH_SPLIT, lay = QD_LAYOUT_EXACT, c = ap.kv_split;
+  int64_t wg = 0, nw = 1;
+  if (ap.wg_single > 0) {
+    path = QD_PATH_ONE_LAUNCH;
+    if (ap.single_gen) lay = QD_LAYOUT_GENERAL;
+    wg = static_cast<int64_t>(batch) * kv_heads * c;
+    nw = ap.wg_single;
+  } else if (ap.stream_k) {
+    path = ap.fused ? QD_PATH_FUSED : QD_PATH_BALANCED;
+    if (ap.gen_wave) lay = QD_LAYOUT_GENERAL;
+    wg = static_cast<int64_t>(ap.wgs) * (ap.fused ? 1 : ap.kv_slices);
+    nw = ap.wg_waves;
+  } else {
+    const SplitKernel kernel =
+        split_kernel(batch, q_heads, kv_heads, head_dim, block_size, num_blocks, dtype, ap.splits, 0, true);
+    if (kernel == SplitKernel::kValu) {
+      lay = QD_LAYOUT_VALU;
+      c = (q_heads / kv_heads + generic_heads(q_heads / kv_heads) - 1) / generic_heads(q_heads / kv_heads);
+    } else {
+      if (kernel == SplitKernel::kGeneral) lay = QD_LAYOUT_GENERAL;
+      c = kernel == SplitKernel::kGeneral ? kv_split_for(q_heads, kv_heads) : 1;
+      nw = wg_waves_for(static_cast<int64_t>(ap.splits) * kv_heads * c * batch,
+                        (static_cast<int64_t>(ap.chunk_pages) * block_size + 15) / 16, dtype, head_dim);
+    }
+    wg = static_cast<int64_t>(ap.splits) * batch * kv_heads * c;
+  }
+  if (layout) *layout = lay;
+  if (chunks) *chunks = c;
+  if (workgroups) *workgroups = static_cast<int>(std::min<int64_t>(wg, 2147483647));
+  if (waves) *waves = static_cast<int>(nw);
+  return path;
 }
 
 #ifdef QD_STAMPS

@@ -208,6 +208,9 @@ def stamps_mode(args) -> None:
                                      table.shape[1], dt, ctypes.byref(w_), ctypes.byref(s_), ctypes.byref(c_))
     if kind < 1:
         raise SystemExit(f"{cfg.name} does not take the balanced path")
+    if args.merge == "auto" and cabi.auto_path(cfg.batch, cfg.q_heads, cfg.kv_heads, cfg.head_dim, cfg.block_size,
+                                               table.shape[1], k.shape[0], dt)[0] == "one launch":
+        raise SystemExit(f"{cfg.name} runs in one launch, which has no timestamps; --merge unfused takes the balanced path")
     waves = w_.value
     flag = {"auto": 0, "fused": cabi.QD_STAGE_FUSED, "unfused": cabi.QD_STAGE_UNFUSED}[args.merge]
     fused = args.merge == "fused" or (args.merge == "auto" and kind == 2)
@@ -675,7 +678,8 @@ def sweep_mode(args) -> None:
                 inputs = make_decode_case(lengths=[length] * batch, q_heads=32, kv_heads=8, head_dim=128,
                                           block_size=16, dtype=dtype, device=dev)
                 maxp = inputs[3].shape[1]
-                kind, waves, _, _ = cabi.auto_info(batch, 32, 8, 128, 16, maxp, cabi.DTYPE[dtype])
+                path, layout, _, wgs, wg_waves = cabi.auto_path(batch, 32, 8, 128, 16, maxp, inputs[1].shape[0],
+                                                                cabi.DTYPE[dtype])
                 samples = time_samples(lambda i: attention_amd.gqa_decode(*inputs), 10, 20, stream)
                 med = statistics.median(samples)
                 ws = cabi.auto_workspace(batch, 32, 8, 128, 16, maxp, cabi.DTYPE[dtype], dev)
@@ -692,10 +696,8 @@ def sweep_mode(args) -> None:
                 row = {"dtype": DT_NAME[dtype], "batch": batch, "length": length, "hq": 32, "hkv": 8,
                        "head_dim": 128, "block_size": 16, "median_us": round(med * 1e3, 3),
                        "min_us": round(min(samples) * 1e3, 3), "max_us": round(max(samples) * 1e3, 3),
-                       "gpu_us": round(gpu_us, 3), "waves": waves,
-                       "gb_s": round(nbytes / (med * 1e-3) / 1e9, 1),
-                       "path": {1: "balanced MFMA + merge", 2: "balanced MFMA, fused merge",
-                                0: "split layout"}.get(kind, "?")}
+                       "gpu_us": round(gpu_us, 3), "waves": wgs * wg_waves,
+                       "gb_s": round(nbytes / (med * 1e-3) / 1e9, 1), "path": f"{path}, {layout} layout"}
                 rows.append(row)
                 print(json.dumps(row), flush=True)
                 del inputs, ws, out
@@ -765,7 +767,7 @@ def models_mode(args) -> None:
             ks.append(k.roll(i, dims=0).contiguous())
             vs.append(v.roll(i, dims=0).contiguous())
         maxp = table.shape[1]
-        kind, waves, _, _ = cabi.auto_info(batch, hq, hkv, d, 16, maxp, cabi.DTYPE[dt])
+        path, layout, _, wgs, wg_waves = cabi.auto_path(batch, hq, hkv, d, 16, maxp, k.shape[0], cabi.DTYPE[dt])
         ws = cabi.auto_workspace(batch, hq, hkv, d, 16, maxp, cabi.DTYPE[dt], dev)
         out = torch.empty_like(q)
         turn = [0]
@@ -781,9 +783,8 @@ def models_mode(args) -> None:
         us = graph_replay_us(enqueue, stream)
         nb = algorithmic_bytes([length] * batch, batch, hq, hkv, d, 16, 2)
         print(json.dumps({"model": args.model, "q_heads": hq, "kv_heads": hkv, "head_dim": d, "batch": batch,
-                          "len": length, "path": "balanced MFMA + merge" if kind >= 1 else "split layout",
-                          "waves": waves if kind >= 1 else None, "pools": pools, "gpu_us": round(us, 2),
-                          "gbs": round(nb / us / 1e3, 1), "pct_of_8tbs": round(nb / us / 8e4, 1),
+                          "len": length, "path": f"{path}, {layout} layout", "waves": wgs * wg_waves,
+                          "pools": pools, "gpu_us": round(us, 2), "gbs": round(nb / us / 1e3, 1), "pct_of_8tbs": round(nb / us / 8e4, 1),
                           "mb": round(nb / 1e6, 1)}), flush=True)
         del q, k, v, table, lens, ks, vs, ws, out
         torch.cuda.empty_cache()
@@ -1089,8 +1090,16 @@ def main() -> None:
     kind = cabi.lib().qd_gqa_decode_kernel_kind(cfg.q_heads, cfg.kv_heads, cfg.head_dim,
                                                 cfg.block_size, cabi.DTYPE[q.dtype],
                                                 cabi.QD_FLAG_FORCE_GENERIC if args.kernel == "generic" else 0)
-    if args.kernel == "auto" and args.splits == 0 and auto_kind == 1:
-        kname, kernels = "decode_mfma_sk_kernel", "decode_mfma_sk_kernel+merge_sk_kernel"
+    if args.kernel == "auto" and args.splits == 0:
+        ran, layout, _, wgs, wg_waves = cabi.auto_path(cfg.batch, cfg.q_heads, cfg.kv_heads, cfg.head_dim,
+                                                       cfg.block_size, table.shape[1], k.shape[0], cabi.DTYPE[q.dtype])
+        if args.compute == "valu":
+            ran = "balanced"
+        kname = {"split": "decode_generic_kernel" if layout == "valu" else "decode_wg_kernel",
+                 "one launch": "decode_wg_kernel"}.get(ran, "decode_mfma_sk_kernel")
+        kernels = kname + {"split": "+combine_kernel" if splits > 1 else "", "balanced": "+merge_sk_kernel"}.get(ran, "")
+        if args.compute != "valu":
+            auto_waves = wgs * wg_waves
     else:
         kname = "decode_wg_kernel" if kind == 1 else "decode_generic_kernel"
         kernels = kname + ("+combine_kernel" if splits > 1 else "")
@@ -1160,7 +1169,7 @@ def main() -> None:
                              f"U{list(cfg.len_range)} seed {10_000 + cfg.seed}: sum {sum(lengths)}, "
                              f"min {min(lengths)}, max {max(lengths)}"),
             "kv_pools_rotated": pools, "path": path, "kernels": kernels, "compute": args.compute,
-            "waves": auto_waves if auto_kind == 1 else None, "splits": splits, "chunk_pages": chunk,
+            "waves": auto_waves or None, "splits": splits, "chunk_pages": chunk,
             "algorithmic_bytes_per_call": alg_bytes,
             "flops_per_call": algorithmic_flops(lengths, cfg.q_heads, cfg.head_dim),
         },

@@ -251,10 +251,25 @@ int qd_gqa_decode_auto_noalloc(const void* q, const void* k_cache, const void* v
  * shape is reported as 0 may run the balanced kernels all the same (the
  * general layout, fp32 from 16384 tokens of capacity), and short contexts of
  * any kind run in one launch; what is reported is what stages, or a
- * workspace of the split layout's size, get.  Any output pointer
- * may be NULL. */
+ * workspace of the split layout's size, get (qd_gqa_decode_auto_path reports
+ * whole calls).  Any output pointer may be NULL. */
 int qd_gqa_decode_auto_info(int batch, int q_heads, int kv_heads, int head_dim, int block_size,
                             int max_pages, int dtype, int* waves, int* splits, int* chunk_pages);
+
+/* What a whole qd_gqa_decode_auto call runs for these shapes and a pool of
+ * num_blocks pages (aligned pointers, a workspace of
+ * qd_gqa_decode_auto_workspace_bytes()): returns QD_PATH_* or -1 for invalid
+ * shapes, with
+ *   *layout      QD_LAYOUT_*: the per-wave kernel body
+ *   *chunks      chunks that each kv-head's q-heads are served in (at most 16
+ *                q-heads each, 8 on the VALU kernel)
+ *   *workgroups  workgroups of the decode kernel
+ *   *waves       waves per workgroup.
+ * Any output pointer may be NULL. */
+enum { QD_PATH_SPLIT = 0, QD_PATH_BALANCED = 1, QD_PATH_FUSED = 2, QD_PATH_ONE_LAUNCH = 3 };
+enum { QD_LAYOUT_VALU = 0, QD_LAYOUT_EXACT = 1, QD_LAYOUT_GENERAL = 2 };
+int qd_gqa_decode_auto_path(int batch, int q_heads, int kv_heads, int head_dim, int block_size, int max_pages,
+                            int64_t num_blocks, int dtype, int* layout, int* chunks, int* workgroups, int* waves);
 
 /* ---- Paged KV-cache append ------------------------------------------
  * Replaces csrc/cuda/cache/kv_append.cu:29-56 (kv_append_cuda) behind the

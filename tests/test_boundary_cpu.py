@@ -349,6 +349,37 @@ def test_auto_plan_f32_balanced_path():
     assert cabi.auto_info(16, 32, 8, 128, 16, 64, F32)[0] == 0
 
 
+@pytest.mark.parametrize("args,path", [
+    ((4, 8, 2, 64, 16, 32, F16), ("one launch", "exact", 1, 8, 4)),
+    ((32, 32, 8, 128, 16, 256, BF16), ("balanced", "exact", 1, 256, 8)),
+    ((16, 32, 32, 80, 16, 128, F16), ("balanced", "general", 1, 256, 8)),
+    ((16, 32, 8, 128, 16, 64, F32), ("balanced", "exact", 1, 256, 4)),       # fp32 from 16384 tokens
+    ((1, 32, 8, 128, 16, 16, F32), ("split", "general", 1, 64, 2)),
+    ((32, 32, 8, 100, 16, 128, BF16), ("split", "valu", 1, 1024, 1)),
+    ((4, 32, 8, 128, 16, 8, F32), ("one launch", "exact", 1, 32, 4)),
+])
+def test_auto_path_reports_what_whole_calls_run(args, path):
+    got = cabi.auto_path(*args[:6], 1 << 20, args[6])
+    assert got[:3] == path[:3] and got[4] == path[4], got
+    if path[0] == "one launch":
+        assert got[3] == path[3]
+    assert cabi.auto_path(4, 8, 3, 64, 16, 4, 64, F16) is None
+
+
+@pytest.mark.parametrize("batch,hq,hkv,d,pages,dt", [
+    (1, 32, 1, 128, 8, F32), (4, 17, 1, 128, 8, F32), (3, 71, 1, 64, 16, F32), (3, 256, 2, 80, 8, F32),
+    (3, 64, 2, 256, 8, F32), (4097, 32, 1, 64, 2, BF16), (4097, 40, 1, 80, 1, F16), (4, 32, 1, 128, 8, BF16),
+    (2, 48, 1, 128, 32, BF16), (32, 128, 1, 128, 128, F16), (32, 48, 1, 128, 128, F32), (32, 100, 1, 72, 64, BF16),
+])
+def test_auto_path_serves_large_groups_in_chunks(batch, hq, hkv, d, pages, dt):
+    # A wave holds 16 q-heads (8 on the VALU kernel): a larger group needs as
+    # many chunks as cover it, and a workgroup (or wave) for each.
+    path, layout, chunks, wgs, waves = cabi.auto_path(batch, hq, hkv, d, 16, pages, 1 << 16, dt)
+    assert chunks * (8 if layout == "valu" else 16) >= hq // hkv, (path, layout)
+    if path == "one launch":
+        assert wgs == batch * hkv * chunks
+
+
 def test_auto_waves_per_workgroup_divide_kv_heads():
     for hkv, per_wg in [(1, 1), (2, 2), (4, 4), (8, 8), (12, 6), (16, 8), (7, 7), (9, 3)]:
         kind, waves, _, _ = cabi.auto_info(4, hkv, hkv, 64, 16, 64, F16)
