@@ -3348,13 +3348,15 @@ SplitKernel split_kernel(int batch, int q_heads, int kv_heads, int head_dim, int
 }
 
 // Plan of a call through the automatic path.  The general layout takes whole
-// calls, 32-bit pool rows, and a workspace of its plan's size; the split
-// layout serves the rest.
+// calls, 32-bit pool rows (in one launch too), and a workspace of its plan's
+// size; the split layout serves the rest.
 int plan_call(int batch, int q_heads, int kv_heads, int head_dim, int block_size, int max_pages, int64_t num_blocks,
               int dtype, bool aligned, bool valu, int stages, size_t workspace_bytes, AutoPlan* ap) {
   const int st = auto_plan(batch, q_heads, kv_heads, head_dim, block_size, max_pages, dtype, aligned, ap, valu);
   if (st != QD_OK) return st;
-  if (ap->general && (stages != QD_STAGE_ALL || !pool_rows_fit(num_blocks, block_size) || workspace_bytes < ap->ws_bytes))
+  const bool rows_fit = pool_rows_fit(num_blocks, block_size);
+  if (((ap->general || ap->single_gen) && !rows_fit) ||
+      (ap->general && (stages != QD_STAGE_ALL || workspace_bytes < ap->ws_bytes)))
     return auto_plan(batch, q_heads, kv_heads, head_dim, block_size, max_pages, dtype, aligned, ap, valu, false);
   return QD_OK;
 }

@@ -380,6 +380,21 @@ def test_auto_path_serves_large_groups_in_chunks(batch, hq, hkv, d, pages, dt):
         assert wgs == batch * hkv * chunks
 
 
+@pytest.mark.parametrize("batch,hq,hkv,d,p,pages,dt", [
+    (1, 1, 1, 8, 16, 8, F32), (4, 4, 1, 16, 5, 20, F32), (1, 8, 1, 256, 16, 8, F32), (1, 2, 1, 32, 16, 2, BF16),
+    (4097, 1, 1, 40, 8, 1, F16), (4097, 1, 1, 40, 8, 1, F32), (16, 4, 4, 80, 16, 64, F16), (8, 8, 2, 72, 16, 128, F32),
+    (1, 1, 1, 8, 16, 4096, F32),
+])
+def test_auto_path_general_layout_needs_32_bit_pool_rows(batch, hq, hkv, d, p, pages, dt):
+    # The general layout forms pool rows (page * block_size + slot) in 32
+    # bits: a pool of more than 2^31 - 1 rows takes the VALU kernel, whichever
+    # path the shape runs on.
+    most = (2**31 - 1) // p
+    assert cabi.auto_path(batch, hq, hkv, d, p, pages, most, dt)[1] == "general"
+    for blocks in (most + 1, 2**31, 2**40, 2**62):
+        assert cabi.auto_path(batch, hq, hkv, d, p, pages, blocks, dt)[1] == "valu", blocks
+
+
 def test_auto_waves_per_workgroup_divide_kv_heads():
     for hkv, per_wg in [(1, 1), (2, 2), (4, 4), (8, 8), (12, 6), (16, 8), (7, 7), (9, 3)]:
         kind, waves, _, _ = cabi.auto_info(4, hkv, hkv, 64, 16, 64, F16)
