@@ -900,6 +900,85 @@ struct MfmaWave {
   }
 };
 
+// Sum over N chunks of K chunk x Q chunk (four fp32 MFMAs each), per lane 16
+// bytes of K row r16 and of query row r16 per chunk (dims 16c + 4*q4 + e).
+//
+// fp32 sums in short chains: a v_mfma_f32_16x16x4_f32 adds its four products
+// one after the other, so one accumulator over head_dim 128 rounds 128 times
+// at growing sums.  Chains of LEN MFMAs (4 * LEN products) and a binary tree
+// over them round like the VALU kernel's 16 lanes and their tree.  Four chains
+// at a time, side by side, the tree's sums between the next four's MFMAs.
+// LEN 4 where the kernel runs one wave per SIMD (head_dim 128: LEN 2 costs 3%
+// of the call for no smaller error), as the VALU kernel has 16 products per
+// lane above head_dim 128.
+//
+// Relative error against 64 bits (2-norm), VALU kernel -> one accumulator ->
+// this, with pv_f32: Hq32/Hkv8 D128 B16 U[64, 1024] 1.72e-7 -> 3.90e-7 ->
+// 1.68e-7; over 90 drawn shapes 0.3 to 1.05 of the VALU kernel's (one
+// accumulator: 1.6 to 3.6 times).  The calls take as long as with one
+// accumulator or up to 4% less: the chain of dependent MFMAs is gone.
+template <int N, int LEN>
+__device__ __forceinline__ f32x4 qk_f32(const u32x4* ka, const u32x4* qf) {
+  static_assert(LEN == 2 || LEN == 4, "half a chunk or a chunk per chain");
+  constexpr int kChains = N * 4 / LEN, kBlocks = (kChains + 3) / 4;
+  f32x4 t[2][4];
+  f32x4 level[4];  // level i: the sum of 2^i finished blocks
+  auto block = [&](int b) {
+#pragma unroll
+    for (int e = 0; e < LEN; ++e)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int at = (4 * b + j) * LEN + e, c = at / 4, w = at % 4;
+        if (4 * b + j >= kChains) continue;
+        t[b & 1][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(ka[c][w]), __uint_as_float(qf[c][w]),
+                                                           e == 0 ? f32x4{0.f, 0.f, 0.f, 0.f} : t[b & 1][j], 0, 0, 0);
+      }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto add = [&](int b) {
+    f32x4* x = t[b & 1];
+#pragma unroll
+    for (int w = 1; w < 4; w *= 2)
+#pragma unroll
+      for (int j = 0; j < 4; j += 2 * w)
+        if (4 * b + j + w < kChains) x[j] += x[j + w];
+    f32x4 y = x[0];
+    int i = 0;
+#pragma unroll
+    for (int k = b; k & 1; k >>= 1) y = level[i++] + y;
+    level[i] = y;
+  };
+  block(0);
+#pragma unroll
+  for (int b = 1; b < kBlocks; ++b) {
+    block(b);
+    add(b - 1);
+  }
+  add(kBlocks - 1);
+  f32x4 s = {0.f, 0.f, 0.f, 0.f};
+  bool first = true;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    if ((kBlocks >> i) & 1) {
+      s = first ? level[i] : level[i] + s;
+      first = false;
+    }
+  }
+  return s;
+}
+
+// acc * alpha + V^T x P^T of one group (MfmaWaveF32's PV layout): the lane's
+// column of rows 4*q4 + 0..3, v, against their weights pr.  The group's sum is
+// formed by itself and added with one rounding.
+__device__ __forceinline__ f32x4 pv_f32(f32x4 acc, float alpha, const float (&v)[4], const float (&pr)[4]) {
+  f32x4 t = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int c = 0; c < 4; ++c) t = __builtin_amdgcn_mfma_f32_16x16x4f32(v[c], pr[c], t, 0, 0, 0);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) acc[i] = fmaf(acc[i], alpha, t[i]);
+  return acc;
+}
+
 // One wave's decode state for one kv-head of an fp32 cache, on the matrix
 // cores in fp32 (v_mfma_f32_16x16x4_f32: fp32 products and sums, the
 // reference's arithmetic).  Lane l, r16 = l % 16, q4 = l / 16:
@@ -995,12 +1074,7 @@ struct MfmaWaveF32 : MfmaWave<D, QD_DTYPE_F32, PF, 1> {
 #pragma unroll
     for (int c = 0; c < KQ; ++c)
       ka[c] = *reinterpret_cast<const u32x4*>(ktile + this->r16 * Tile::kStride + 64 * c + 16 * this->q4);
-    f32x4 s = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int c = 0; c < KQ; ++c)
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-        s = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(ka[c][e]), __uint_as_float(qf[c][e]), s, 0, 0, 0);
+    const f32x4 s = qk_f32<KQ, D == 128 ? 4 : 2>(ka, qf);
     float x[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) x[i] = (4 * this->q4 + i <= last) ? s[i] : -INFINITY;
@@ -1015,16 +1089,11 @@ struct MfmaWaveF32 : MfmaWave<D, QD_DTYPE_F32, PF, 1> {
     for (int i = 0; i < 4; ++i) pr[i] = fast_exp2(fmaf(x[i], p.sl2, -mref));
     this->l_run[0] = fmaf(this->l_run[0], alpha, (pr[0] + pr[1]) + (pr[2] + pr[3]));
     this->m_run[0] = mn;
-    if (__builtin_amdgcn_read_exec() & __ballot(alpha != 1.f)) {
-#pragma unroll
-      for (int d = 0; d < DV; ++d) this->acc[0][d] *= alpha;
-    }
 #pragma unroll
     for (int d = 0; d < DV; ++d)
-#pragma unroll
-      for (int c = 0; c < 4; ++c)
-        this->acc[0][d] = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(buf.v[c].w[d]), pr[c],
-                                                               this->acc[0][d], 0, 0, 0);
+      this->acc[0][d] = pv_f32(this->acc[0][d], alpha, {__uint_as_float(buf.v[0].w[d]), __uint_as_float(buf.v[1].w[d]),
+                                                        __uint_as_float(buf.v[2].w[d]), __uint_as_float(buf.v[3].w[d])},
+                               pr);
     __builtin_amdgcn_sched_barrier(0);
   }
 
@@ -1233,15 +1302,11 @@ struct GenWave : MfmaWave<VD, DT, PF, 1> {
     for (int c = 0; c < KCG; ++c)
       ka[c] = *reinterpret_cast<const u32x4*>(ktile + this->r16 * kStride + 64 * c + 16 * this->q4);
     f32x4 s = {0.f, 0.f, 0.f, 0.f};
+    if constexpr (kF32) {
+      s = qk_f32<KCG, KCG <= 8 ? 2 : 4>(ka, qg);
+    } else {
 #pragma unroll
-    for (int c = 0; c < KCG; ++c) {
-      if constexpr (kF32) {
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-          s = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(ka[c][e]), __uint_as_float(qg[c][e]), s, 0, 0, 0);
-      } else {
-        s = Ops::qk(ka[c], qg[c], s);
-      }
+      for (int c = 0; c < KCG; ++c) s = Ops::qk(ka[c], qg[c], s);
     }
     float x[4];
 #pragma unroll
@@ -1257,18 +1322,17 @@ struct GenWave : MfmaWave<VD, DT, PF, 1> {
     for (int i = 0; i < 4; ++i) pr[i] = fast_exp2(fmaf(x[i], p.sl2, -mref));
     this->l_run[0] = fmaf(this->l_run[0], alpha, (pr[0] + pr[1]) + (pr[2] + pr[3]));
     this->m_run[0] = mn;
-    if (__builtin_amdgcn_read_exec() & __ballot(alpha != 1.f)) {
-#pragma unroll
-      for (int d = 0; d < EV; ++d) this->acc[0][d] *= alpha;
-    }
     if constexpr (kF32) {
 #pragma unroll
       for (int d = 0; d < EV; ++d)
-#pragma unroll
-        for (int c = 0; c < 4; ++c)
-          this->acc[0][d] = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(buf.v[c].w[d]), pr[c],
-                                                                 this->acc[0][d], 0, 0, 0);
+        this->acc[0][d] = pv_f32(this->acc[0][d], alpha, {__uint_as_float(buf.v[0].w[d]), __uint_as_float(buf.v[1].w[d]),
+                                                          __uint_as_float(buf.v[2].w[d]), __uint_as_float(buf.v[3].w[d])},
+                                 pr);
     } else {
+      if (__builtin_amdgcn_read_exec() & __ballot(alpha != 1.f)) {
+#pragma unroll
+        for (int d = 0; d < EV; ++d) this->acc[0][d] *= alpha;
+      }
       const u32x2 hi = {Ops::pack2(pr[0], pr[1]), Ops::pack2(pr[2], pr[3])};
       const u32x4 w = {hi[0], hi[1], Ops::rest2(pr[0], pr[1], hi[0]), Ops::rest2(pr[2], pr[3], hi[1])};
 #pragma unroll
@@ -2564,9 +2628,17 @@ bool f32_mfma_applies(int q_heads, int kv_heads, int head_dim, int block_size, i
 // The same kernel below that capacity, as a whole call only (stages and
 // qd_gqa_decode_auto_info keep the split layout there): since its kv-head
 // passes have workgroups of their own it wins from kF32GeneralTokens of
-// capacity on (Hq32/Hkv8 D128, us per call, split layout -> balanced: B16
-// U[64, 1024] 24.5 -> 20.4, B16/L1024 33.8 -> 32.4, B4/L4096 33.9 -> 32.2, Hkv1
-// B40 U[300, 1000] 25.4 -> 16.8; B4/L1024 16.5 -> 16.4, B1/L1024 11.9 -> 14.1).
+// capacity on, for every head_dim, group size and mix of lengths measured.
+// Split layout -> balanced (Hkv8, group 4, us per call, fresh inputs):
+//   capacity          4096          8192          12288         16384         20480
+//   D128 uniform L    21.5 -> 20.7  27.4 -> 26.7  36.8 -> 32.8  38.7 -> 37.9  50.3 -> 43.4
+//   D128 U[64, 1024]                23.2 -> 19.7  29.1 -> 24.0  33.9 -> 25.1  42.9 -> 30.6
+//   D64 uniform L     14.6 -> 18.0  20.9 -> 20.0  22.9 -> 23.1  31.4 -> 25.0  40.3 -> 25.5
+//   D80 uniform L     19.9 -> 20.4  22.5 -> 25.0  35.2 -> 30.2  59.4 -> 35.6  74.2 -> 40.9
+//   D128 Hkv32 unif.                52.6 -> 56.5  82.4 -> 77.1  93.1 -> 90.7
+//   D128 Hq8/Hkv1                   14.5 -> 17.3  16.1 -> 18.9  23.1 -> 20.7
+// (up to 12288 the split layout's own kernels as of now; from 16384 on the VALU
+// kernel that the split layout would run).  Below, it depends on the shape.
 // Those read fresh inputs; repeated over one 134 MB input that the Infinity
 // Cache holds, the split layout keeps 29.6 against 32 us at B4/L4096 and
 // B16/L1024.
