@@ -3279,14 +3279,18 @@ int auto_plan(int batch, int q_heads, int kv_heads, int head_dim, int block_size
                          : mfma_applies(vkv * gv, vkv, head_dim, block_size, dtype);
   const int64_t groups = (static_cast<int64_t>(max_pages) * block_size + 15) / 16;  // of one sequence, at most
   const int64_t gmax = static_cast<int64_t>(batch) * groups;
+  // fp32 at head_dim 256 stays on the VALU kernel, whose rows of 16 whole
+  // elements per lane need no guards (us per call, VALU -> general: Hkv8 B4/L4096
+  // 84.7 -> 96.7, B16/L2048 146 -> 157, in one launch B1/L128 18.0 -> 21.0); with
+  // guards, at other head dims above 128, it takes about twice as long.
+  const bool gen_ok = allow_general && general_applies(head_dim, dtype) && !(f32 && head_dim == 256);
   const bool general =
-      !exact && !valu && allow_general &&
-      general_applies(head_dim, dtype) &&
+      !exact && !valu && gen_ok &&
       (!f32 || static_cast<int64_t>(batch) * max_pages * block_size >= kF32GeneralTokens);
   // (fp32 head_dim 64 and 128 on whole-group pages keep MfmaWaveF32.)
   const bool gen_wave = general && !f32_mfma_applies(q_heads, kv_heads, head_dim, block_size, dtype);
   const bool f32_wave = f32_mfma_applies(q_heads, kv_heads, head_dim, block_size, dtype);
-  const bool single_gen = !exact && !f32_wave && allow_general && general_applies(head_dim, dtype);
+  const bool single_gen = !exact && !f32_wave && gen_ok;
   if (aligned && split > 0 && !valu && (exact || f32_wave || single_gen)) {
     ap->wg_single = vkv <= 65535 && wg_single_applies(static_cast<int64_t>(batch) * vkv, groups, dtype, head_dim, single_gen)
                         ? wg_waves_for(static_cast<int64_t>(batch) * vkv, groups, dtype, head_dim)

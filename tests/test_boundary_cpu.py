@@ -357,6 +357,9 @@ def test_auto_plan_f32_balanced_path():
     ((1, 32, 8, 128, 16, 16, F32), ("split", "general", 1, 64, 2)),
     ((32, 32, 8, 100, 16, 128, BF16), ("split", "valu", 1, 1024, 1)),
     ((4, 32, 8, 128, 16, 8, F32), ("one launch", "exact", 1, 32, 4)),
+    ((4, 32, 8, 256, 16, 8, F32), ("split", "general", 1, 128, 2)),          # fp32 at 256: splits only
+    ((16, 32, 8, 256, 16, 128, F32), ("split", "valu", 1, 1024, 1)),
+    ((16, 32, 8, 240, 16, 128, F32), ("balanced", "general", 1, 256, 4)),
 ])
 def test_auto_path_reports_what_whole_calls_run(args, path):
     got = cabi.auto_path(*args[:6], 1 << 20, args[6])
@@ -368,7 +371,7 @@ def test_auto_path_reports_what_whole_calls_run(args, path):
 
 @pytest.mark.parametrize("batch,hq,hkv,d,pages,dt", [
     (1, 32, 1, 128, 8, F32), (4, 17, 1, 128, 8, F32), (3, 71, 1, 64, 16, F32), (3, 256, 2, 80, 8, F32),
-    (3, 64, 2, 256, 8, F32), (4097, 32, 1, 64, 2, BF16), (4097, 40, 1, 80, 1, F16), (4, 32, 1, 128, 8, BF16),
+    (3, 64, 2, 192, 8, F32), (3, 64, 2, 256, 8, F32), (4097, 32, 1, 64, 2, BF16), (4097, 40, 1, 80, 1, F16), (4, 32, 1, 128, 8, BF16),
     (2, 48, 1, 128, 32, BF16), (32, 128, 1, 128, 128, F16), (32, 48, 1, 128, 128, F32), (32, 100, 1, 72, 64, BF16),
 ])
 def test_auto_path_serves_large_groups_in_chunks(batch, hq, hkv, d, pages, dt):
