@@ -1747,7 +1747,8 @@ __host__ __device__ constexpr int shared_list_tiles(int mode) { return mode == k
 __host__ __device__ constexpr size_t mla_shared_lds_bytes(int mode) {
   return static_cast<size_t>(shared_bufs(mode)) * kShTileBytes  // tile ring (prologue arrays before the first tile)
          + static_cast<size_t>(shared_list_tiles(mode) + kShCtlPad) * 16  // tile list
-         + (mode == kShGather ? static_cast<size_t>(kShGatherTiles + kShCtlPad) * kShTokens * 4 : 0);  // row list
+         + (mode == kShGather ? static_cast<size_t>(kShGatherTiles + kShCtlPad) * kShTokens * 4 : 0)  // row list
+         + (mode == kShFold ? 1024 : 0);  // a latent row of zeros
 }
 
 static_assert(kShRows * (4 + 4 + 8) + kShListTiles * 16 <= (kShBufs - 1) * kShTileBytes,
@@ -1857,9 +1858,7 @@ __device__ __forceinline__ void lds_wait_tied(u32x2& a, u32x2& b) {
 // heads heads ([B, T, H, *] is that already), so the cache is read once for
 // all of them; each lane masks the tokens its query does not see.
 // us per call (latent write and decode) against the wave kernel: fp16 2 x 32
-// heads, B48, U[512, 4096] 76.5 -> 56.5.  A token that some queries of its
-// sequence see must hold finite values, as any visible token must (an Inf or
-// NaN there reaches all of them).
+// heads, B48, U[512, 4096] 76.5 -> 56.5.
 template <int DT, bool NT, int MODE>
 __global__ __launch_bounds__(kShThreads) void mla_attend_shared_kernel(MlaParams p) {
   using E = Elem<DT>;
@@ -1868,6 +1867,7 @@ __global__ __launch_bounds__(kShThreads) void mla_attend_shared_kernel(MlaParams
   constexpr int kDc = 512;
   constexpr int kW = 576;
   constexpr int kBufs = shared_bufs(MODE);
+  constexpr bool kSplit = Ops::kSplitWeights;
   extern __shared__ __align__(16) char smem[];
   const int tid = static_cast<int>(threadIdx.x);
   const int lane = tid & 63;
@@ -1886,6 +1886,10 @@ __global__ __launch_bounds__(kShThreads) void mla_attend_shared_kernel(MlaParams
   char* ring = smem;
   i32x4* ctl = reinterpret_cast<i32x4*>(smem + kBufs * kShTileBytes);
   [[maybe_unused]] uint32_t* prow = reinterpret_cast<uint32_t*>(ctl + shared_list_tiles(MODE) + kShCtlPad);  // pool rows
+  [[maybe_unused]] char* zeros = reinterpret_cast<char*>(ctl + shared_list_tiles(MODE) + kShCtlPad);  // kShFold
+  if constexpr (MODE == kShFold) {
+    if (tid < 64) *reinterpret_cast<u32x4*>(zeros + 16 * tid) = u32x4{0u, 0u, 0u, 0u};  // read after the barriers below
+  }
   // Prologue arrays, inside the ring.
   int* rt = reinterpret_cast<int*>(ring);                      // [rows] tiles
   int* re = rt + kShRows;                                      // [rows] visible end
@@ -2218,12 +2222,34 @@ __global__ __launch_bounds__(kShThreads) void mla_attend_shared_kernel(MlaParams
     // The first PV operand reads, in flight during the softmax (inline asm,
     // TrRead: the builtin form would wait for the next tiles' DMA, issued
     // during QK).
-    const uint32_t trb = lds_addr(slot) + (4 * q4 + (r16 >> 2)) * kShLatStride + 8 * (r16 & 3);
+    uint32_t tr0, tr1;  // rows 4 q4 + r16 / 4 of the two row blocks
+    [[maybe_unused]] int seen = kShTokens;                      // kShFold: rows that this lane's query sees
+    [[maybe_unused]] int s_min = kShTokens, s_max = kShTokens;  // ... over the wave's heads
+    {
+      const uint32_t tile = lds_addr(slot) + 8 * (r16 & 3);
+      const int row = 4 * q4 + (r16 >> 2);
+      tr0 = tile + row * kShLatStride;
+      tr1 = tr0 + 16 * kShLatStride;
+      if constexpr (MODE == kShFold) {
+        // row_end, with the table's capacity in nv.
+        const int tok0 = kShTokens * (e[2] >> 7);
+        seen = h < p.H ? min(p.causal && q_pos < q_len ? q_pos + 1 : q_len, tok0 + nv) - tok0 : kShTokens;
+        if (__ballot(seen < kShTokens)) {
+          // Only rows that all of the wave's heads see go into the products, in
+          // place of the others the last of them (or zeros) with weight 0: a
+          // weight of 0 alone would not hide a row (0 x Inf is NaN).
+          s_min = __builtin_amdgcn_readfirstlane(row16_min(seen));
+          s_max = -__builtin_amdgcn_readfirstlane(row16_min(h < p.H ? -seen : 0));
+          tr0 = s_min > 0 ? tile + min(row, s_min - 1) * kShLatStride : lds_addr(zeros) + 8 * (r16 & 3);
+          tr1 = s_min > 0 ? tile + min(16 + row, s_min - 1) * kShLatStride : tr0;
+        }
+      }
+    }
     u32x2 av[kShPvAhead][2];
     static_for<0, kShPvAhead>([&](auto c) {
       constexpr int cb = decltype(c)::value;
-      TrRead<32 * cb>::issue(trb, av[cb][0]);
-      TrRead<16 * kShLatStride + 32 * cb>::issue(trb, av[cb][1]);
+      TrRead<32 * cb>::issue(tr0, av[cb][0]);
+      TrRead<32 * cb>::issue(tr1, av[cb][1]);
     });
 
     // Softmax over the tile's 32 tokens: lane holds tokens 16 tb + 4 q4 + i.
@@ -2237,17 +2263,11 @@ __global__ __launch_bounds__(kShThreads) void mla_attend_shared_kernel(MlaParams
 #pragma unroll
       for (int i = 0; i < 4; ++i) x[tb][i] = st[i] * p.sl2;
     }
-    if constexpr (MODE == kShFold) {
-      // Tokens this lane's query does not see (row_end, with the table's
-      // capacity in nv), in the tiles that hold any.
-      const int tok0 = kShTokens * (e[2] >> 7);
-      const int seen = min(p.causal && q_pos < q_len ? q_pos + 1 : q_len, tok0 + nv) - tok0;
-      if (__ballot(seen < kShTokens)) {
+    if (MODE == kShFold && s_min < kShTokens) {  // uniform
 #pragma unroll
-        for (int tb = 0; tb < 2; ++tb)
+      for (int tb = 0; tb < 2; ++tb)
 #pragma unroll
-          for (int i = 0; i < 4; ++i) x[tb][i] = 16 * tb + 4 * q4 + i < seen ? x[tb][i] : -INFINITY;
-      }
+        for (int i = 0; i < 4; ++i) x[tb][i] = 16 * tb + 4 * q4 + i < seen ? x[tb][i] : -INFINITY;
     }
     float mx = fmaxf(fmaxf(fmaxf(x[0][0], x[0][1]), fmaxf(x[0][2], x[0][3])),
                      fmaxf(fmaxf(x[1][0], x[1][1]), fmaxf(x[1][2], x[1][3])));
@@ -2261,28 +2281,45 @@ __global__ __launch_bounds__(kShThreads) void mla_attend_shared_kernel(MlaParams
       for (int cb = 0; cb < kShColBlocks; ++cb) acc[cb] *= alpha;
     }
     const float m_use = m_run == -INFINITY ? 0.f : m_run;
+    float pr[2][4];
+#pragma unroll
+    for (int tb = 0; tb < 2; ++tb)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) pr[tb][i] = fast_exp2(x[tb][i] - m_use);
+    if constexpr (MODE == kShGather) {
+      if (e[1] != -1) {  // uniform
+#pragma unroll
+        for (int tb = 0; tb < 2; ++tb)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) pr[tb][i] = (e[1] >> (16 * tb + 4 * q4 + i)) & 1 ? pr[tb][i] : 0.f;
+      }
+    } else if (MODE == kShDense && nv < kShTokens) {  // uniform
+#pragma unroll
+      for (int tb = 0; tb < 2; ++tb)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) pr[tb][i] = 16 * tb + 4 * q4 + i < nv ? pr[tb][i] : 0.f;
+    }
+    float wp[2][4];  // kShFold: of the rows in the products
+#pragma unroll
+    for (int tb = 0; tb < 2; ++tb)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) wp[tb][i] = pr[tb][i];
+    if (MODE == kShFold && s_min < s_max) {  // uniform
+#pragma unroll
+      for (int tb = 0; tb < 2; ++tb)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) wp[tb][i] = 16 * tb + 4 * q4 + i < s_min ? wp[tb][i] : 0.f;
+    }
     u32x4 pbl[2];
     u32x2 pb[2];
 #pragma unroll
     for (int tb = 0; tb < 2; ++tb) {
-      float pr[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) pr[i] = fast_exp2(x[tb][i] - m_use);
-      if constexpr (MODE == kShGather) {
-        if (e[1] != -1) {  // uniform
-#pragma unroll
-          for (int i = 0; i < 4; ++i) pr[i] = (e[1] >> (16 * tb + 4 * q4 + i)) & 1 ? pr[i] : 0.f;
-        }
-      } else if (MODE == kShDense && nv < kShTokens) {  // uniform
-#pragma unroll
-        for (int i = 0; i < 4; ++i) pr[i] = 16 * tb + 4 * q4 + i < nv ? pr[i] : 0.f;
-      }
-      pb[tb] = u32x2{Ops::pack2(pr[0], pr[1]), Ops::pack2(pr[2], pr[3])};
+      pb[tb] = u32x2{Ops::pack2(wp[tb][0], wp[tb][1]), Ops::pack2(wp[tb][2], wp[tb][3])};
       pbl[tb] = u32x4{pb[tb][0], pb[tb][1], 0u, 0u};
-      if constexpr (Ops::kSplitWeights) {
-        pbl[tb][2] = Ops::rest2(pr[0], pr[1], pb[tb][0]);
-        pbl[tb][3] = Ops::rest2(pr[2], pr[3], pb[tb][1]);
-        l_run += (pr[0] + pr[1]) + (pr[2] + pr[3]);
+      if constexpr (kSplit) {
+        pbl[tb][2] = Ops::rest2(wp[tb][0], wp[tb][1], pb[tb][0]);
+        pbl[tb][3] = Ops::rest2(wp[tb][2], wp[tb][3], pb[tb][1]);
+        l_run += (wp[tb][0] + wp[tb][1]) + (wp[tb][2] + wp[tb][3]);
       } else {
         l_run += Ops::sum2(pb[tb][0]) + Ops::sum2(pb[tb][1]);
       }
@@ -2310,13 +2347,43 @@ __global__ __launch_bounds__(kShThreads) void mla_attend_shared_kernel(MlaParams
       lds_wait_tied<later>(av[j][0], av[j][1]);
       const u32x4 a = {av[j][0][0], av[j][0][1], av[j][1][0], av[j][1][1]};
       if constexpr (cb + kShPvAhead < kShColBlocks) {
-        TrRead<32 * (cb + kShPvAhead)>::issue(trb, av[j][0]);
-        TrRead<16 * kShLatStride + 32 * (cb + kShPvAhead)>::issue(trb, av[j][1]);
+        TrRead<32 * (cb + kShPvAhead)>::issue(tr0, av[j][0]);
+        TrRead<32 * (cb + kShPvAhead)>::issue(tr1, av[j][1]);
       }
       acc[cb] = Ops::mma32(a, bhi, acc[cb]);
-      if constexpr (Ops::kSplitWeights) acc[cb] = Ops::mma32(a, blo, acc[cb]);
+      if constexpr (kSplit) acc[cb] = Ops::mma32(a, blo, acc[cb]);
       __builtin_amdgcn_sched_barrier(0);
     });
+
+    if (MODE == kShFold && __builtin_expect(s_min < s_max, 0)) {
+      // Rows that some of the wave's heads see and others do not (heads of
+      // several queries): row by row, on the lanes that see them.
+#pragma clang loop unroll(disable)
+      for (int t = max(s_min, 0); t < s_max; ++t) {
+        float wt = 0.f;
+#pragma unroll
+        for (int tb = 0; tb < 2; ++tb)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) wt = 16 * tb + i == (t & 19) ? pr[tb][i] : wt;
+        wt = __shfl(wt, 16 * ((t >> 2) & 3) + r16);
+        if (t < seen) {
+          const char* vr = slot + t * kShLatStride + 8 * q4;
+#pragma unroll
+          for (int cb = 0; cb < kShColBlocks; ++cb) {
+            const u32x2 v = *reinterpret_cast<const u32x2*>(vr + 32 * cb);
+            const f32x2 v0 = Ops::unpack2(v[0]), v1 = Ops::unpack2(v[1]);
+            acc[cb][0] = fmaf(wt, v0[0], acc[cb][0]);
+            acc[cb][1] = fmaf(wt, v0[1], acc[cb][1]);
+            acc[cb][2] = fmaf(wt, v1[0], acc[cb][2]);
+            acc[cb][3] = fmaf(wt, v1[1], acc[cb][3]);
+          }
+        }
+      }
+#pragma unroll
+      for (int tb = 0; tb < 2; ++tb)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) l_run += 16 * tb + 4 * q4 + i < s_min ? 0.f : pr[tb][i];
+    }
 
     if (last) {
       [[maybe_unused]] const uint64_t st_re0 = QD_MLA_STAMPS_ON ? __builtin_amdgcn_s_memtime() : 0;

@@ -72,6 +72,15 @@ __device__ __forceinline__ float row16_sum(float x) {
   return x;
 }
 
+// Smallest of each row of 16 lanes, in every lane of the row.
+__device__ __forceinline__ int row16_min(int x) {
+  x = min(x, __builtin_amdgcn_update_dpp(x, x, 0xB1, 0xF, 0xF, false));   // as in row16_sum
+  x = min(x, __builtin_amdgcn_update_dpp(x, x, 0x4E, 0xF, 0xF, false));
+  x = min(x, __builtin_amdgcn_update_dpp(x, x, 0x141, 0xF, 0xF, false));
+  x = min(x, __builtin_amdgcn_update_dpp(x, x, 0x140, 0xF, 0xF, false));
+  return x;
+}
+
 __device__ __forceinline__ float wave_max(float x) {
   for (int off = 32; off >= 1; off >>= 1) x = fmaxf(x, __shfl_xor(x, off));
   return x;
@@ -163,7 +172,8 @@ struct MfmaOps<QD_DTYPE_BF16> {
     const f32x2 v = {x, y};
     return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2));
   }
-  // Sum of the two 16-bit values packed in w, in fp32.
+  // The two 16-bit values packed in w, and their sum, in fp32.
+  __device__ static f32x2 unpack2(uint32_t w) { return f32x2{__uint_as_float(w << 16), __uint_as_float(w & 0xFFFF0000u)}; }
   __device__ static float sum2(uint32_t w) { return __uint_as_float(w << 16) + __uint_as_float(w & 0xFFFF0000u); }
   // Weights for the PV product as hi + lo: bf16 keeps 8 significant bits,
   // and a single rounding of the softmax weights (relative 2^-9 each) put
@@ -191,8 +201,9 @@ struct MfmaOps<QD_DTYPE_F16> {
     const f32x2 v = {x, y};
     return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, f16x2));
   }
+  __device__ static f32x2 unpack2(uint32_t w) { return __builtin_convertvector(__builtin_bit_cast(f16x2, w), f32x2); }
   __device__ static float sum2(uint32_t w) {
-    const f32x2 v = __builtin_convertvector(__builtin_bit_cast(f16x2, w), f32x2);
+    const f32x2 v = unpack2(w);
     return v[0] + v[1];
   }
   // fp16 keeps 11 significant bits: one rounding of the weights stays far
