@@ -2800,12 +2800,30 @@ int cpt_for(int W) {
 constexpr int kNoGather = 1 << 30;  // internal plan flag
 
 // Whether the q_len queries of a sequence run as one row of q_len * heads
-// heads of the shared-tile kernel (dense rows): from 32 on, where its workgroup
-// of 64 is half full (the wave kernel reads every cache row once per query and
-// 16 heads).  us per call, wave kernel -> folded: 2 x 16 heads B48 U[512, 4096]
-// 60.5 -> 50.2, B128 U[512, 2000] 91.8 -> 67.4; 3 x 16 B48 81.0 -> 55.0; 2 x 20 B48
-// 72.3 -> 51.4; 4 x 8 B16 50.7 -> 45.4.
-bool shared_fold_applies(int q_len, int heads) { return q_len * heads >= 32; }
+// heads of the shared-tile kernel (dense rows) and not as rows of their own,
+// which read every cache row once per query and 16 heads (wave kernel).  us per
+// mla_decode, bf16, rows of their own -> folded, "queries x heads":
+//   from 32 heads in all: 2 x 16 B32/L512 34.7 -> 33.8, 4 x 8 B32/L512 39.8 -> 34.6, 3 x 32
+//     B8/L2048 41.9 -> 39.7, 16 x 16 B8/L2048 60.6 -> 47.9, 64 x 32 B1/L4096 83.2 -> 64.4;
+//   below 64 per query: from 64 on a workgroup holds one query's heads as it is,
+//     and folding only makes every query walk the longest one's tiles: 2 x 64
+//     B8/L2048 39.1 -> 41.7, 64 x 64 B1/L4096 85.7 -> 155.8, 128 x 128 252 -> 1775;
+//   from kFoldTokens (sequences x queries x 16-head groups x capacity), less
+//     fits the CUs as it is: 8 x 8 B4/L64 (2K) 21.4 -> 26.8;
+//   a context of kFoldContext times the queries at least: a chunk of its own
+//     context has half of its pairs hidden, 16 x 20 B4/L64 23.9 -> 27.6, 32 x 32 30.8
+//     -> 34.3, 128 x 8 B4/L128 46.8 -> 51.5; but for rows that fill the wave
+//     kernel's list: 96 x 8 B32/L512 611 -> 146;
+//   up to kFoldHeads in all: more head groups leave each few ranges, whose
+//     prologues walk all queries, 128 x 32 B1/L4096 142 -> 167, 128 x 48 206 -> 394; but
+//     for many rows: 128 x 32 B8/L2048 809 -> 516.
+constexpr int64_t kFoldTokens = 8192, kFoldHeads = 2560, kFoldContext = 8;
+
+bool shared_fold_applies(int batch, int q_len, int heads, int64_t cap) {
+  const int64_t rows = static_cast<int64_t>(batch) * q_len, all_heads = static_cast<int64_t>(q_len) * heads;
+  return q_len > 1 && heads < 64 && all_heads >= 32 && rows * ((heads + 15) / 16) * cap >= kFoldTokens &&
+         (cap >= kFoldContext * q_len || rows >= kWaveRows) && (all_heads <= kFoldHeads || rows >= kWaveRows / 2);
+}
 
 // Ranges (workgroups per head group) for `rows` rows of at most `tiles` tiles:
 // the CUs, but per row at most per_row * sqrt(tiles).  A row split over x
@@ -2874,7 +2892,7 @@ AttendPlan plan_attend(const AttendShape& a, int forced, int flags) {
     // waves, one workgroup per CU.
     const bool dense512 = a.Dc == 512 && a.Dr == 64 && a.nk < 0 && a.P % kSubTokens == 0;
     const bool paged32 = dense512 && a.P % kShTokens == 0;
-    const int mode = paged32 && a.T > 1 && shared_fold_applies(a.T, a.H) && cap < (int64_t{1} << 29) ? kShFold
+    const int mode = paged32 && shared_fold_applies(a.B, a.T, a.H, cap) && cap < (int64_t{1} << 29) ? kShFold
                      : paged32                                                                      ? kShDense
                                                                                                     : kShGather;
     const bool gather = (flags & kNoGather) == 0 && a.Dc == 512 && a.Dr == 64 && (a.nk >= 0 || a.P % kSubTokens != 0);

@@ -386,8 +386,10 @@ size_t qd_mla_attend_workspace_bytes(int batch, int q_len, int heads, int latent
 
 /* The plan qd_mla_attend would use: returns 3 for the shared-tile MFMA
  * kernel (latent 512, rope 64: 64 heads or more on listed tokens, on pages of
- * a multiple of 32 tokens or of no multiple of 16, or q_len * heads >= 32 with
- * q_len > 1 on dense pages of a multiple of 32 tokens), 2 for the
+ * a multiple of 32 tokens or of no multiple of 16; or fewer heads and several
+ * queries on dense pages of a multiple of 32 tokens, folded into q_len * heads
+ * heads, *head_groups = ceil(q_len * heads / 64): shared_fold_applies in
+ * mla.hip), 2 for the
  * wave-streamed MFMA kernel (latent 512, rope 64, the other dense rows on
  * pages of a multiple of 16 tokens), 1 for the
  * workgroup-staged MFMA kernel (*out_splits = stream-K workgroups per head

@@ -591,6 +591,9 @@ FOLD_SHAPES = [
     ("h20-t4", 20, 4, 32, [33, 500]),                 # 80 heads: a quarter of the second head group
     ("h32-t2", 32, 2, 64, [1, 2, 63, 64, 65, 2500]),
     ("h128-t3", 128, 3, 32, [31, 32, 34, 900]),
+    ("h8-t16", 8, 16, 32, [16, 17, 40, 700]),         # queries that end in different tiles
+    ("h20-t40", 20, 40, 64, [39, 41, 1000]),
+    ("h64-t24", 64, 24, 64, [24, 300]),               # rows of their own
 ]
 
 
@@ -614,6 +617,25 @@ def test_mla_folded_queries(gpu, shape, dtype, causal):
     ref = _oracle_attend(c, qa, scale, causal, None, dtype)
     for s in (0, 1, 3, 7):
         _close(_attend(c, qa, scale, causal=causal, splits=s), ref, dtype, f"{name} splits={s}")
+
+
+@pytest.mark.parametrize("B,T,H,pages,folded", [
+    (48, 2, 32, 64, True), (32, 4, 8, 8, True), (8, 16, 16, 32, True), (1, 64, 32, 64, True), (32, 96, 8, 8, True),
+    (8, 2, 15, 32, False),                               # fewer than 32 heads in all
+    (8, 2, 64, 32, False), (1, 64, 64, 64, False), (1, 128, 128, 64, False),    # 64 heads per query
+    (4, 8, 8, 1, False),                                 # few tokens in all
+    (4, 16, 20, 1, False), (4, 128, 8, 2, False),        # a chunk of its own context
+    (1, 128, 32, 64, False),                             # many head groups, few rows
+])
+def test_mla_folds_queries_where_it_pays(gpu, B, T, H, pages, folded):
+    say(f"mla plan B{B} T{T} H{H} pages {pages}")
+    kind, _, groups = cabi.mla_attend_info(B, T, H, 512, 64, 64, pages)
+    if folded:
+        assert (kind, groups) == (3, -(-T * H // 64))
+    else:
+        assert groups != -(-T * H // 64) or kind != 3
+        if H >= 64:
+            assert (kind, groups) == (3, -(-H // 64))    # a row per query on the same kernel
 
 
 # (heads, q_len, page, lengths): speculated tokens, the shared-tile and the wave kernel.
