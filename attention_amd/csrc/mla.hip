@@ -1240,7 +1240,7 @@ struct WaveTile {
 // them), writes meta, gtotal and the empty rows.
 // NT: nontemporal cache loads (one head group); with several head groups the
 // tiles are loaded into L2 for the other groups' workgroups on the XCD.
-template <int DT, int NB, int RC, bool NT>
+template <int DT, int NB, int RC, bool NT, bool SPLIT>
 __global__ __launch_bounds__(kAttendThreads) void mla_attend_wave_kernel(MlaParams p) {
   using E = Elem<DT>;
   using Ops = MfmaOps<DT>;
@@ -1648,11 +1648,11 @@ __global__ __launch_bounds__(kAttendThreads) void mla_attend_wave_kernel(MlaPara
       float pr[4];
 #pragma unroll
       for (int i = 0; i < 4; ++i) pr[i] = fast_exp2(x[i] - m_use);
-      // Weights as hi + lo for bf16 (MfmaOps::kSplitWeights); the
+      // Weights as hi + lo (MfmaOps::kSplitWeights, AttendPlan::split); the
       // denominator sums what the PV product uses.
       const u32x2 pb = {Ops::pack2(pr[0], pr[1]), Ops::pack2(pr[2], pr[3])};
       u32x4 pbl = {pb[0], pb[1], 0u, 0u};
-      if constexpr (Ops::kSplitWeights) {
+      if constexpr (SPLIT) {
         pbl[2] = Ops::rest2(pr[0], pr[1], pb[0]);
         pbl[3] = Ops::rest2(pr[2], pr[3], pb[1]);
         l_run += (pr[0] + pr[1]) + (pr[2] + pr[3]);
@@ -1682,9 +1682,9 @@ __global__ __launch_bounds__(kAttendThreads) void mla_attend_wave_kernel(MlaPara
           const uint32_t sel = (e & 1) ? 0x07060302u : 0x05040100u;
           const u32x2 a = {__builtin_amdgcn_perm(raw[1][wd], raw[0][wd], sel),
                            __builtin_amdgcn_perm(raw[3][wd], raw[2][wd], sel)};
-          // bf16: one 16x16x32 MFMA over the lane's 4 tokens twice, [hi, lo]
+          // Split: one 16x16x32 MFMA over the lane's 4 tokens twice, [hi, lo]
           // weights in B (any consistent k order sums the same).
-          if constexpr (Ops::kSplitWeights)
+          if constexpr (SPLIT)
             acc[bb][e] = Ops::mma32(u32x4{a[0], a[1], a[0], a[1]}, pbl, acc[bb][e]);
           else
             acc[bb][e] = Ops::pv(a, pb, acc[bb][e]);
@@ -1859,7 +1859,7 @@ __device__ __forceinline__ void lds_wait_tied(u32x2& a, u32x2& b) {
 // all of them; each lane masks the tokens its query does not see.
 // us per call (latent write and decode) against the wave kernel: fp16 2 x 32
 // heads, B48, U[512, 4096] 76.5 -> 56.5.
-template <int DT, bool NT, int MODE>
+template <int DT, bool NT, int MODE, bool SPLIT>
 __global__ __launch_bounds__(kShThreads) void mla_attend_shared_kernel(MlaParams p) {
   using E = Elem<DT>;
   using Ops = MfmaOps<DT>;
@@ -1867,7 +1867,6 @@ __global__ __launch_bounds__(kShThreads) void mla_attend_shared_kernel(MlaParams
   constexpr int kDc = 512;
   constexpr int kW = 576;
   constexpr int kBufs = shared_bufs(MODE);
-  constexpr bool kSplit = Ops::kSplitWeights;
   extern __shared__ __align__(16) char smem[];
   const int tid = static_cast<int>(threadIdx.x);
   const int lane = tid & 63;
@@ -2316,7 +2315,7 @@ __global__ __launch_bounds__(kShThreads) void mla_attend_shared_kernel(MlaParams
     for (int tb = 0; tb < 2; ++tb) {
       pb[tb] = u32x2{Ops::pack2(wp[tb][0], wp[tb][1]), Ops::pack2(wp[tb][2], wp[tb][3])};
       pbl[tb] = u32x4{pb[tb][0], pb[tb][1], 0u, 0u};
-      if constexpr (kSplit) {
+      if constexpr (SPLIT) {
         pbl[tb][2] = Ops::rest2(wp[tb][0], wp[tb][1], pb[tb][0]);
         pbl[tb][3] = Ops::rest2(wp[tb][2], wp[tb][3], pb[tb][1]);
         l_run += (wp[tb][0] + wp[tb][1]) + (wp[tb][2] + wp[tb][3]);
@@ -2351,7 +2350,7 @@ __global__ __launch_bounds__(kShThreads) void mla_attend_shared_kernel(MlaParams
         TrRead<32 * (cb + kShPvAhead)>::issue(tr1, av[j][1]);
       }
       acc[cb] = Ops::mma32(a, bhi, acc[cb]);
-      if constexpr (kSplit) acc[cb] = Ops::mma32(a, blo, acc[cb]);
+      if constexpr (SPLIT) acc[cb] = Ops::mma32(a, blo, acc[cb]);
       __builtin_amdgcn_sched_barrier(0);
     });
 
@@ -2787,6 +2786,7 @@ struct AttendPlan {
   bool wave;   // MFMA path through mla_attend_wave_kernel
   bool shared;  // MFMA path through mla_attend_shared_kernel
   int mode;     // its tiles (kShDense, kShGather, kShFold)
+  bool split;   // wave and shared-tile kernel: fp16 weights as hi + lo (split_weights)
 };
 
 // Smallest instantiated DMA-chunk count covering ceil(W/64), 0 if none.
@@ -2851,6 +2851,18 @@ int range_count(int64_t rows, int64_t tiles, int groups, double per_row) {
   return static_cast<int>(n);
 }
 
+// Whether fp16 softmax weights go into the products as hi + lo, as bf16 ones
+// always do.  Rounded once, they leave a range's largest weight exact, so the
+// more ranges share a row the smaller the error; fewer ranges than CUs
+// (range_count), listed tokens and folded queries (where the staged and the
+// wave kernel used all CUs) brought 1-5% more error against 64 bits.  Split,
+// it is 0-6% below: H64 B1/L1178 4.51e-4 with all CUs, 4.72e-4 -> 4.49e-4; 128
+// heads, 256 listed, B13 4.19e-4, 4.32e-4 -> 4.10e-4.  Costs (us per call): listed
+// tokens 52.3 -> 54.5, folded 2 x 32 heads B48 57.0 -> 58.7, H64 B1/L4000 33.3 -> 34.9.
+// With a range on every CU the shared-tile kernel is bound by its products
+// (bf16 74.3, fp16 65.1 us at B32 H128), and rounding once stays.
+bool split_weights(int wgs, int groups) { return wgs < device_cus() / groups / 8 * 8; }
+
 AttendPlan plan_attend(const AttendShape& a, int forced, int flags) {
   AttendPlan pl{};
   const int W = a.Dc + a.Dr;
@@ -2908,6 +2920,7 @@ AttendPlan plan_attend(const AttendShape& a, int forced, int flags) {
       if ((smax + wgs - 1) / wgs + 1 <= shared_list_tiles(mode)) {
         pl.shared = true;
         pl.mode = mode;
+        pl.split = mode != kShDense || split_weights(wgs, groups);
         pl.nht = 1;
         pl.head_groups = groups;
         pl.wgs = wgs;
@@ -2921,6 +2934,7 @@ AttendPlan plan_attend(const AttendShape& a, int forced, int flags) {
           forced > 0 ? forced : range_count(rows, (cap + kSubTokens - 1) / kSubTokens, groups, kWaveRangesPerRow);
       if ((gmax + wgs - 1) / wgs + 1 <= kWaveListTiles) {
         pl.wave = true;
+        pl.split = split_weights(wgs, groups);
         pl.nht = 1;
         pl.head_groups = groups;
         pl.wgs = wgs;
@@ -2997,9 +3011,9 @@ hipError_t launch_attend_mfma(const MlaParams& prm, const AttendPlan& pl, int64_
   return hipSuccess;
 }
 
-template <int DT, bool NT>
-hipError_t launch_attend_wave(const MlaParams& prm, const AttendPlan& pl, int64_t grid, hipStream_t st) {
-  auto fn = mla_attend_wave_kernel<DT, 4, 2, NT>;
+template <int DT, bool NT, bool SPLIT>
+hipError_t launch_attend_wave_split(const MlaParams& prm, const AttendPlan& pl, int64_t grid, hipStream_t st) {
+  auto fn = mla_attend_wave_kernel<DT, 4, 2, NT, SPLIT>;
   static std::once_flag once;
   static hipError_t attr = hipSuccess;
   std::call_once(once, [&] {
@@ -3011,9 +3025,15 @@ hipError_t launch_attend_wave(const MlaParams& prm, const AttendPlan& pl, int64_
   return hipSuccess;
 }
 
-template <int DT, bool NT, int MODE>
+template <int DT, bool NT>
+hipError_t launch_attend_wave(const MlaParams& prm, const AttendPlan& pl, int64_t grid, hipStream_t st) {
+  if (DT == QD_DTYPE_BF16 || pl.split) return launch_attend_wave_split<DT, NT, true>(prm, pl, grid, st);
+  return launch_attend_wave_split<DT, NT, DT == QD_DTYPE_BF16>(prm, pl, grid, st);
+}
+
+template <int DT, bool NT, int MODE, bool SPLIT>
 hipError_t launch_attend_shared_mode(const MlaParams& prm, const AttendPlan& pl, int64_t grid, hipStream_t st) {
-  auto fn = mla_attend_shared_kernel<DT, NT, MODE>;
+  auto fn = mla_attend_shared_kernel<DT, NT, MODE, SPLIT>;
   static std::once_flag once;
   static hipError_t attr = hipSuccess;
   std::call_once(once, [&] {
@@ -3027,9 +3047,10 @@ hipError_t launch_attend_shared_mode(const MlaParams& prm, const AttendPlan& pl,
 
 template <int DT, bool NT>
 hipError_t launch_attend_shared(const MlaParams& prm, const AttendPlan& pl, int64_t grid, hipStream_t st) {
-  if (pl.mode == kShGather) return launch_attend_shared_mode<DT, NT, kShGather>(prm, pl, grid, st);
-  if (pl.mode == kShFold) return launch_attend_shared_mode<DT, NT, kShFold>(prm, pl, grid, st);
-  return launch_attend_shared_mode<DT, NT, kShDense>(prm, pl, grid, st);
+  if (pl.mode == kShGather) return launch_attend_shared_mode<DT, NT, kShGather, true>(prm, pl, grid, st);
+  if (pl.mode == kShFold) return launch_attend_shared_mode<DT, NT, kShFold, true>(prm, pl, grid, st);
+  if (DT == QD_DTYPE_BF16 || pl.split) return launch_attend_shared_mode<DT, NT, kShDense, true>(prm, pl, grid, st);
+  return launch_attend_shared_mode<DT, NT, kShDense, DT == QD_DTYPE_BF16>(prm, pl, grid, st);
 }
 
 template <int DT>

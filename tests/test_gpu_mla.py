@@ -686,3 +686,37 @@ def test_mla_queries_do_not_see_later_tokens(gpu, shape, dtype):
                                 assert torch.equal(got[b, t], want[b, t]), (kind, first, s, b, t)
                             else:
                                 _close(got[b, t], _np(want[b, t]), dtype, (kind, first, s, b, t))
+
+
+# (heads, q_len, page, listed tokens or None): wave, shared-tile dense, folded and gathered.
+FP16_ERROR_SHAPES = [(16, 1, 64, None), (64, 1, 64, None), (128, 1, 32, None), (32, 2, 64, None), (20, 3, 64, None),
+                     (64, 1, 64, 256), (128, 1, 1, None)]
+
+
+@pytest.mark.parametrize("shape", FP16_ERROR_SHAPES, ids=lambda s: f"h{s[0]}-t{s[1]}-p{s[2]}-k{s[3]}")
+def test_mla_f16_weights_keep_the_output_to_its_own_rounding(gpu, shape):
+    """fp16 with fewer ranges than CUs: the softmax weights go into the products
+    as hi + lo (22 bits), so with one range (no partials) the result is as far
+    from 64 bits as rounding the exact result to fp16 puts it: 5% allowed for
+    the fp32 sums, whose error is 2^-13 of the rounding's (weights rounded once
+    to 11 bits give 15-35%)."""
+    heads, q_len, page, k = shape
+    say(f"mla f16 error h{heads} t{q_len} p{page} k{k}")
+    lengths = [300, 700, 33, 1200]
+    c = _case(gpu, lengths=lengths, q_len=q_len, heads=heads, block_size=page, dtype=torch.float16, num_indices=k)
+    qa = _absorbed(c, torch.float16).to(torch.float16).to(gpu)
+    scale = default_mla_scale(c["q_nope"].shape[-1], c["q_rope"].shape[-1])
+    got = _attend(c, qa, scale, indices=c["indices"], splits=1).double().cpu()
+    q = torch.cat([qa, c["q_rope"]], -1).double().cpu()
+    cache, table = c["cache"].double().cpu(), c["table"].long().cpu()
+    ref = torch.empty(got.shape, dtype=torch.float64)
+    for b, n in enumerate(lengths):
+        context = cache[table[b, :-(-n // page)]].reshape(-1, 576)
+        for t in range(q_len):
+            rows = context[:min(n, int(c["positions"][b, t]) + 1)]
+            if k is not None:
+                idx = c["indices"][b, t].cpu().long()
+                rows = rows[idx[idx >= 0]]
+            ref[b, t] = torch.softmax(q[b, t] @ rows.t() * scale, -1) @ rows[:, :512]
+    err, rounding = ((x - ref).norm().item() for x in (got, ref.half().double()))
+    assert err <= 1.05 * rounding, (err / rounding)
