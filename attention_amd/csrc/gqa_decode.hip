@@ -418,6 +418,16 @@ __device__ __forceinline__ VRow<D> load_vrow(const char* ptr) {
   return r;
 }
 
+// A lane's V rows first .. first + 3 of a group, those past row `last` to zero:
+// they re-read the last row, and a weight of 0 does not hide an Inf there.
+template <int D>
+__device__ __forceinline__ void zero_rows(VRow<D> (&v)[4], int first, int last) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int w = 0; w < VRow<D>::kWords; ++w) v[i].w[w] = first + i <= last ? v[i].w[w] : 0u;
+}
+
 // Registers for one 16-token group in flight, for NKV kv-heads.
 // Stores NW 32-bit words at dst: one 8-byte store for 2, 16-byte stores for
 // a multiple of 4 (dst aligned to match), else one word at a time.
@@ -497,9 +507,16 @@ __device__ __forceinline__ int vhead_count(const DecodeParams& p, int v) {
 // so every lane owns one head's softmax state and a contiguous slice of
 // DV*4 output elements of that head.  Heads r16 >= group size carry zero
 // queries and are never stored.
-template <int D, int DT, int PF, int NKV>
+//
+// SPLIT: fp16 weights as hi + lo, scaled by 2^kShift (MfmaOps::split2); m_run
+// stays unscaled, l_run and acc carry the factor until a partial is stored
+// (kUnscale, an exact power of two).
+template <int D, int DT, int PF, int NKV, bool SPLIT = false>
 struct MfmaWave {
   using Ops = MfmaOps<DT>;
+  static_assert(!SPLIT || DT == QD_DTYPE_F16, "bf16 always splits (kSplitWeights)");
+  static constexpr int kShift = SPLIT ? MfmaOps<QD_DTYPE_F16>::kWeightShift : 0;
+  static constexpr float kUnscale = 1.f / (1 << kShift);
   using Buf = GroupBuf<D, NKV>;
   static constexpr int KC = D / 32;
   static constexpr int DV = D / 16;
@@ -593,8 +610,13 @@ struct MfmaWave {
     __builtin_amdgcn_sched_barrier(0);
   }
 
-  __device__ void compute(const DecodeParams& p, const Buf& buf, char* ktile) {
+  // TAIL: the group may hold the end of the sequence.
+  template <bool TAIL>
+  __device__ void compute(const DecodeParams& p, Buf& buf, char* ktile) {
     const int last = len - 1 - buf.tg;
+    if constexpr (TAIL && SPLIT) {
+      if (last < 15) zero_rows(buf.v[0], 4 * q4, last);
+    }
 #pragma unroll
     for (int j = 0; j < NKV; ++j) {
       // Transpose K through LDS into the A layout: lane (r16, q4), chunk c
@@ -621,7 +643,7 @@ struct MfmaWave {
       const float alpha = fast_exp2(m_run[j] - mref);
       float pr[4];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) pr[i] = fast_exp2(fmaf(x[i], p.sl2, -mref));
+      for (int i = 0; i < 4; ++i) pr[i] = fast_exp2(fmaf(x[i], p.sl2, kShift - mref));
       l_run[j] = fmaf(l_run[j], alpha, (pr[0] + pr[1]) + (pr[2] + pr[3]));
       m_run[j] = mn;
       if (__builtin_amdgcn_read_exec() & __ballot(alpha != 1.f)) {
@@ -633,18 +655,30 @@ struct MfmaWave {
       // One 16x16x32 MFMA takes both: a lane's k-block of 8 is its 4 tokens
       // twice, V in A and [hi, lo] in B (the MFMA sums over any consistent
       // k order), so the split costs no extra instruction.
-      const u32x2 pb = {Ops::pack2(pr[0], pr[1]), Ops::pack2(pr[2], pr[3])};
-      const u32x4 pbl = {pb[0], pb[1], Ops::rest2(pr[0], pr[1], pb[0]), Ops::rest2(pr[2], pr[3], pb[1])};
+      u32x4 pbl;
+      if constexpr (SPLIT) {
+        uint32_t hi, lo;
+        Ops::split2(pr[0], pr[1], hi, lo);
+        pbl[0] = hi;
+        pbl[2] = lo;
+        Ops::split2(pr[2], pr[3], hi, lo);
+        pbl[1] = hi;
+        pbl[3] = lo;
+      } else {
+        pbl = u32x4{Ops::pack2(pr[0], pr[1]), Ops::pack2(pr[2], pr[3]), 0u, 0u};
+        pbl[2] = Ops::rest2(pr[0], pr[1], pbl[0]);
+        pbl[3] = Ops::rest2(pr[2], pr[3], pbl[1]);
+      }
 #pragma unroll
       for (int d = 0; d < DV; ++d) {
         const int w = d >> 1;
         const uint32_t sel = (d & 1) ? 0x07060302u : 0x05040100u;
         const u32x2 a = {__builtin_amdgcn_perm(buf.v[j][1].w[w], buf.v[j][0].w[w], sel),
                          __builtin_amdgcn_perm(buf.v[j][3].w[w], buf.v[j][2].w[w], sel)};
-        if constexpr (Ops::kSplitWeights)
+        if constexpr (SPLIT || Ops::kSplitWeights)
           acc[j][d] = Ops::mma32(u32x4{a[0], a[1], a[0], a[1]}, pbl, acc[j][d]);
         else
-          acc[j][d] = Ops::pv(a, pb, acc[j][d]);
+          acc[j][d] = Ops::pv(a, u32x2{pbl[0], pbl[1]}, acc[j][d]);
       }
     }
     __builtin_amdgcn_sched_barrier(0);
@@ -684,7 +718,7 @@ struct MfmaWave {
 #pragma unroll
           for (int u = 0; u < PF; ++u) {
             issue(p, buf[(u + PF - 1) % PF], g_lo + i + u + PF - 1);
-            compute(p, buf[u], ktile);
+            compute<PF == 1>(p, buf[u], ktile);
           }
         }
       } else {
@@ -697,7 +731,7 @@ struct MfmaWave {
 #pragma unroll
         for (int u = 0; u < PF; ++u) {
           if (i + u + PF - 1 < n) issue(p, buf[(u + PF - 1) % PF], g_lo + i + u + PF - 1);
-          if (i + u < n) compute(p, buf[u], ktile);
+          if (i + u < n) compute<true>(p, buf[u], ktile);
         }
       }
       g_lo = g_hi;
@@ -876,6 +910,7 @@ struct MfmaWave {
   // stores, for a merge by another workgroup of the same launch.
   template <bool COH = false>
   __device__ void store_partial(const DecodeParams& p, int jk, float* w, int64_t head_stride, float l_tot) {
+    static_assert(!SPLIT || !COH, "scaled accumulators");
     if (r16 >= hcount) return;
     w += r16 * head_stride;
     if (q4 == 0) {
@@ -883,7 +918,7 @@ struct MfmaWave {
         coherent_store2(w, m_run[jk] * kLn2, l_tot);
       } else {
         w[0] = m_run[jk] * kLn2;
-        w[1] = l_tot;
+        w[1] = l_tot * kUnscale;
       }
     }
 #pragma unroll
@@ -894,7 +929,7 @@ struct MfmaWave {
         if constexpr (COH)
           coherent_store2(dst + j, acc[jk][j][i], acc[jk][j + 1][i]);
         else
-          *reinterpret_cast<f32x2*>(dst + j) = f32x2{acc[jk][j][i], acc[jk][j + 1][i]};
+          *reinterpret_cast<f32x2*>(dst + j) = f32x2{acc[jk][j][i] * kUnscale, acc[jk][j + 1][i] * kUnscale};
       }
     }
   }
@@ -908,15 +943,16 @@ struct MfmaWave {
 // at growing sums.  Chains of LEN MFMAs (4 * LEN products) and a binary tree
 // over them round like the VALU kernel's 16 lanes and their tree.  Four chains
 // at a time, side by side, the tree's sums between the next four's MFMAs.
-// LEN 4 where the kernel runs one wave per SIMD (head_dim 128: LEN 2 costs 3%
-// of the call for no smaller error), as the VALU kernel has 16 products per
-// lane above head_dim 128.
+// LEN 4 where the kernel runs one wave per SIMD (head_dim 128: LEN 2 takes 3%
+// more of the call for a 6% smaller error), and above 128, where the VALU kernel
+// has 16 products per lane.
 //
 // Relative error against 64 bits (2-norm), VALU kernel -> one accumulator ->
 // this, with pv_f32: Hq32/Hkv8 D128 B16 U[64, 1024] 1.72e-7 -> 3.90e-7 ->
 // 1.68e-7; over 90 drawn shapes 0.3 to 1.05 of the VALU kernel's (one
-// accumulator: 1.6 to 3.6 times).  The calls take as long as with one
-// accumulator or up to 4% less: the chain of dependent MFMAs is gone.
+// accumulator: 1.6 to 3.6 times).  Us per call, one accumulator -> this: D128
+// B4/L4096 37.0 -> 37.3, B16/L8192 176 -> 180; D64 B16/L8192 94.4 -> 94.6; on the
+// general layout D80 B16/L2048 52.0 -> 54.9, D128 on 1-token pages 61.8 -> 66.7.
 template <int N, int LEN>
 __device__ __forceinline__ f32x4 qk_f32(const u32x4* ka, const u32x4* qf) {
   static_assert(LEN == 2 || LEN == 4, "half a chunk or a chunk per chain");
@@ -1183,9 +1219,10 @@ constexpr int kGenWinPages = 512;  // page-table window of the general layout (L
 //          bytes from memory); K's pad columns are zero in the LDS tile and in
 //          the query, and V's pad columns reach only accumulators that are
 //          never stored.
-// The softmax weights enter the PV product as hi + lo for fp16 too (this
-// layout replaces the VALU kernel, which keeps them in fp32; the second half
-// of the 16x16x32 product costs nothing).
+// The softmax weights enter the PV product as hi + lo (MfmaOps::split2): this
+// layout replaces the VALU kernel, which keeps them in fp32, and the second
+// half of the 16x16x32 product costs nothing.  Rows past the end count as
+// zeros in V, so that an Inf in the last token's row stays Inf.
 //
 // Bound by HBM like MfmaWave.  Against the VALU kernel on the split layout
 // that served these shapes (us per call): fp16 head_dim 80, Hq32/Hkv32, P16,
@@ -1197,6 +1234,8 @@ struct GenWave : MfmaWave<VD, DT, PF, 1> {
   using Ops = MfmaOps<DT>;
   using S = typename Elem<DT>::S;
   static constexpr bool kF32 = DT == QD_DTYPE_F32;
+  static constexpr int kShift = DT == QD_DTYPE_F16 ? MfmaOps<QD_DTYPE_F16>::kWeightShift : 0;  // as MfmaWave's
+  static constexpr float kUnscale = 1.f / (1 << kShift);
   static constexpr int ES = kF32 ? 4 : 2;           // bytes per element
   using VR = VRow<VD * ES / 2>;                     // a lane's EV elements of a V row
   static constexpr int EV = VD / 16;                // V elements per lane and row
@@ -1293,8 +1332,13 @@ struct GenWave : MfmaWave<VD, DT, PF, 1> {
     __builtin_amdgcn_sched_barrier(0);
   }
 
-  __device__ void compute(const DecodeParams& p, const Buf& buf, char* ktile) {
+  // TAIL: the group may hold the end of the sequence.
+  template <bool TAIL>
+  __device__ void compute(const DecodeParams& p, Buf& buf, char* ktile) {
     const int last = this->len - 1 - buf.tg;
+    if constexpr (TAIL) {
+      if (last < 15) zero_rows(buf.v, 4 * this->q4, last);
+    }
 #pragma unroll
     for (int c = 0; c < KCG; ++c) *reinterpret_cast<u32x4*>(ktile + krow[c] * kStride + kcol[c]) = buf.k[c];
     u32x4 ka[KCG];
@@ -1319,7 +1363,7 @@ struct GenWave : MfmaWave<VD, DT, PF, 1> {
     const float alpha = fast_exp2(this->m_run[0] - mref);
     float pr[4];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) pr[i] = fast_exp2(fmaf(x[i], p.sl2, -mref));
+    for (int i = 0; i < 4; ++i) pr[i] = fast_exp2(fmaf(x[i], p.sl2, kShift - mref));
     this->l_run[0] = fmaf(this->l_run[0], alpha, (pr[0] + pr[1]) + (pr[2] + pr[3]));
     this->m_run[0] = mn;
     if constexpr (kF32) {
@@ -1333,8 +1377,10 @@ struct GenWave : MfmaWave<VD, DT, PF, 1> {
 #pragma unroll
         for (int d = 0; d < EV; ++d) this->acc[0][d] *= alpha;
       }
-      const u32x2 hi = {Ops::pack2(pr[0], pr[1]), Ops::pack2(pr[2], pr[3])};
-      const u32x4 w = {hi[0], hi[1], Ops::rest2(pr[0], pr[1], hi[0]), Ops::rest2(pr[2], pr[3], hi[1])};
+      uint32_t h0, l0, h1, l1;
+      Ops::split2(pr[0], pr[1], h0, l0);
+      Ops::split2(pr[2], pr[3], h1, l1);
+      const u32x4 w = {h0, h1, l0, l1};
 #pragma unroll
       for (int d = 0; d < EV; ++d) {
         const uint32_t sel = (d & 1) ? 0x07060302u : 0x05040100u;
@@ -1366,7 +1412,7 @@ struct GenWave : MfmaWave<VD, DT, PF, 1> {
 #pragma unroll
           for (int u = 0; u < PF; ++u) {
             issue(p, buf[(u + PF - 1) % PF], g_lo + i + u + PF - 1);
-            compute(p, buf[u], ktile);
+            compute<PF == 1>(p, buf[u], ktile);
           }
         }
       } else {
@@ -1378,7 +1424,7 @@ struct GenWave : MfmaWave<VD, DT, PF, 1> {
 #pragma unroll
         for (int u = 0; u < PF; ++u) {
           if (i + u + PF - 1 < n) issue(p, buf[(u + PF - 1) % PF], g_lo + i + u + PF - 1);
-          if (i + u < n) compute(p, buf[u], ktile);
+          if (i + u < n) compute<true>(p, buf[u], ktile);
         }
       }
       g_lo = g_hi;
@@ -1409,14 +1455,14 @@ struct GenWave : MfmaWave<VD, DT, PF, 1> {
 
   // w: the lane's partial row {m (natural log), l, acc[dm]}, 8-byte aligned.
   __device__ void put_partial(float* w, float l_tot) const {
-    if (this->q4 == 0) *reinterpret_cast<f32x2*>(w) = f32x2{this->m_run[0] * kLn2, l_tot};
+    if (this->q4 == 0) *reinterpret_cast<f32x2*>(w) = f32x2{this->m_run[0] * kLn2, l_tot * kUnscale};
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       if (!block_ok(i)) continue;
       float* dst = w + 2 + EV * (4 * this->q4 + i);
 #pragma unroll
       for (int j = 0; j < EV; j += 2)
-        *reinterpret_cast<f32x2*>(dst + j) = f32x2{this->acc[0][j][i], this->acc[0][j + 1][i]};
+        *reinterpret_cast<f32x2*>(dst + j) = f32x2{this->acc[0][j][i] * kUnscale, this->acc[0][j + 1][i] * kUnscale};
     }
   }
 
@@ -1835,7 +1881,7 @@ constexpr int wg_wave_merge_bytes(int vd) { return (vd / 16) * 1024 + 512; }
 // after the other (the figures stand at wg_single_applies and wg_waves_for).
 // A lane keeps its own head and columns through the merge, so the exchange is
 // lane-contiguous 16-byte LDS accesses without conflicts.
-template <int D, int DT, int PF, int KCG = 0>
+template <int D, int DT, int PF, int KCG = 0, bool SPLIT = false>
 __global__ __launch_bounds__((64 * sk_max_waves<D, 1, 0, PF, DT>())) void decode_wg_kernel(DecodeParams p) {
   using S = typename Elem<DT>::S;
   constexpr bool kGen = KCG > 0;
@@ -1857,7 +1903,7 @@ __global__ __launch_bounds__((64 * sk_max_waves<D, 1, 0, PF, DT>())) void decode
   using Wave = std::conditional_t<
       kGen, GenWave<D, kGen ? KCG : 1, DT, PF>,
       std::conditional_t<DT == QD_DTYPE_F32, MfmaWaveF32<(DT == QD_DTYPE_F32 && !kGen) ? D : 64, PF>,
-                         MfmaWave<D, DT, PF, 1>>>;
+                         MfmaWave<D, DT, PF, 1, SPLIT>>>;
   Wave wv;
   char* tile = wg_lds + wid * kTile;
   if constexpr (kGen)
@@ -1957,9 +2003,10 @@ __global__ __launch_bounds__((64 * sk_max_waves<D, 1, 0, PF, DT>())) void decode
       }
     } else {
       float* w = part + wv.r16 * head_stride;
-      if (i == 0 && wv.q4 == 0) *reinterpret_cast<f32x2*>(w) = f32x2{M * kLn2, L};
+      if (i == 0 && wv.q4 == 0) *reinterpret_cast<f32x2*>(w) = f32x2{M * kLn2, L * Wave::kUnscale};
 #pragma unroll
-      for (int d = 0; d < DV; d += 2) *reinterpret_cast<f32x2*>(w + 2 + col + d) = f32x2{o[d], o[d + 1]};
+      for (int d = 0; d < DV; d += 2)
+        *reinterpret_cast<f32x2*>(w + 2 + col + d) = f32x2{o[d] * Wave::kUnscale, o[d + 1] * Wave::kUnscale};
     }
   }
 }
@@ -2771,13 +2818,14 @@ KernelFn pick_general_merge_dt(int dtype, int head_dim, bool one_head) {
 }
 
 // decode_wg_kernel for a head_dim: exact layout (fp32: 64 or 128) or general.
-template <int DT>
+// decode_wg_kernel of the exact layout; SPLIT: MfmaWave's.
+template <int DT, bool SPLIT>
 KernelFn pick_wg(int D) {
   switch (D) {
-    case 64: return decode_wg_kernel<64, DT, kPrefetch64>;
-    case 96: return decode_wg_kernel<96, DT, kPrefetch>;
-    case 128: return decode_wg_kernel<128, DT, kPrefetch>;
-    default: return decode_wg_kernel<256, DT, 2>;
+    case 64: return decode_wg_kernel<64, DT, kPrefetch64, 0, SPLIT>;
+    case 96: return decode_wg_kernel<96, DT, kPrefetch, 0, SPLIT>;
+    case 128: return decode_wg_kernel<128, DT, kPrefetch, 0, SPLIT>;
+    default: return decode_wg_kernel<256, DT, 2, 0, SPLIT>;
   }
 }
 
@@ -2802,8 +2850,9 @@ KernelFn pick_wg_dt(int dtype, int D, bool general) {
   if (dtype == QD_DTYPE_F32 && general) return pick_wg_general_f32(D);
   if (dtype == QD_DTYPE_F32)
     return D == 64 ? decode_wg_kernel<64, QD_DTYPE_F32, kPrefetch> : decode_wg_kernel<128, QD_DTYPE_F32, kPrefetch>;
-  if (dtype == QD_DTYPE_F16) return general ? pick_wg_general<QD_DTYPE_F16>(D) : pick_wg<QD_DTYPE_F16>(D);
-  return general ? pick_wg_general<QD_DTYPE_BF16>(D) : pick_wg<QD_DTYPE_BF16>(D);
+  if (general) return dtype == QD_DTYPE_F16 ? pick_wg_general<QD_DTYPE_F16>(D) : pick_wg_general<QD_DTYPE_BF16>(D);
+  if (dtype == QD_DTYPE_F16) return pick_wg<QD_DTYPE_F16, false>(D);
+  return pick_wg<QD_DTYPE_BF16, false>(D);
 }
 
 // Dynamic LDS of a decode_wg_kernel workgroup of nw waves.

@@ -184,6 +184,15 @@ struct MfmaOps<QD_DTYPE_BF16> {
   __device__ static uint32_t rest2(float x, float y, uint32_t hi) {
     return pack2(x - __uint_as_float(hi << 16), y - __uint_as_float(hi & 0xFFFF0000u));
   }
+  // Two weights x, y >= 0 as hi + lo to 16 bits, both parts above 0 wherever the
+  // weight is (hi rounded towards 0, lo at least the smallest normal): an Inf
+  // in V stays Inf, where Inf x 0 or Inf x -lo would make it NaN.
+  static constexpr int kWeightShift = 0;
+  __device__ static void split2(float x, float y, uint32_t& hi, uint32_t& lo) {
+    hi = __builtin_amdgcn_perm(__float_as_uint(y), __float_as_uint(x), 0x07060302u);
+    lo = pack2(fmaxf(x - __uint_as_float(hi << 16), fminf(x, 0x1p-126f)),
+               fmaxf(y - __uint_as_float(hi & 0xFFFF0000u), fminf(y, 0x1p-126f)));
+  }
 };
 
 template <>
@@ -207,12 +216,23 @@ struct MfmaOps<QD_DTYPE_F16> {
     return v[0] + v[1];
   }
   // fp16 keeps 11 significant bits: one rounding of the weights stays far
-  // inside the 16-bit bar (measured 0.2 of it at worst), so no split.
-  // rest2 serves the kernels that split them all the same.
+  // inside the 16-bit bar (measured 0.2 of it at worst), so no split where
+  // the fp32 weights were never used.  rest2 and split2 serve the kernels that
+  // split them all the same.
   static constexpr bool kSplitWeights = false;
   __device__ static uint32_t rest2(float x, float y, uint32_t hi) {
-    const f32x2 v = __builtin_convertvector(__builtin_bit_cast(f16x2, hi), f32x2);
+    const f32x2 v = unpack2(hi);
     return pack2(x - v[0], y - v[1]);
+  }
+  // As for bf16, to 22 bits.  The weights come times 2^kWeightShift (at most
+  // 2^15, inside fp16): unscaled, everything below 2^-25 of the largest weight
+  // would round to 0, and the rest lose their low bits to fp16's fixed grid.
+  static constexpr int kWeightShift = 15;
+  __device__ static void split2(float x, float y, uint32_t& hi, uint32_t& lo) {
+    const float tx = x > 0.f ? 0x1p-24f : 0.f, ty = y > 0.f ? 0x1p-24f : 0.f;
+    hi = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(fmaxf(x, tx), fmaxf(y, ty)));
+    const f32x2 v = unpack2(hi);
+    lo = pack2(fmaxf(x - v[0], tx), fmaxf(y - v[1], ty));
   }
 };
 

@@ -1345,3 +1345,78 @@ def test_f32_matrix_core_error_like_the_valu_kernel(gpu, shape):
     torch.cuda.synchronize()
     err = [((x.double().cpu() - ref).norm() / ref.norm()).item() for x in (out, valu)]
     assert err[0] <= 1.2 * err[1], err
+
+
+# (dtype, Hq, Hkv, D, P, lengths): the layouts that took over from the VALU kernel.
+SMALL_WEIGHT_SHAPES = [
+    (torch.float16, 4, 4, 80, 16, [20000, 3000]),     # balanced
+    (torch.float16, 8, 2, 128, 8, [9000]),
+    (torch.float16, 8, 4, 160, 16, [4000]),
+    (torch.float16, 4, 2, 72, 16, [200, 131]),        # one launch
+    (torch.bfloat16, 4, 4, 80, 16, [20000]),
+    (torch.float32, 4, 4, 80, 16, [20000]),
+]
+
+
+@pytest.mark.parametrize("shape", SMALL_WEIGHT_SHAPES,
+                         ids=lambda s: f"{DT_NAME[s[0]]}-Hq{s[1]}-Hkv{s[2]}-D{s[3]}-P{s[4]}-B{len(s[5])}")
+def test_small_weights_count(gpu, shape):
+    """Weights far below the largest one still count: in every group of 16
+    tokens one token takes nearly all of the softmax with a zero value row, the
+    other 15 have weights of about 2^-26 of it and large values.  Unscaled,
+    fp16 has no numbers that small and the result was 0.  Tolerance: two
+    roundings of the output (2^-10 fp16, 2^-7 bf16), 1e-5 for fp32 sums."""
+    dtype, hq, hkv, d, p, lengths = shape
+    say(f"small weights {DT_NAME[dtype]} D{d} P{p} B{len(lengths)}")
+    q, k, v, table, lens = make_decode_case(lengths=lengths, q_heads=hq, kv_heads=hkv, head_dim=d, block_size=p,
+                                            dtype=dtype, seed=172)
+    q.fill_(1.0)
+    k.zero_()
+    v.uniform_(20000.0, 60000.0)
+    key = 18.02 * math.sqrt(d) / d  # score 18.02 = 26 ln 2 above the others
+    for b, n in enumerate(lengths):
+        for t in range(5, n, 16):
+            k[int(table[b, t // p]), t % p] = key
+            v[int(table[b, t // p]), t % p] = 0.0
+        if n % 16 <= 5 and n > 16:  # the last group has no such token: give it one
+            k[int(table[b, (n - 1) // p]), (n - 1) % p] = key
+            v[int(table[b, (n - 1) // p]), (n - 1) % p] = 0.0
+    case = to_dev((q, k, v, table, lens), gpu)
+    ref = _exact64(*case)
+    got = attention_amd.gqa_decode(*case).double().cpu()
+    assert ref.abs().min() > 1e-4
+    rel = ((got - ref).abs() / ref.abs()).max().item()
+    assert rel <= {torch.float16: 2 ** -10, torch.bfloat16: 2 ** -7, torch.float32: 1e-5}[dtype], rel
+
+
+@pytest.mark.parametrize("shape", [s for s in GENERAL_SHAPES if len(s[5]) < 10] +
+                         [s for s in ONE_LAUNCH_SHAPES if s[0] == torch.float16 and len(s[5]) < 10 and s[3] == 112] +
+                         [(torch.float32, *s) for s in GENERAL_F32_SHAPES if len(s[4]) < 10] +
+                         [(torch.float32, 32, 8, 128, 16, [1, 16, 17, 100]), (torch.float32, 8, 2, 64, 16, [9000, 8001])],
+                         ids=lambda s: f"{DT_NAME[s[0]]}-Hq{s[1]}-Hkv{s[2]}-D{s[3]}-P{s[4]}-B{len(s[5])}")
+def test_inf_values_stay_inf(gpu, shape):
+    """An Inf in V reaches exactly its column of its sequence and kv-head, as
+    Inf of its sign (the token's weight is above 0), whether or not the token
+    is the last one and whatever bits its weight has; the rest matches the
+    oracle.  (Split layout: an early token of long sequences only, as its merge
+    and the VALU kernel re-read their last row with weight 0; fp32 at head_dim 64
+    and 128: not the last token, for the same reason.)"""
+    dtype, hq, hkv, d, p, lengths = shape
+    say(f"inf values {DT_NAME[dtype]} D{d} P{p} B{len(lengths)}")
+    case = make_decode_case(lengths=lengths, q_heads=hq, kv_heads=hkv, head_dim=d, block_size=p, dtype=dtype, seed=173)
+    q, k, v, table, lens = to_dev(case, gpu)
+    ref, rows = oracle_rows((q, k, v, table, lens))
+    want = torch.zeros(len(lengths), hkv, d)
+    path, layout = cabi.auto_path(len(lengths), hq, hkv, d, p, table.shape[1], k.shape[0], cabi.DTYPE[dtype])[:2]
+    last_counts = dtype != torch.float32 or layout != "exact"
+    for b, n in enumerate(lengths):
+        tokens = ({0} if n > 200 else set()) if path == "split" else ({0, n // 3, n - 1} if n else set())
+        for i, tok in enumerate(sorted(tokens if last_counts else tokens - {n - 1})):
+            col, kvh, sign = (7 * b + 5 * i + 3) % d, (b + i) % hkv, 1.0 if i % 2 else -1.0
+            v[int(table[b, tok // p]), tok % p, kvh, col] = sign * float("inf")
+            want[b, kvh, col] = sign
+    out = attention_amd.gqa_decode(q, k, v, table, lens).float().cpu().view(len(lengths), hkv, -1, d)
+    hit = want[:, :, None, :].expand_as(out)
+    assert torch.equal(out[hit != 0], hit[hit != 0] * float("inf"))
+    ref = torch.from_numpy(np.asarray(ref)).float().view_as(out)
+    assert_close(out[hit == 0], ref[hit == 0].numpy(), DT_NAME[dtype], what="finite columns")
