@@ -103,14 +103,16 @@ struct DecodeParams {
 
 #ifdef QD_STAMPS
 // Diagnostic build only (-DQD_STAMPS): 16 words per wave of the stream-K
-// kernel, at stamps[(workgroup * waves + wave) * 16]: s_memrealtime (100 MHz)
+// kernel, at stamps[(workgroup * waves + wave) * 16] (workgroup: slice * ranges +
+// range): s_memrealtime (100 MHz)
 // at entry [0], after the partition search [1], at the end of streaming [2],
 // after the partial stores retired [3], after the arrival atomics returned
 // [4], after the last merge [5]; the XCD id [6]; merges done [7]; the shader
 // clock counter (s_memtime) at entry [8] and at the end of streaming [9].
 __device__ __forceinline__ void stamp_wave(const DecodeParams& p, int slot, uint64_t value) {
   if (p.stamps && (threadIdx.x & 63) == 0)
-    p.stamps[(static_cast<int64_t>(blockIdx.x) * p.wg_waves + (threadIdx.x >> 6)) * 16 + slot] = value;
+    p.stamps[((static_cast<int64_t>(blockIdx.y) * gridDim.x + blockIdx.x) * p.wg_waves + (threadIdx.x >> 6)) * 16 + slot] =
+        value;
 }
 __device__ __forceinline__ uint64_t stamp_now() { return __builtin_amdgcn_s_memrealtime(); }
 __device__ __forceinline__ uint64_t stamp_clock() { return __builtin_amdgcn_s_memtime(); }
@@ -3203,6 +3205,7 @@ int wg_waves_for(int64_t wgs, int64_t groups, int dtype, int head_dim) {
   } else if (head_dim > 128 && wgs >= 256) {
     cap = 1;
   }
+  cap = std::min(cap, wg_max_waves(dtype, head_dim));
   int nw = 1;
   while (2 * nw <= cap && 2 * nw <= groups) nw *= 2;
   return nw;

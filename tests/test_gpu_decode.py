@@ -1255,6 +1255,10 @@ GENERAL_F32_SHAPES = [
     (8, 8, 80, 16, [4500, 1, 0, 900]),                # balanced
     (8, 2, 64, 8, [3000] + _fused_lengths(69, 1, 500, 146)),
     (16, 4, 128, 20, [6000, 17, 2999]),
+    (16, 4, 160, 16, [9000, 33, 0, 4100]),            # ... one wave per SIMD, 256-column merge
+    (8, 2, 192, 16, [4500, 4096, 1, 2000]),
+    (8, 4, 240, 20, _fused_lengths(30, 1, 700, 148)),
+    (4, 2, 256, 16, [9000, 8100]),                    # the VALU kernel's
 ]
 
 
@@ -1277,11 +1281,19 @@ def test_general_layout_f32(gpu, shape):
     k[~used.to(gpu)] = float("inf")
     v[~used.to(gpu)] = float("nan")
     ws = cabi.auto_workspace(len(lengths), hq, hkv, d, p, table.shape[1], cabi.DTYPE[q.dtype], gpu, fill=0xFF)
+    before = ws.clone()
     out = torch.full_like(q, float("nan"))
     rc = cabi.auto_launch(q, k, v, table, lens, out, scale=1 / math.sqrt(d), workspace=ws)
     assert rc == 0, cabi.error_string(rc)
     torch.cuda.synchronize()
     assert_close(out, ref, "f32", rows, "general fp32")
+    path, layout = cabi.auto_path(len(lengths), hq, hkv, d, p, table.shape[1], k.shape[0], cabi.DTYPE[q.dtype])[:2]
+    if len(lengths) * table.shape[1] * p >= 16384 and d != 256:
+        assert path == "balanced"
+    if path != "split":
+        # The balanced kernel writes its meta table and partials, one launch nothing.
+        assert layout == ("exact" if d in (64, 128) and p % 16 == 0 else "general")
+        assert torch.equal(ws, before) == (path == "one launch")
     for splits in (1, 3):
         parts = torch.full((max(1, q.shape[0] * hq * splits * (d + 2)),), float("nan"), device=gpu)
         out = torch.full_like(q, float("nan"))
