@@ -612,13 +612,8 @@ struct MfmaWave {
     __builtin_amdgcn_sched_barrier(0);
   }
 
-  // TAIL: the group may hold the end of the sequence.
-  template <bool TAIL>
-  __device__ void compute(const DecodeParams& p, Buf& buf, char* ktile) {
+  __device__ void compute(const DecodeParams& p, const Buf& buf, char* ktile) {
     const int last = len - 1 - buf.tg;
-    if constexpr (TAIL && SPLIT) {
-      if (last < 15) zero_rows(buf.v[0], 4 * q4, last);
-    }
 #pragma unroll
     for (int j = 0; j < NKV; ++j) {
       // Transpose K through LDS into the A layout: lane (r16, q4), chunk c
@@ -720,7 +715,7 @@ struct MfmaWave {
 #pragma unroll
           for (int u = 0; u < PF; ++u) {
             issue(p, buf[(u + PF - 1) % PF], g_lo + i + u + PF - 1);
-            compute<PF == 1>(p, buf[u], ktile);
+            compute(p, buf[u], ktile);
           }
         }
       } else {
@@ -733,7 +728,7 @@ struct MfmaWave {
 #pragma unroll
         for (int u = 0; u < PF; ++u) {
           if (i + u + PF - 1 < n) issue(p, buf[(u + PF - 1) % PF], g_lo + i + u + PF - 1);
-          if (i + u < n) compute<true>(p, buf[u], ktile);
+          if (i + u < n) compute(p, buf[u], ktile);
         }
       }
       g_lo = g_hi;

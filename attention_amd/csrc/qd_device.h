@@ -185,13 +185,15 @@ struct MfmaOps<QD_DTYPE_BF16> {
     return pack2(x - __uint_as_float(hi << 16), y - __uint_as_float(hi & 0xFFFF0000u));
   }
   // Two weights x, y >= 0 as hi + lo to 16 bits, both parts above 0 wherever the
-  // weight is (hi rounded towards 0, lo at least the smallest normal): an Inf
-  // in V stays Inf, where Inf x 0 or Inf x -lo would make it NaN.
+  // weight is: both rounded towards 0 and lo's last bit set, which rounds the
+  // sum to odd (no bias; lo is at least 2^-133, and the products keep subnormal
+  // operands).  An Inf in V stays Inf, where Inf x 0 or Inf x -lo would make it
+  // NaN.
   static constexpr int kWeightShift = 0;
   __device__ static void split2(float x, float y, uint32_t& hi, uint32_t& lo) {
     hi = __builtin_amdgcn_perm(__float_as_uint(y), __float_as_uint(x), 0x07060302u);
-    lo = pack2(fmaxf(x - __uint_as_float(hi << 16), fminf(x, 0x1p-126f)),
-               fmaxf(y - __uint_as_float(hi & 0xFFFF0000u), fminf(y, 0x1p-126f)));
+    const float rx = x - __uint_as_float(hi << 16), ry = y - __uint_as_float(hi & 0xFFFF0000u);
+    lo = __builtin_amdgcn_perm(__float_as_uint(ry), __float_as_uint(rx), 0x07060302u) | 0x00010001u;
   }
 };
 
@@ -224,15 +226,17 @@ struct MfmaOps<QD_DTYPE_F16> {
     const f32x2 v = unpack2(hi);
     return pack2(x - v[0], y - v[1]);
   }
-  // As for bf16, to 22 bits.  The weights come times 2^kWeightShift (at most
-  // 2^15, inside fp16): unscaled, everything below 2^-25 of the largest weight
-  // would round to 0, and the rest lose their low bits to fp16's fixed grid.
+  // As for bf16, to 22 bits (lo at least 2^-24).  The weights come times
+  // 2^kWeightShift (at most 2^15, inside fp16): unscaled, everything below 2^-25
+  // of the largest weight would round to 0, and the rest lose their low bits to
+  // fp16's fixed grid.  hi is 0 below 2^-39 of the largest weight.
   static constexpr int kWeightShift = 15;
   __device__ static void split2(float x, float y, uint32_t& hi, uint32_t& lo) {
-    const float tx = x > 0.f ? 0x1p-24f : 0.f, ty = y > 0.f ? 0x1p-24f : 0.f;
-    hi = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(fmaxf(x, tx), fmaxf(y, ty)));
-    const f32x2 v = unpack2(hi);
-    lo = pack2(fmaxf(x - v[0], tx), fmaxf(y - v[1], ty));
+    const auto h = __builtin_amdgcn_cvt_pkrtz(x, y);
+    hi = __builtin_bit_cast(uint32_t, h);
+    lo = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(fmaf(static_cast<float>(h[0]), -1.f, x),
+                                                                 fmaf(static_cast<float>(h[1]), -1.f, y))) |
+         0x00010001u;
   }
 };
 

@@ -1432,8 +1432,8 @@ def test_inf_values_stay_inf(gpu, shape):
     Inf of its sign (the token's weight is above 0), whether or not the token
     is the last one and whatever bits its weight has; the rest matches the
     oracle.  (Split layout: an early token of long sequences only, as its merge
-    and the VALU kernel re-read their last row with weight 0; fp32 at head_dim 64
-    and 128: not the last token, for the same reason.)"""
+    and the VALU kernel re-read their last row with weight 0; the exact layouts:
+    not the last token, for the same reason.)"""
     dtype, hq, hkv, d, p, lengths = shape
     say(f"inf values {DT_NAME[dtype]} D{d} P{p} B{len(lengths)}")
     case = make_decode_case(lengths=lengths, q_heads=hq, kv_heads=hkv, head_dim=d, block_size=p, dtype=dtype, seed=173)
@@ -1441,7 +1441,7 @@ def test_inf_values_stay_inf(gpu, shape):
     ref, rows = oracle_rows((q, k, v, table, lens))
     want = torch.zeros(len(lengths), hkv, d)
     path, layout = cabi.auto_path(len(lengths), hq, hkv, d, p, table.shape[1], k.shape[0], cabi.DTYPE[dtype])[:2]
-    last_counts = dtype != torch.float32 or layout != "exact"
+    last_counts = layout != "exact"
     for b, n in enumerate(lengths):
         tokens = ({0} if n > 200 else set()) if path == "split" else ({0, n // 3, n - 1} if n else set())
         for i, tok in enumerate(sorted(tokens if last_counts else tokens - {n - 1})):
