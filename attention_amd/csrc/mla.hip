@@ -2221,14 +2221,15 @@ __global__ __launch_bounds__(kShThreads) void mla_attend_shared_kernel(MlaParams
     // The first PV operand reads, in flight during the softmax (inline asm,
     // TrRead: the builtin form would wait for the next tiles' DMA, issued
     // during QK).
-    uint32_t tr0, tr1;  // rows 4 q4 + r16 / 4 of the two row blocks
+    uint32_t tr0, tr1;  // rows 4 q4 + r16 / 4 of the two row blocks (kShFold; else tr1 = tr0, kTr1 further)
+    constexpr int kTr1 = MODE == kShFold ? 0 : 16 * kShLatStride;
     [[maybe_unused]] int seen = kShTokens;                      // kShFold: rows that this lane's query sees
     [[maybe_unused]] int s_min = kShTokens, s_max = kShTokens;  // ... over the wave's heads
     {
       const uint32_t tile = lds_addr(slot) + 8 * (r16 & 3);
       const int row = 4 * q4 + (r16 >> 2);
       tr0 = tile + row * kShLatStride;
-      tr1 = tr0 + 16 * kShLatStride;
+      tr1 = tr0 + 16 * kShLatStride - kTr1;
       if constexpr (MODE == kShFold) {
         // row_end, with the table's capacity in nv.
         const int tok0 = kShTokens * (e[2] >> 7);
@@ -2248,7 +2249,7 @@ __global__ __launch_bounds__(kShThreads) void mla_attend_shared_kernel(MlaParams
     static_for<0, kShPvAhead>([&](auto c) {
       constexpr int cb = decltype(c)::value;
       TrRead<32 * cb>::issue(tr0, av[cb][0]);
-      TrRead<32 * cb>::issue(tr1, av[cb][1]);
+      TrRead<kTr1 + 32 * cb>::issue(tr1, av[cb][1]);
     });
 
     // Softmax over the tile's 32 tokens: lane holds tokens 16 tb + 4 q4 + i.
@@ -2347,7 +2348,7 @@ __global__ __launch_bounds__(kShThreads) void mla_attend_shared_kernel(MlaParams
       const u32x4 a = {av[j][0][0], av[j][0][1], av[j][1][0], av[j][1][1]};
       if constexpr (cb + kShPvAhead < kShColBlocks) {
         TrRead<32 * (cb + kShPvAhead)>::issue(tr0, av[j][0]);
-        TrRead<32 * (cb + kShPvAhead)>::issue(tr1, av[j][1]);
+        TrRead<kTr1 + 32 * (cb + kShPvAhead)>::issue(tr1, av[j][1]);
       }
       acc[cb] = Ops::mma32(a, bhi, acc[cb]);
       if constexpr (SPLIT) acc[cb] = Ops::mma32(a, blo, acc[cb]);
