@@ -3213,24 +3213,46 @@ int wg_waves_for(int64_t wgs, int64_t groups, int dtype, int head_dim) {
 // us per group (4 waves).  Graph replays, us per call, balanced (fp32: split
 // layout) -> one launch:
 //   bf16 Hq32/Hkv8 D128  B1/L128 11.9 -> 7.5, B1/L512 12.9 -> 11.9, B16/L256 17.2 ->
-//                        11.2, B64/L512 33.8 -> 27.9, B64 U[1, 1024] 36.0 -> 35.0
+//                        11.2, B64/L512 33.8 -> 27.9
 //   bf16 Hq8/Hkv2 D64    B4/L512 10.6 -> 9.9, B256/L1024 34.2 -> 27.6
 //   fp32 Hq32/Hkv8 D128  B1/L128 12.8 -> 9.6, B16/L256 19.3 -> 16.3, B64/L512 60.0 -> 48.9
-// and what lies past the limits: more than 32 groups on few workgroups
-// (B1/L1024 13.9 -> 17.8), more than 64 (B64 U[1, 2048] 51.5 -> 60.8), more than
-// 32768 groups in all (B128 U[1, 1024] 54.7 -> 58.7); head_dim 256 past 16
-// groups (B16 U[1, 512] 19.2 -> 21.3); the general layout past 32 groups or
-// 16384 in all (D80 B64 U[1, 1024] 30.4 -> 34.1); fp32 D128 past 8 groups on few
-// workgroups (B4/L256 14.0 -> 15.1).
-bool wg_single_applies(int64_t wgs, int64_t groups, int dtype, int head_dim, bool general) {
+// and what lies past the limits, where a balanced plan is the alternative
+// (`balanced`): more than 32 groups on few workgroups (B1/L1024 13.9 -> 17.8),
+// more than 64 (B64 U[1, 2048] 51.5 -> 60.8); fp32 D128 past 8 groups on few
+// workgroups (B4/L256 14.0 -> 15.1), and by one launch / balanced over 915
+// exact-layout shapes of B1-512, lengths 64-1024, four head counts:
+//   head_dim 64   at most 1.02 up to 24576 groups in all; 16 groups x 2048
+//                 1.06 and 1.07 (bf16, fp16)
+//   head_dim 96   at most 1.01 up to 32 groups and 14336 in all; 24 x 640 1.02,
+//                 8 x 2048 1.12, 16 x 2048 1.22, 48 and 64 groups up to 1.29
+//   head_dim 128  at most 1.02 up to 28672 in all (above 16 groups 18432, or 32768
+//                 from 768 workgroups on); 16 x 2048 1.03, 32 x 640 and 64 x 320
+//                 mixed lengths 1.05 and 1.04, 32 groups on 4 workgroups 1.07
+//   head_dim 256  at most 1.00 up to 16 groups and 16384 in all; 16 x 1184 1.10
+//   fp32          at most 0.98 up to 16384 in all and 32 groups (head_dim 64
+//                 within 256 workgroups: 48); D64 48 x 296 1.05, 16 x 2048 1.08,
+//                 D128 64 x 512 1.25 (lengths U[1, 1024])
+// Without one (batches past the balanced kernel's, fp32 below kF32SkTokens) the
+// alternative is the split layout, and for the general layout, which has more
+// instructions per group, the line is 32 groups and 16384 in all (D80 B64
+// U[1, 1024] balanced 30.4 -> 34.1).
+bool wg_single_applies(int64_t wgs, int64_t groups, int dtype, int head_dim, bool general, bool balanced) {
   int64_t most = 32, work = 32768;
   if (dtype == QD_DTYPE_F32) {
     most = wgs >= 512 ? 64 : wgs >= 128 ? (head_dim <= 64 ? 64 : 16) : (head_dim <= 64 ? 16 : 8);
     if (general) most = std::min<int64_t>(most, 32);
+    if (balanced) {
+      most = std::min<int64_t>(most, head_dim <= 64 && wgs <= 256 ? 48 : 32);
+      work = 16384;
+    }
   } else if (head_dim > 128) {
     most = 16;
+    if (balanced) work = 16384;
   } else if (general) {
     work = 16384;
+  } else if (balanced) {
+    most = head_dim == 96 ? 32 : wgs >= 64 ? 64 : head_dim == 128 && wgs < 8 ? 24 : 32;
+    work = head_dim == 96 ? 14336 : head_dim == 64 ? 24576 : groups <= 16 ? 28672 : wgs >= 768 ? 32768 : 18432;
   } else if (wgs >= 64) {
     most = 64;
   }
@@ -3342,8 +3364,10 @@ int auto_plan(int batch, int q_heads, int kv_heads, int head_dim, int block_size
   const bool f32_wave = f32_mfma_applies(q_heads, kv_heads, head_dim, block_size, dtype);
   const bool single_gen = !exact && !f32_wave && gen_ok;
   if (aligned && split > 0 && !valu && (exact || f32_wave || single_gen)) {
-    ap->wg_single = vkv <= 65535 && wg_single_applies(static_cast<int64_t>(batch) * vkv, groups, dtype, head_dim, single_gen)
-                        ? wg_waves_for(static_cast<int64_t>(batch) * vkv, groups, dtype, head_dim)
+    const int64_t wgs = static_cast<int64_t>(batch) * vkv;
+    const bool balanced = exact && batch <= kSkMaxBatch;
+    ap->wg_single = vkv <= 65535 && wg_single_applies(wgs, groups, dtype, head_dim, single_gen, balanced)
+                        ? wg_waves_for(wgs, groups, dtype, head_dim)
                         : 0;
     ap->single_gen = single_gen;
     ap->kv_split = split;  // also where no balanced plan follows

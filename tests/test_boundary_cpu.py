@@ -369,6 +369,25 @@ def test_auto_path_reports_what_whole_calls_run(args, path):
     assert cabi.auto_path(4, 8, 3, 64, 16, 4, 64, F16) is None
 
 
+@pytest.mark.parametrize("hq,hkv,d,dt,inside,outside", [
+    # (batch, 16-token pages): the last that measured level or faster in one
+    # launch, the first that measured slower than the balanced kernel.
+    (32, 8, 64, BF16, [(48, 64), (128, 24)], [(256, 16), (49, 64)]),
+    (32, 8, 96, BF16, [(16, 32), (112, 16)], [(16, 48), (48, 64), (128, 16), (256, 8)]),
+    (8, 1, 128, F16, [(4, 24), (8, 32)], [(4, 32), (1, 64), (448, 65)]),
+    (32, 8, 128, BF16, [(1, 32), (64, 32), (224, 16), (128, 32)], [(256, 16), (80, 32), (64, 64), (12, 65)]),
+    (32, 8, 256, F16, [(128, 16)], [(148, 16), (16, 17)]),
+    (8, 2, 64, F32, [(100, 48), (256, 32)], [(148, 48), (256, 48)]),
+    (32, 8, 64, F32, [(1024, 2)], [(256, 16)]),
+    (8, 2, 128, F32, [(256, 24), (256, 32)], [(256, 48), (256, 64)]),
+])
+def test_auto_path_one_launch_only_where_not_slower(hq, hkv, d, dt, inside, outside):
+    for path, sizes in (("one launch", inside), ("balanced", outside)):
+        for batch, pages in sizes:
+            got = cabi.auto_path(batch, hq, hkv, d, 16, pages, 1 << 20, dt)
+            assert got[:2] == (path, "exact"), (batch, pages, got)
+
+
 @pytest.mark.parametrize("batch,hq,hkv,d,pages,dt", [
     (1, 32, 1, 128, 8, F32), (4, 17, 1, 128, 8, F32), (3, 71, 1, 64, 16, F32), (3, 256, 2, 80, 8, F32),
     (3, 64, 2, 192, 8, F32), (3, 64, 2, 256, 8, F32), (4097, 32, 1, 64, 2, BF16), (4097, 40, 1, 80, 1, F16), (4, 32, 1, 128, 8, BF16),
