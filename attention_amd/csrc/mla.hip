@@ -2809,8 +2809,12 @@ constexpr int kNoGather = 1 << 30;  // internal plan flag
 //   below 64 per query: from 64 on a workgroup holds one query's heads as it is,
 //     and folding only makes every query walk the longest one's tiles: 2 x 64
 //     B8/L2048 39.1 -> 41.7, 64 x 64 B1/L4096 85.7 -> 155.8, 128 x 128 252 -> 1775;
-//   from kFoldTokens (sequences x queries x 16-head groups x capacity), less
-//     fits the CUs as it is: 8 x 8 B4/L64 (2K) 21.4 -> 26.8;
+//   with kFoldRows rows of 16 heads (sequences x queries x 16-head groups) of their
+//     own, which fill the CUs, or from kFoldTokens of capacity for all of them:
+//     what lies between was, over 800 sizes in bf16 and fp16, as often slower as
+//     faster (2 x 32 B32/L128 28.0 -> 32.1, 4 x 20 B8/L128 25.4 -> 27.9, 16 x 8 B4/L333 28.9
+//     -> 32.5); up to kFoldFewRows, which ranges of their own do not fill the CUs
+//     with, from kFoldFewTokens (mean 0.97, at most 1.10; 8 x 8 B4/L64 21.4 -> 26.8);
 //   a context of kFoldContext times the queries at least: a chunk of its own
 //     context has half of its pairs hidden, 16 x 20 B4/L64 23.9 -> 27.6, 32 x 32 30.8
 //     -> 34.3, 128 x 8 B4/L128 46.8 -> 51.5; but for rows that fill the wave
@@ -2818,11 +2822,14 @@ constexpr int kNoGather = 1 << 30;  // internal plan flag
 //   up to kFoldHeads in all: more head groups leave each few ranges, whose
 //     prologues walk all queries, 128 x 32 B1/L4096 142 -> 167, 128 x 48 206 -> 394; but
 //     for many rows: 128 x 32 B8/L2048 809 -> 516.
-constexpr int64_t kFoldTokens = 8192, kFoldHeads = 2560, kFoldContext = 8;
+constexpr int64_t kFoldRows = 224, kFoldTokens = 45056, kFoldFewRows = 24, kFoldFewTokens = 8192;
+constexpr int64_t kFoldHeads = 2560, kFoldContext = 8;
 
 bool shared_fold_applies(int batch, int q_len, int heads, int64_t cap) {
   const int64_t rows = static_cast<int64_t>(batch) * q_len, all_heads = static_cast<int64_t>(q_len) * heads;
-  return q_len > 1 && heads < 64 && all_heads >= 32 && rows * ((heads + 15) / 16) * cap >= kFoldTokens &&
+  const int64_t groups = rows * ((heads + 15) / 16);
+  return q_len > 1 && heads < 64 && all_heads >= 32 &&
+         (groups >= kFoldRows || groups * cap >= (groups <= kFoldFewRows ? kFoldFewTokens : kFoldTokens)) &&
          (cap >= kFoldContext * q_len || rows >= kWaveRows) && (all_heads <= kFoldHeads || rows >= kWaveRows / 2);
 }
 

@@ -626,6 +626,8 @@ def test_mla_folded_queries(gpu, shape, dtype, causal):
     (4, 8, 8, 1, False),                                 # few tokens in all
     (4, 16, 20, 1, False), (4, 128, 8, 2, False),        # a chunk of its own context
     (1, 128, 32, 64, False),                             # many head groups, few rows
+    (32, 2, 32, 2, False), (8, 4, 20, 2, False), (16, 2, 32, 10, False),        # neither rows nor tokens enough
+    (75, 4, 16, 1, True), (16, 2, 32, 11, True), (6, 4, 16, 6, True),           # rows, tokens, few rows
 ])
 def test_mla_folds_queries_where_it_pays(gpu, B, T, H, pages, folded):
     say(f"mla plan B{B} T{T} H{H} pages {pages}")
