@@ -2756,8 +2756,8 @@ using KernelFn = void (*)(DecodeParams);
 // 26.8, B16 D160 P32 327.3 -> 45.4, B16 D256 P8 136.0 -> 55.6, B16 D128 P1
 // U[1000, 6000] 89.7 -> 47.0, B64 Hq8/Hkv2 D32 28.9 -> 15.5, B1 Hq8/Hkv1 D16
 // 11.3 -> 9.4; fp32, from kF32GeneralTokens of capacity: Hq32/Hkv4 D72
-// B3/L14328 91.5 -> 36.1, Hq16/Hkv2 D192 B30 107.5 -> 36.8, Hq32/Hkv8 D256 B16
-// 90.0 -> 70.2 (two rows of registers spill there).
+// B3/L14328 91.5 -> 36.1, Hq16/Hkv2 D192 B30 107.5 -> 36.8 (auto_plan leaves
+// fp32 at head_dim 256 on the VALU kernel).
 bool general_applies(int head_dim, int dtype) {
   return (dtype == QD_DTYPE_F16 || dtype == QD_DTYPE_BF16 || dtype == QD_DTYPE_F32) &&
          (head_dim <= 128 ? head_dim % 8 == 0 : head_dim % 16 == 0 && head_dim <= 256);

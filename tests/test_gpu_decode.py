@@ -1,6 +1,6 @@
 """GPU parity of the HIP decode path against the CPU oracle.
 
-Tolerance (BASELINE.json north_star): |err| <= 2e-3 + 1e-2*|ref| for
+Tolerance: |err| <= 2e-3 + 1e-2*|ref| for
 bf16/fp16 caches with fp32 accumulation; fp32 caches use 1e-5 + 1e-4*|ref|.
 Index handling (page permutation, poisoned unused slots, -1 padding) must be
 bit-exact.  Every case prints its name before touching the GPU.

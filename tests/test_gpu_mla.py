@@ -2,7 +2,7 @@
 csrc/cuda/mla/mla.cu:16-198, attention/mla.py:16-53) against the CPU oracle
 (oracle/mla_oracle.py).  Every case prints its name first.
 
-Tolerance (north_star, 16-bit): |got - ref| <= 2e-3 + 1e-2 |ref|; fp32:
+Tolerance (16-bit): |got - ref| <= 2e-3 + 1e-2 |ref|; fp32:
 1e-4 + 1e-4 |ref| (the reference's MLA benchmark tolerance, 1e-4 to 5e-4).
 Copies (latent_kv_write) are bitwise.
 """
