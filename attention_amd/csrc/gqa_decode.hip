@@ -3480,19 +3480,44 @@ int auto_plan(int batch, int q_heads, int kv_heads, int head_dim, int block_size
 // 22.6; 1032, B3 31.4 -> 40.7).
 constexpr int64_t kF32WideSplits = 512;
 
+// Whether fp32 splits of at most `groups` 16-token groups each, `wgs` of them
+// over all (sequence, kv-head) pairs, are left to the VALU kernel at head_dim 64
+// and less: its waves are small and start with one table load, where a GenWave
+// workgroup lays the table window out in LDS and merges its waves, which few
+// groups of short rows do not pay for.  Over 2784 drawn shapes, general / VALU
+// (us per call, VALU -> general):
+//   head_dim <= 32  up to 2.74 (D16 B23 8 splits 46.6 -> 82.4, D32 B232 4 splits
+//                   54.7 -> 92.6) on more than 512 workgroups of up to 16 groups,
+//                   or up to 3 groups; elsewhere at most 1.12, mean 0.49
+//   head_dim 64     up to 1.94 (B51 64 splits 87.8 -> 139) on more than 512 of up
+//                   to 6 groups, or 1 group; elsewhere at most 1.20, mean 0.58
+//   between         up to 1.57 (B130 8 splits 73.7 -> 93.2) on more than 512 of up
+//                   to 2 groups; elsewhere at most 1.00, mean 0.54
+// From 5 q-heads on (8 per VALU wave) and from head_dim 72 on the general layout
+// was faster (mean 0.5; of 735, five up to 1.22 at head_dim 8 to 32, and two of
+// more than 17000 one-group splits 1.13 and 1.14 at 72).
+bool f32_splits_on_valu(int group, int head_dim, int64_t wgs, int64_t groups) {
+  if (group > 4 || head_dim > 64) return false;
+  const int64_t many = head_dim <= 32 ? 16 : head_dim == 64 ? 6 : 2, any = head_dim <= 32 ? 3 : head_dim == 64 ? 1 : 0;
+  return groups <= (wgs > 512 ? many : any);
+}
+
 // Kernel of the explicit split layout: the exact MFMA layout, the general one
 // where that does not apply (groups above kMfmaHeads in chunks as on the
-// balanced path), else the VALU kernel.
+// balanced path), else the VALU kernel.  A split has at most chunk_pages pages.
 enum class SplitKernel { kValu, kExact, kGeneral };
 
 SplitKernel split_kernel(int batch, int q_heads, int kv_heads, int head_dim, int block_size, int64_t num_blocks,
-                         int dtype, int splits, int flags, bool aligned) {
+                         int dtype, int splits, int64_t chunk_pages, int flags, bool aligned) {
   if (!aligned || (flags & QD_FLAG_FORCE_GENERIC) != 0) return SplitKernel::kValu;
   if (mfma_applies(q_heads, kv_heads, head_dim, block_size, dtype)) return SplitKernel::kExact;
   const int64_t chunks = static_cast<int64_t>(kv_heads) * kv_split_for(q_heads, kv_heads);
+  const int64_t wgs = static_cast<int64_t>(splits) * chunks * batch;
   const bool general = general_applies(head_dim, dtype) && chunks > 0 && chunks <= 65535 &&
-                       (dtype != QD_DTYPE_F32 || head_dim <= 96 ||
-                        static_cast<int64_t>(splits) * chunks * batch <= kF32WideSplits) &&
+                       (dtype != QD_DTYPE_F32 ||
+                        (head_dim > 96 ? wgs <= kF32WideSplits
+                                       : !f32_splits_on_valu(q_heads / kv_heads, head_dim, wgs,
+                                                             (chunk_pages * block_size + 15) / 16))) &&
                        pool_rows_fit(num_blocks, block_size);
   return general ? SplitKernel::kGeneral : SplitKernel::kValu;
 }
@@ -3812,16 +3837,16 @@ int qd_gqa_decode_launch(const void* q, const void* k_cache, const void* v_cache
   // pairs); the VALU kernel stores single elements.
   const bool aligned = aligned16(q) && aligned16(k_cache) && aligned16(v_cache) && aligned16(out) &&
                        (splits <= 1 || (reinterpret_cast<uintptr_t>(workspace) & 7u) == 0);
+  const int64_t cp = chunk_pages > 0 ? chunk_pages : (static_cast<int64_t>(max_pages) + splits - 1) / splits;
   const SplitKernel kernel =
-      split_kernel(batch, q_heads, kv_heads, head_dim, block_size, num_blocks, dtype, splits, flags, aligned);
+      split_kernel(batch, q_heads, kv_heads, head_dim, block_size, num_blocks, dtype, splits, cp, flags, aligned);
   (void)hipGetLastError();  // start from a clean error state
   if (kernel != SplitKernel::kValu) {
     const bool general = kernel == SplitKernel::kGeneral;
     const int split_kv = kv_split_for(q_heads, kv_heads);
-    const int cp = chunk_pages > 0 ? chunk_pages : (max_pages + splits - 1) / splits;
     if (general && split_kv > 1) use_kv_chunks(&prm, q_heads, kv_heads, split_kv);
     prm.wg_waves = wg_waves_for(static_cast<int64_t>(splits) * prm.Hkv * batch,
-                                (static_cast<int64_t>(cp) * block_size + 15) / 16, dtype, head_dim);
+                                (cp * block_size + 15) / 16, dtype, head_dim);
     st = launch_wg(prm, dtype, head_dim, general, false, splits, prm.Hkv, batch, stm);
     if (st != QD_OK) return st;
   } else {
@@ -4018,7 +4043,8 @@ int qd_gqa_decode_auto_path(int batch, int q_heads, int kv_heads, int head_dim, 
     nw = ap.wg_waves;
   } else {
     const SplitKernel kernel =
-        split_kernel(batch, q_heads, kv_heads, head_dim, block_size, num_blocks, dtype, ap.splits, 0, true);
+        split_kernel(batch, q_heads, kv_heads, head_dim, block_size, num_blocks, dtype, ap.splits, ap.chunk_pages, 0,
+                     true);
     if (kernel == SplitKernel::kValu) {
       lay = QD_LAYOUT_VALU;
       c = (q_heads / kv_heads + generic_heads(q_heads / kv_heads) - 1) / generic_heads(q_heads / kv_heads);

@@ -402,6 +402,17 @@ def test_auto_path_serves_large_groups_in_chunks(batch, hq, hkv, d, pages, dt):
         assert wgs == batch * hkv * chunks
 
 
+@pytest.mark.parametrize("batch,hq,hkv,d,p,pages,layout", [
+    (1, 32, 8, 64, 64, 115, "valu"), (1, 32, 8, 64, 64, 64, "general"),    # 920 and 512 splits of 4 groups
+    (1, 32, 8, 72, 64, 115, "general"), (1, 40, 8, 64, 64, 115, "general"),  # above head_dim 64, 5 q-heads
+    (2, 32, 8, 32, 12, 79, "valu"), (2, 32, 8, 40, 12, 79, "general"),     # 3 groups, 432 splits
+    (1, 32, 8, 32, 64, 200, "valu"), (1, 8, 2, 32, 64, 128, "general"),    # 800 splits of 8 groups, 256 of 4
+])
+def test_auto_path_short_fp32_splits_on_the_valu_kernel(batch, hq, hkv, d, p, pages, layout):
+    got = cabi.auto_path(batch, hq, hkv, d, p, pages, 1 << 16, F32)
+    assert got[:2] == ("split", layout), got
+
+
 @pytest.mark.parametrize("batch,hq,hkv,d,p,pages,dt", [
     (1, 1, 1, 8, 16, 8, F32), (4, 4, 1, 16, 5, 20, F32), (1, 8, 1, 256, 16, 8, F32), (1, 2, 1, 32, 16, 2, BF16),
     (4097, 1, 1, 40, 8, 1, F16), (4097, 1, 1, 40, 8, 1, F32), (16, 4, 4, 80, 16, 64, F16), (8, 8, 2, 72, 16, 128, F32),
