@@ -3190,8 +3190,21 @@ constexpr int64_t kFusedMaxTrips = 2;
 // splits, us per call with 1 -> 4 waves (graph replays): B4 U[2048, 4096] 4
 // splits 43.0 -> 20.5, 16 splits 18.7 -> 18.2; B1/L16000 16 splits 44.5 -> 21.6;
 // B16 4 splits 48.1 -> 44.2; D64 B32 8 splits 44.2 -> 38.9.
-int wg_waves_for(int64_t wgs, int64_t groups, int dtype, int head_dim) {
+//
+// Splits (`whole` false) stay single waves earlier than whole calls, since the
+// rest of the chip is filled by other splits and a merge of waves comes before
+// the merge of splits.  4 waves over 1, means of 961 drawn shapes: 16 bits up to
+// head_dim 128, more than 768 workgroups of up to 16 groups 1.02 to 1.20 (1.32 at
+// most), more than 256 of up to 4 groups 1.01 to 1.05; fp32, more than 512 of up
+// to 16 groups 1.01 to 1.31.  Short of that 0.3 to 1.02 (16 bits) and 0.3 to 1.01
+// with the waves below.
+int wg_waves_for(int64_t wgs, int64_t groups, int dtype, int head_dim, bool whole) {
   if (wgs > 1024 && groups <= 8) return 1;
+  if (!whole && dtype == QD_DTYPE_F32) {
+    if (wgs > 512 && groups <= 16) return 1;
+  } else if (!whole && head_dim <= 128) {
+    if (groups <= (wgs > 768 ? 16 : wgs > 256 ? 4 : 0)) return 1;
+  }
   int cap = 4;
   if (dtype == QD_DTYPE_F32) {
     if (head_dim > 64 && wgs >= 512) cap = wgs >= 1024 ? 1 : 2;
@@ -3367,7 +3380,7 @@ int auto_plan(int batch, int q_heads, int kv_heads, int head_dim, int block_size
     const int64_t wgs = static_cast<int64_t>(batch) * vkv;
     const bool balanced = exact && batch <= kSkMaxBatch;
     ap->wg_single = vkv <= 65535 && wg_single_applies(wgs, groups, dtype, head_dim, single_gen, balanced)
-                        ? wg_waves_for(wgs, groups, dtype, head_dim)
+                        ? wg_waves_for(wgs, groups, dtype, head_dim, true)
                         : 0;
     ap->single_gen = single_gen;
     ap->kv_split = split;  // also where no balanced plan follows
@@ -3846,7 +3859,7 @@ int qd_gqa_decode_launch(const void* q, const void* k_cache, const void* v_cache
     const int split_kv = kv_split_for(q_heads, kv_heads);
     if (general && split_kv > 1) use_kv_chunks(&prm, q_heads, kv_heads, split_kv);
     prm.wg_waves = wg_waves_for(static_cast<int64_t>(splits) * prm.Hkv * batch,
-                                (cp * block_size + 15) / 16, dtype, head_dim);
+                                (cp * block_size + 15) / 16, dtype, head_dim, false);
     st = launch_wg(prm, dtype, head_dim, general, false, splits, prm.Hkv, batch, stm);
     if (st != QD_OK) return st;
   } else {
@@ -4052,7 +4065,7 @@ int qd_gqa_decode_auto_path(int batch, int q_heads, int kv_heads, int head_dim, 
       if (kernel == SplitKernel::kGeneral) lay = QD_LAYOUT_GENERAL;
       c = kernel == SplitKernel::kGeneral ? kv_split_for(q_heads, kv_heads) : 1;
       nw = wg_waves_for(static_cast<int64_t>(ap.splits) * kv_heads * c * batch,
-                        (static_cast<int64_t>(ap.chunk_pages) * block_size + 15) / 16, dtype, head_dim);
+                        (static_cast<int64_t>(ap.chunk_pages) * block_size + 15) / 16, dtype, head_dim, false);
     }
     wg = static_cast<int64_t>(ap.splits) * batch * kv_heads * c;
   }

@@ -402,6 +402,15 @@ def test_auto_path_serves_large_groups_in_chunks(batch, hq, hkv, d, pages, dt):
         assert wgs == batch * hkv * chunks
 
 
+@pytest.mark.parametrize("batch,hq,hkv,d,pages,waves", [
+    (1, 40, 8, 72, 64, 2), (2, 40, 8, 72, 64, 2),                          # 256 and 512 splits of 2 groups
+    (3, 40, 8, 72, 64, 1), (8, 40, 8, 72, 64, 1), (8, 40, 8, 72, 100, 1),   # 768 of 2, 1024 of 4, 960 of 7
+])
+def test_auto_path_many_short_splits_are_single_waves(batch, hq, hkv, d, pages, waves):
+    got = cabi.auto_path(batch, hq, hkv, d, 16, pages, 1 << 16, F32)
+    assert got[:2] == ("split", "general") and got[4] == waves, got
+
+
 @pytest.mark.parametrize("batch,hq,hkv,d,p,pages,layout", [
     (1, 32, 8, 64, 64, 115, "valu"), (1, 32, 8, 64, 64, 64, "general"),    # 920 and 512 splits of 4 groups
     (1, 32, 8, 72, 64, 115, "general"), (1, 40, 8, 64, 64, 115, "general"),  # above head_dim 64, 5 q-heads
