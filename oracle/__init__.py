@@ -3,7 +3,7 @@
 This package restates the reference algorithm on the CPU so that the HIP
 path can be checked against it.  Only ``tests/``, ``__graft_entry__.smoke()``
 and ``bench.py``'s ``cpu_baseline`` leg may import, call, link or execute
-anything under ``oracle/``, and only as the checker (or, for the CPU
+anything under ``oracle/``, and only to check against (or, for the CPU
 baseline, as the timed reference CPU path) — never as a product code path.
 The product (``attention_amd``) fails loudly when its HIP library is missing.
 

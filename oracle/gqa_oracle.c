@@ -1,7 +1,7 @@
 /*
  * C restatement of the paged GQA decode oracle — TEST INFRASTRUCTURE ONLY
  * (only tests/, __graft_entry__.smoke() and bench.py's cpu_baseline leg may
- * use it, as the checker).
+ * use it, to check against).
  *
  * Follows, per (sequence b, q-head h), reference attention/reference/gqa.py:29-43
  * with the element addressing of csrc/cuda/dense/gqa_decode.cu:31 and :43-47:

@@ -1,5 +1,5 @@
 """Pins the MLA oracle (oracle/mla_oracle.py) before it is trusted as the
-checker of the MLA kernels.
+reference of the MLA kernels.
 
 The reference ships no golden vectors for MLA (its benchmarks compare the
 CUDA ops with torch expressions at runtime, bench_attention_primitives.py:

@@ -1,4 +1,4 @@
-"""Pins the CPU oracle (oracle/) before it is trusted as the checker.
+"""Pins the CPU oracle (oracle/) before it is trusted.
 
 The reference ships no golden vectors and its CUDA sources cannot be built
 here, so each oracle function is fixed by: an independent float64 brute
